@@ -108,6 +108,46 @@ __device__ inline float buffer_load_f32(__amdgpu_buffer_rsrc_t r, unsigned voff,
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
 }
 
+// Read-only array of an earlier kernel, read at wave-uniform indices through
+// the scalar cache: the values land in scalar registers, which cost no LDS
+// bandwidth and no vector registers (a wave-uniform index is made with
+// readfirstlane).
+template <typename T> using smem = __attribute__((address_space(4))) const T;
+template <typename T> __device__ inline smem<T> *scalar_ptr(const T *p) { return (smem<T> *)(uintptr_t)p; }
+
+// Per-wave record lists of one staging round, in record order.  Thread t of
+// the block holds the NL-bit mask of the lists that record base + t belongs
+// to; list w receives the threads t of its members in ascending order (the
+// caller adds base).  NW waves, NL lists; wl[w]: NW * 64 entries; cnt: NL x NW;
+// wlen[w]: the length of list w.  Two block barriers; the caller puts one
+// more before the next round.
+template <int NW, int NL>
+__device__ inline void wave_lists(unsigned mask, unsigned short (*wl)[NW * 64], int (*cnt)[NW], int *wlen)
+{
+    const int lane = threadIdx.x & 63, hw = threadIdx.x >> 6;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    unsigned long long mw[NL];
+#pragma unroll
+    for (int w = 0; w < NL; w++) {
+        mw[w] = __ballot((mask >> w) & 1u);
+        if (lane == 0) cnt[w][hw] = __popcll(mw[w]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < NL; w++) {
+        int o = 0, t = 0;
+#pragma unroll
+        for (int h = 0; h < NW; h++) {
+            const int c = cnt[w][h];
+            if (h < hw) o += c;
+            t += c;
+        }
+        if ((mask >> w) & 1u) wl[w][o + __popcll(mw[w] & below)] = (unsigned short)threadIdx.x;
+        if (threadIdx.x == 0) wlen[w] = t;
+    }
+    __syncthreads();
+}
+
 // LDS written by some lanes of a wave, then read by others: order the wave's
 // LDS traffic (the lanes of a wave execute together).
 __device__ inline void wave_sync()

@@ -41,7 +41,7 @@
 // the second volume axis' spacing for every volume axis.  The derivatives are
 // those of the integrand at the samples (the same moment contraction, with the
 // samples for nodes).
-#include "gt_common.h"
+#include "gt_pixel.h"
 
 namespace gt {
 
@@ -91,6 +91,73 @@ struct alignas(16) PsfRec {
     float s[2];          // pixel half-widths
 };
 static_assert(sizeof(PsfRec) == 96, "PsfRec must stay 96 bytes");
+
+// Tensor rules on whole cells.  Over a cell the exponent is that of its centre
+// plus a linear part l . delta plus the quadratic form of the offset delta
+// from the centre, and the last depends on the record and the node only.  So
+//   int_cell 2^q = 2^q(centre) sum_nodes W[node] prod_axes 2^(l_k delta_k),
+// with W[node] = weights x 2^(form(delta)) tabulated once per record: per
+// cell one exponential for the centre and NP (even) or NP - 1 (odd) per axis
+// instead of NP^K.  W(delta) = W(-delta), so with the sums and differences
+// Xe = X+ + X-, Xo = X+ - X- of a node pair only products with an even number
+// of differences remain (half the terms).  Magnitude index m of a rule: NP
+// even: the NP / 2 positive nodes; NP odd: the centre node, then the positive
+// ones (the centre has Xe = 1, Xo = 0).
+template <int NP> struct PsfNodes {
+    static constexpr int M = (NP + 1) / 2;
+    static constexpr bool ODD = (NP & 1) != 0;
+};
+template <int NP> __host__ __device__ constexpr double psf_node(int m)
+{
+    return NP == 3   ? (m == 0 ? 0.0 : 0.7745966692414834)
+           : NP == 4 ? (m == 0 ? 0.3399810435848563 : 0.8611363115940526)
+           : NP == 5 ? (m == 0 ? 0.0 : (m == 1 ? 0.5384693101056831 : 0.9061798459386640))
+                     : (m == 0 ? 0.2386191860831969 : (m == 1 ? 0.6612093864662645 : 0.9324695142031521));
+}
+template <int NP> __host__ __device__ constexpr double psf_weight(int m)
+{
+    return NP == 3   ? (m == 0 ? 8.0 / 9.0 : 5.0 / 9.0)
+           : NP == 4 ? (m == 0 ? 0.6521451548625461 : 0.3478548451374538)
+           : NP == 5 ? (m == 0 ? 0.5688888888888889 : (m == 1 ? 0.4786286704993665 : 0.2369268850561891))
+                     : (m == 0 ? 0.4679139345726910 : (m == 1 ? 0.3607615730481386 : 0.1713244923791704));
+}
+
+// The points per axis of a whole cell of half-widths s whose axes have the
+// marginal and conditional standard deviations sig and cs: the largest of the
+// axes' rules (3 to 6), or 0 where a cell needs pieces or 8 points (cells
+// wider than two standard deviations: psf_pixel / psf_voxel).
+__device__ inline int psf_whole_rule(int K, const float *s, const float *sig, const float *cs)
+{
+    int np = 0, o;
+    for (int k = 0; k < K; k++) {
+        if (!(s[k] <= sig[k])) return 0;
+        np = max(np, psf_rule(2.0f * s[k], cs[k], o));
+    }
+    return np <= 6 ? np : 0;
+}
+
+// Sums and differences of the node pairs of one axis, t = l x (cell half-width).
+template <int NP> __device__ inline void psf_axis(float t, float *e, float *o)
+{
+#pragma unroll
+    for (int m = 0; m < PsfNodes<NP>::M; m++) {
+        if (PsfNodes<NP>::ODD && m == 0) {
+            e[0] = 1.0f;
+            o[0] = 0.0f;
+            continue;
+        }
+        const float a = t * (float)psf_node<NP>(m);
+        const float p = __builtin_amdgcn_exp2f(a), n = __builtin_amdgcn_exp2f(-a);
+        e[m] = p + n;
+        o[m] = p - n;
+    }
+}
+
+// Exponent of a cell's centre below which the cell holds no support: the
+// nodes of a whole cell lie within 3 x 0.85 of its centre in the metric of the
+// exponent (|.|^2 = -q), so a cell with a node at q >= kappa has its centre at
+// q > -84.
+constexpr float PSF_CELL_MIN = -84.0f;
 
 // R = 1 / min diag U (:25-30) and the atom's total I (pi/30) / det U, or
 // I sqrt(pi/30) / det U in 2D (:60-65): the constants of the sampled rule.
@@ -198,12 +265,57 @@ __device__ inline void psf_setup(const PairGeom<D> &g, const float *const *det, 
     }
 }
 
+// Node table of one (atom, angle) for whole pixels: w[(m0 M + m1) 2 + {0, 1}]
+// multiplies Xe Ye and Xo Yo (alpha and the pixel's area included).
+struct alignas(16) PsfNode2 {
+    int np;        // 3 to 6, or 0: psf_pixel
+    float pad;
+    float w[18];
+};
+static_assert(sizeof(PsfNode2) == 80, "PsfNode2 must stay 80 bytes");
+
+template <int NP>
+__device__ inline void psf_node_table(const PairRec &r, const float *s, PsfNode2 &T)
+{
+    constexpr int M = PsfNodes<NP>::M;
+    const double q0 = r.q[0], q1 = r.q[1], q2 = r.q[2];
+    const double area = (double)r.alpha * s[0] * s[1];
+#pragma unroll
+    for (int m0 = 0; m0 < M; m0++)
+#pragma unroll
+        for (int m1 = 0; m1 < M; m1++) {
+            const double a = s[0] * psf_node<NP>(m0), b = s[1] * psf_node<NP>(m1);
+            const double w = area * psf_weight<NP>(m0) * psf_weight<NP>(m1);
+            const bool z = PsfNodes<NP>::ODD && (m0 == 0 || m1 == 0);
+            const double d = w * exp2(q0 * a * a + q2 * b * b), c = z ? 1.0 : exp2(q1 * a * b);
+            T.w[(m0 * M + m1) * 2] = (float)(z ? d : 0.5 * d * (c + 1.0 / c));
+            T.w[(m0 * M + m1) * 2 + 1] = (float)(z ? 0.0 : 0.5 * d * (c - 1.0 / c));
+        }
+}
+
+__device__ inline void psf_node_record(const PsfRec &R, PsfNode2 &T)
+{
+    const float cs[2] = {psf_csig(R.r.q[0]), psf_csig(R.r.q[2])};
+    T.np = psf_whole_rule(2, R.s, R.sig, cs);
+    T.pad = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 18; k++) T.w[k] = 0.0f;
+    switch (T.np) {
+    case 3: psf_node_table<3>(R.r, R.s, T); break;
+    case 4: psf_node_table<4>(R.r, R.s, T); break;
+    case 5: psf_node_table<5>(R.r, R.s, T); break;
+    case 6: psf_node_table<6>(R.r, R.s, T); break;
+    default: break;
+    }
+}
+
 // half width of the cells of an ascending coordinate vector, from its first
 // spacing (the reference's assumption of a uniform grid, :533, 563)
 __device__ inline float psf_cell_half(const float *v) { return 0.5f * fabsf(v[1] - v[0]); }
 
 template <int D>
-__global__ __launch_bounds__(256) void psf_setup_kernel(gt_atoms A, gt_geom G, PsfRec *recs, int rule)
+__global__ __launch_bounds__(256) void psf_setup_kernel(gt_atoms A, gt_geom G, PsfRec *recs, int rule,
+                                                        PsfNode2 *nodes)
 {
     const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= (long)A.n * G.nA) return;
@@ -220,6 +332,11 @@ __global__ __launch_bounds__(256) void psf_setup_kernel(gt_atoms A, gt_geom G, P
     else
         psf_setup<D>(g, det, nd, hs, R);
     recs[idx] = R;
+    if (D == 3 && nodes) {
+        PsfNode2 T;
+        psf_node_record(R, T);
+        nodes[idx] = T;
+    }
 }
 
 // Pieces and step of the composite rule on [L, U]: pieces of at most 2 sigma.
@@ -557,8 +674,155 @@ __device__ inline int psf_stage(const PsfRec *__restrict__ ra, int base, int N, 
     return total;
 }
 
-// Forward: block = (angle, 16 x 16 pixels) for 2D detectors, numbered centre
-// tiles first (block b: angle b % nA, tile of Morton rank b / nA over the
+// The forward of 2D detectors with pixel integrals: block = (angle, 8 x 64
+// pixels) of 4 waves, numbered centre tiles first (block b: angle b % nA, tile
+// of Morton rank b / nA); wave w owns the 8 x 16 pixels of columns 16 w .. 16 w
+// + 15, lane l column l % 16, rows l / 16 and l / 16 + 4.  A thread tests one
+// record against the four rectangles (index box, then the support against the
+// rectangle widened by half a pixel, support_meets_rect); the waves walk their
+// own lists with the record and its node table in scalar registers.  Four
+// records' values are summed in FP32 and added to an FP64 total.  Bound by VALU
+// issue (an exponential counts four): with the node tables a pixel costs 5 to
+// 13 exponentials instead of 9 to 36 and one form evaluation per node; 1000
+// atoms, 61 x 128^2: 1.59 -> 0.43 ms.
+constexpr int PF_WAVES = 4, PF_CHUNK = PF_WAVES * 64, PF_ROWS = 8, PF_COLS = 16 * PF_WAVES;
+
+template <int NP> __device__ inline float psf_pixel_nodes(smem<float> *w, float t0, float t1)
+{
+    constexpr int M = PsfNodes<NP>::M;
+    float Xe[M], Xo[M], Ye[M], Yo[M];
+    psf_axis<NP>(t0, Xe, Xo);
+    psf_axis<NP>(t1, Ye, Yo);
+    float s = 0.0f;
+#pragma unroll
+    for (int m0 = 0; m0 < M; m0++) {
+        float a = 0.0f, b = 0.0f;
+#pragma unroll
+        for (int m1 = 0; m1 < M; m1++) {
+            const bool z = PsfNodes<NP>::ODD && (m0 == 0 || m1 == 0);
+            if (PsfNodes<NP>::ODD && m1 == 0)
+                a = w[m0 * M * 2];
+            else
+                a = fmaf(w[(m0 * M + m1) * 2], Ye[m1], a);
+            if (!z) b = fmaf(w[(m0 * M + m1) * 2 + 1], Yo[m1], b);
+        }
+        if (PsfNodes<NP>::ODD && m0 == 0)
+            s += a;
+        else
+            s = fmaf(Xe[m0], a, fmaf(Xo[m0], b, s));
+    }
+    return s;
+}
+
+// One record's integrals over a lane's two pixels.
+template <int NP>
+__device__ inline void psf_two_pixels(smem<PsfRec> *R, smem<float> *w, float pc, float prA, float prB, float &vA,
+                                      float &vB)
+{
+    const float q0 = R->r.q[0], q1 = R->r.q[1], q2 = R->r.q[2], q3 = R->r.q[3], q4 = R->r.q[4], q5 = R->r.q[5];
+    const float d1 = (pc - R->r.c_hi[1]) - R->r.c_lo[1];
+    const float row = fmaf(q1, d1, q3), col = fmaf(fmaf(q2, d1, q4), d1, q5);
+    const float l1 = fmaf(2.0f * q2, d1, q4);
+    const float dA = (prA - R->r.c_hi[0]) - R->r.c_lo[0], dB = (prB - R->r.c_hi[0]) - R->r.c_lo[0];
+    const float hA = fmaf(q0, dA, row), hB = fmaf(q0, dB, row);
+    const float eA = fmaf(hA, dA, col), eB = fmaf(hB, dB, col);
+    const float s0 = R->s[0], s1 = R->s[1];
+    const float nA = psf_pixel_nodes<NP>(w, fmaf(q0, dA, hA) * s0, fmaf(q1, dA, l1) * s1);
+    const float nB = psf_pixel_nodes<NP>(w, fmaf(q0, dB, hB) * s0, fmaf(q1, dB, l1) * s1);
+    vA = eA > PSF_CELL_MIN ? __builtin_amdgcn_exp2f(eA) * nA : 0.0f;
+    vB = eB > PSF_CELL_MIN ? __builtin_amdgcn_exp2f(eB) * nB : 0.0f;
+}
+
+__global__ __launch_bounds__(PF_WAVES * 64) void psf_project_kernel(const PsfRec *__restrict__ recs,
+                                                                    const PsfNode2 *__restrict__ nodes, int N, int nA,
+                                                                    int n0, int n1, const float *__restrict__ p0,
+                                                                    const float *__restrict__ p1,
+                                                                    float *__restrict__ R, int e0, int e1)
+{
+    __shared__ unsigned short wl[PF_WAVES][PF_CHUNK];
+    __shared__ int cnt[PF_WAVES][PF_WAVES];
+    __shared__ int wlen[PF_WAVES];
+    const int tilesR = (n0 + PF_ROWS - 1) / PF_ROWS, tilesC = (n1 + PF_COLS - 1) / PF_COLS;
+    const int a = (int)(blockIdx.x % (unsigned)nA);
+    const int e[3] = {e0, e1, 0};
+    int t[3];
+    morton_ranks(blockIdx.x / (unsigned)nA, e, t);
+    if (t[0] >= tilesR || t[1] >= tilesC) return;  // whole block: no tile of this rank
+    const int row0 = centre_out(t[0], tilesR) * PF_ROWS, col0 = centre_out(t[1], tilesC) * PF_COLS;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i1 = col0 + 16 * wave + (lane & 15), rA = row0 + (lane >> 4), rB = rA + 4;
+    const float pc = p1[min(i1, n1 - 1)], prA = p0[min(rA, n0 - 1)], prB = p0[min(rB, n0 - 1)];
+    const float s0 = psf_cell_half(p0), s1 = psf_cell_half(p1);
+    const float xa = p0[row0] - s0, xb = p0[min(row0 + PF_ROWS - 1, n0 - 1)] + s0;
+    float cy[2 * PF_WAVES];
+#pragma unroll
+    for (int w = 0; w < PF_WAVES; w++) {
+        cy[2 * w] = p1[min(col0 + 16 * w, n1 - 1)] - s1;
+        cy[2 * w + 1] = p1[min(col0 + 16 * w + 15, n1 - 1)] + s1;
+    }
+    const PsfRec *ra = recs + (size_t)a * N;
+    const PsfNode2 *na = nodes + (size_t)a * N;
+    double sA = 0.0, sB = 0.0;
+    for (int base = 0; base < N; base += PF_CHUNK) {
+        unsigned mask = 0;
+        const int j = base + (int)threadIdx.x;
+        if (j < N) {
+            const float4 *src = reinterpret_cast<const float4 *>(ra + j);
+            const float4 f0 = src[0], f1 = src[1], f2 = src[2];
+            const int4 bx = reinterpret_cast<const int4 *>(ra + j)[3];  // lo[0], lo[1], hi[0], hi[1]
+            if (bx.x <= row0 + PF_ROWS - 1 && bx.z >= row0 && bx.y <= col0 + PF_COLS - 1 && bx.w >= col0) {
+#pragma unroll
+                for (int w = 0; w < PF_WAVES; w++) {
+                    const int c = col0 + 16 * w;
+                    if (bx.y <= c + 15 && bx.w >= c &&
+                        support_meets_rect(f1, f2, (xa - f0.y) - f0.w, (xb - f0.y) - f0.w, (cy[2 * w] - f0.z) - f1.x,
+                                           (cy[2 * w + 1] - f0.z) - f1.x))
+                        mask |= 1u << w;
+                }
+            }
+        }
+        wave_lists<PF_WAVES, PF_WAVES>(mask, wl, cnt, wlen);
+        const int len = __builtin_amdgcn_readfirstlane(wlen[wave]);
+        float gA = 0.0f, gB = 0.0f;
+        for (int k = 0; k < len; k++) {
+            const int jj = base + __builtin_amdgcn_readfirstlane((int)wl[wave][k]);
+            smem<PsfRec> *rec = scalar_ptr(ra) + jj;
+            smem<PsfNode2> *nd = scalar_ptr(na) + jj;
+            smem<float> *w = nd->w;
+            float vA, vB;
+            switch (nd->np) {
+            case 3: psf_two_pixels<3>(rec, w, pc, prA, prB, vA, vB); break;
+            case 4: psf_two_pixels<4>(rec, w, pc, prA, prB, vA, vB); break;
+            case 5: psf_two_pixels<5>(rec, w, pc, prA, prB, vA, vB); break;
+            case 6: psf_two_pixels<6>(rec, w, pc, prA, prB, vA, vB); break;
+            default: {
+                float m[1];
+                psf_pixel<2, 1>(ra[jj], prA, pc, m);
+                vA = rec->r.alpha * m[0];
+                psf_pixel<2, 1>(ra[jj], prB, pc, m);
+                vB = rec->r.alpha * m[0];
+            }
+            }
+            gA += vA;
+            gB += vB;
+            if ((k & 3) == 3) {
+                sA += (double)gA;
+                sB += (double)gB;
+                gA = gB = 0.0f;
+            }
+        }
+        sA += (double)gA;
+        sB += (double)gB;
+        __syncthreads();
+    }
+    if (i1 < n1) {
+        if (rA < n0) R[((size_t)a * n0 + rA) * n1 + i1] = (float)sA;
+        if (rB < n0) R[((size_t)a * n0 + rB) * n1 + i1] = (float)sB;
+    }
+}
+
+// Forward of the sampled rule and of 1D detectors: block = (angle, 16 x 16
+// pixels) for 2D detectors, numbered centre tiles first (block b: angle b % nA, tile of Morton rank b / nA over the
 // centre-out tile ranks, 2^e0 x 2^e1), or (angle = blockIdx.y, 256 pixels) for
 // 1D ones.
 template <int K, int RULE>
@@ -1137,14 +1401,20 @@ using namespace gt;
 
 static size_t psf_rec_bytes(const gt_atoms *a, const gt_geom *g) { return align_up((size_t)a->n * g->nA * sizeof(PsfRec)); }
 
+// node tables of the 2D-detector forward
+static size_t psf_node_bytes(const gt_atoms *a, const gt_geom *g)
+{
+    return a->dim == 3 ? align_up((size_t)a->n * g->nA * sizeof(PsfNode2)) : 0;
+}
+
 extern "C" size_t gt_psf_forward_workspace(const gt_atoms *atoms, const gt_geom *geom)
 {
     if (!atoms || !geom) return 0;
-    return psf_rec_bytes(atoms, geom);
+    return psf_rec_bytes(atoms, geom) + psf_node_bytes(atoms, geom);
 }
 
 static int psf_prepare(const gt_atoms *atoms, const gt_geom *geom, int rule, void *ws, size_t ws_bytes, size_t need,
-                       hipStream_t st, const char *who)
+                       hipStream_t st, const char *who, PsfNode2 *nodes = nullptr)
 {
     int rc;
     if ((rc = check_atoms(atoms)) || (rc = check_geom(geom, atoms->dim))) return rc;
@@ -1164,9 +1434,10 @@ static int psf_prepare(const gt_atoms *atoms, const gt_geom *geom, int rule, voi
     const long pairs = (long)atoms->n * geom->nA;
     const dim3 grid((unsigned)((pairs + 255) / 256));
     if (atoms->dim == 3)
-        hipLaunchKernelGGL(psf_setup_kernel<3>, grid, dim3(256), 0, st, *atoms, *geom, recs, rule);
+        hipLaunchKernelGGL(psf_setup_kernel<3>, grid, dim3(256), 0, st, *atoms, *geom, recs, rule, nodes);
     else
-        hipLaunchKernelGGL(psf_setup_kernel<2>, grid, dim3(256), 0, st, *atoms, *geom, recs, rule);
+        hipLaunchKernelGGL(psf_setup_kernel<2>, grid, dim3(256), 0, st, *atoms, *geom, recs, rule,
+                           (PsfNode2 *)nullptr);
     GT_HIP(hipGetLastError());
     return 0;
 }
@@ -1180,8 +1451,10 @@ extern "C" int gt_psf_forward_rule(const gt_atoms *atoms, const gt_geom *geom, i
         set_error("gt_psf_forward: atoms or geometry is NULL");
         return GT_EINVAL;
     }
+    const bool whole = atoms->dim == 3 && rule == GT_PSF_EXACT;
+    PsfNode2 *nodes = whole ? (PsfNode2 *)((char *)ws + psf_rec_bytes(atoms, geom)) : nullptr;
     if ((rc = psf_prepare(atoms, geom, rule, ws, ws_bytes, gt_psf_forward_workspace(atoms, geom), st,
-                          "gt_psf_forward")))
+                          "gt_psf_forward", nodes)))
         return rc;
     GT_CHECK_ARG(R != nullptr, "gt_psf_forward: R is NULL");
     const int n1 = atoms->dim == 3 ? geom->n1 : 1;
@@ -1194,16 +1467,18 @@ extern "C" int gt_psf_forward_rule(const gt_atoms *atoms, const gt_geom *geom, i
     }
     const PsfRec *recs = (const PsfRec *)ws;
     prof_begin(st, GT_K_FORWARD);
-    if (atoms->dim == 3) {
+    if (whole) {
+        const int e0 = ceil_log2((geom->n0 + PF_ROWS - 1) / PF_ROWS), e1 = ceil_log2((n1 + PF_COLS - 1) / PF_COLS);
+        GT_CHECK_ARG(((unsigned long long)geom->nA << (e0 + e1)) < (1ull << 31), "gt_psf_forward: too many tiles");
+        hipLaunchKernelGGL(psf_project_kernel, dim3((unsigned)((unsigned long long)geom->nA << (e0 + e1))),
+                           dim3(PF_WAVES * 64), 0, st, recs, (const PsfNode2 *)nodes, atoms->n, geom->nA, geom->n0, n1,
+                           geom->p0, geom->p1, R, e0, e1);
+    } else if (atoms->dim == 3) {
         const int e0 = ceil_log2((geom->n0 + 15) / 16), e1 = ceil_log2((n1 + 15) / 16);
         GT_CHECK_ARG(((unsigned long long)geom->nA << (e0 + e1)) < (1ull << 31), "gt_psf_forward: too many tiles");
         const dim3 grid((unsigned)((unsigned long long)geom->nA << (e0 + e1)));
-        if (rule == GT_PSF_SAMPLED)
-            hipLaunchKernelGGL((psf_forward_kernel<2, GT_PSF_SAMPLED>), grid, dim3(256), 0, st, recs, atoms->n,
-                               geom->nA, geom->n0, n1, geom->p0, geom->p1, R, e0, e1);
-        else
-            hipLaunchKernelGGL((psf_forward_kernel<2, GT_PSF_EXACT>), grid, dim3(256), 0, st, recs, atoms->n, geom->nA,
-                               geom->n0, n1, geom->p0, geom->p1, R, e0, e1);
+        hipLaunchKernelGGL((psf_forward_kernel<2, GT_PSF_SAMPLED>), grid, dim3(256), 0, st, recs, atoms->n, geom->nA,
+                           geom->n0, n1, geom->p0, geom->p1, R, e0, e1);
     } else {
         const dim3 grid((unsigned)((geom->n0 + 255) / 256), (unsigned)geom->nA);
         if (rule == GT_PSF_SAMPLED)

@@ -1,0 +1,52 @@
+"""Whole-cell rules of the point-spread kernels (tabulated node weights)
+against the FP64 oracle, at the cell widths where the number of points per
+axis changes and at detector sizes around the kernels' tiles.
+
+Tolerance: the rules hold about 1e-7 of (peak x cell), the exponents |q| < 43
+and the four-term FP32 sums add a few 1e-7 of the largest value; 2e-6 of the
+largest value covers both.
+"""
+import importlib
+
+import numpy as np
+import pytest
+
+from conftest import f32
+
+pytestmark = pytest.mark.gpu
+
+TOL = 2e-6
+
+
+def _rel(a, b):
+    return float(np.abs(np.asarray(a, float) - b).max() / np.abs(b).max())
+
+
+def _atoms(rng, n, cell, ratio, corr):
+    """n atoms whose conditional standard deviations are cell / ratio (times
+    up to 1.1), correlated when corr > 0."""
+    d = ratio / cell / np.sqrt(60) * rng.uniform(0.9, 1.0, (n, 3))
+    o = corr * d[:, :1] * rng.uniform(-1, 1, (n, 3))
+    x = rng.uniform(-0.6, 0.6, (n, 3))
+    x[0] = 1.02  # cut by the edge of the grid
+    return rng.uniform(0.5, 1.5, n), x, np.concatenate((d, o), 1)
+
+
+# cell width over the standard deviation: rules of 3, 4, 5 and 6 points, and pieces / 8 points
+@pytest.mark.parametrize("ratio", [0.45, 0.95, 1.35, 1.9, 2.6])
+@pytest.mark.parametrize("n0,n1,n", [(7, 5, 3), (8, 64, 4), (9, 65, 5), (17, 130, 3)])
+def test_project(gt, oracle, cuda, ratio, n0, n1, n):
+    psf = importlib.import_module("2018_dictionary_tomography_amd.psf")
+    W = importlib.import_module("2018_dictionary_tomography_amd.workloads")
+    rng = np.random.default_rng(int(100 * ratio) + n0)
+    cell = 2.0 / 65
+    det = [cell * (np.arange(m) - 0.5 * (m - 1)) for m in (n0, n1)]
+    T, ortho, _ = W.tilt_series(3, 50.0, axis=(0.1, 1.0, 0.2), det=8)
+    space = gt.ProjSpace(orientations=T, ortho=ortho, detector=det)
+    I, x, r = _atoms(rng, n, cell, ratio, 0.2)
+    x[1:] *= 0.5 * cell * np.array([n0, n1, n1])
+    x[0, 0] = 0.5 * cell * n0  # on the edge
+    atoms = gt.AtomElement(gt.AtomSpace(3, isotropic=False), x, r, I, device=cuda)
+    P = psf.forward(atoms, space).cpu().numpy()
+    og = oracle.Geometry(f32(space.orientations), tuple(f32(o) for o in space.ortho), [f32(q) for q in det])
+    assert _rel(P, oracle.psf_radproj(f32(I), f32(x), f32(r), og, 24)) < TOL
