@@ -1093,11 +1093,8 @@ constexpr double PSF_SQRT_NEG_KAPPA = 6.578818071009935;  // sqrt(30 log2 e)
 
 // Rule GT_PSF_SAMPLED: hw = (R, total, s) with s half the second axis'
 // spacing, voxel box = the voxels within |R| + s of x per axis.
-template <int D>
-__global__ __launch_bounds__(256) void psf_vol_setup_kernel(gt_atoms A, gt_vol V, PsfVolRec *recs, int rule)
+template <int D> __device__ inline PsfVolRec psf_vol_record(const gt_atoms &A, const gt_vol &V, int j, int rule)
 {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= A.n) return;
     constexpr int NR = Dims<D>::NR;
     PairGeom<D> g;
     load_atom<D>(A, j, g);
@@ -1131,8 +1128,7 @@ __global__ __launch_bounds__(256) void psf_vol_setup_kernel(gt_atoms A, gt_vol V
             R.lo[c] = lower_idx(y[c], m[c], g.x[c] - reach - pad);
             R.hi[c] = upper_idx(y[c], m[c], g.x[c] + reach + pad);
         }
-        recs[j] = R;
-        return;
+        return R;
     }
     const float hv[3] = {psf_cell_half(V.y0), psf_cell_half(V.y1), D == 3 ? psf_cell_half(V.y2) : 0.0f};
     double Ui[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
@@ -1165,7 +1161,14 @@ __global__ __launch_bounds__(256) void psf_vol_setup_kernel(gt_atoms A, gt_vol V
         R.lo[c] = lower_idx(y[c], m[c], g.x[c] - hw - hv[c] - pad);
         R.hi[c] = upper_idx(y[c], m[c], g.x[c] + hw + hv[c] + pad);
     }
-    recs[j] = R;
+    return R;
+}
+
+template <int D>
+__global__ __launch_bounds__(256) void psf_vol_setup_kernel(gt_atoms A, gt_vol V, PsfVolRec *recs, int rule)
+{
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j < A.n) recs[j] = psf_vol_record<D>(A, V, j, rule);
 }
 
 // exponent of one node: -|U'(y - x)|^2 with y - x from the float pairs
@@ -1317,6 +1320,261 @@ template <int D> __device__ inline float psf_voxel_sampled(const PsfVolRec &R, c
     return w * acc;
 }
 
+// Node table of one 3D atom for whole voxels: w[((m0 M + m1) M + m2) 4 + k], k =
+// 0..3, multiplies Xe Ye Ze, Xe Yo Zo, Xo Ye Zo and Xo Yo Ze (amplitude and
+// the voxel's volume included).
+struct alignas(16) PsfNode3 {
+    int np;  // 3 to 6, or 0: psf_voxel
+    float pad[3];
+    float w[108];
+};
+static_assert(sizeof(PsfNode3) == 448, "PsfNode3 must stay 448 bytes");
+
+// Entry idx (m0, m1, m2) of the table: the weights of the node and of its
+// reflections in the second, third and first axis, combined.
+template <int NP>
+__device__ inline void psf_node_entry(const PsfVolRec &R, const float *hv, int idx, float *w)
+{
+    constexpr int M = PsfNodes<NP>::M;
+    if (idx >= M * M * M) return;
+    const int mi[3] = {idx / (M * M), (idx / M) % M, idx % M};
+    double d[3], f = (double)R.amp;
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        double x = psf_node<NP>(0), wt = psf_weight<NP>(0);
+#pragma unroll
+        for (int m = 1; m < M; m++)
+            if (mi[c] == m) {
+                x = psf_node<NP>(m);
+                wt = psf_weight<NP>(m);
+            }
+        d[c] = hv[c] * x;
+        f *= hv[c] * wt;
+    }
+    // signs (+++), (++-), (+-+), (-++)
+    double W[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const double d0 = k == 3 ? -d[0] : d[0], d1 = k == 2 ? -d[1] : d[1], d2 = k == 1 ? -d[2] : d[2];
+        const double a0 = R.u[0] * d0 + R.u[3] * d1 + R.u[5] * d2, a1 = R.u[1] * d1 + R.u[4] * d2, a2 = R.u[2] * d2;
+        W[k] = 0.25 * f * exp2(-(a0 * a0 + a1 * a1 + a2 * a2));
+    }
+    w[idx * 4 + 0] = (float)(W[0] + W[1] + W[2] + W[3]);
+    w[idx * 4 + 1] = (float)(W[0] - W[1] - W[2] + W[3]);
+    w[idx * 4 + 2] = (float)(W[0] - W[1] + W[2] - W[3]);
+    w[idx * 4 + 3] = (float)(W[0] + W[1] - W[2] - W[3]);
+}
+
+// |column c of U'|^2: the curvature of the exponent along axis c
+__device__ inline void psf_col_norms(const PsfVolRec &R, float *cn)
+{
+    cn[0] = R.u[0] * R.u[0];
+    cn[1] = fmaf(R.u[3], R.u[3], R.u[1] * R.u[1]);
+    cn[2] = fmaf(R.u[5], R.u[5], fmaf(R.u[4], R.u[4], R.u[2] * R.u[2]));
+}
+
+// Record and node table of one atom per wave: lane 0 the record, the lanes one
+// table entry each.
+__global__ __launch_bounds__(64) void psf_voxel_setup_kernel(gt_atoms A, gt_vol V, PsfVolRec *recs, PsfNode3 *nodes)
+{
+    __shared__ PsfVolRec R;
+    const int j = blockIdx.x, lane = threadIdx.x;
+    if (lane == 0) {
+        R = psf_vol_record<3>(A, V, j, GT_PSF_EXACT);
+        recs[j] = R;
+    }
+    wave_sync();
+    const float hv[3] = {psf_cell_half(V.y0), psf_cell_half(V.y1), psf_cell_half(V.y2)};
+    float cn[3], sig[3], cs[3];
+    psf_col_norms(R, cn);
+    for (int c = 0; c < 3; c++) {
+        sig[c] = R.hw[c] * 0.12909944487358055f;  // hw / sqrt(60)
+        cs[c] = psf_csig(-cn[c]);
+    }
+    const int np = psf_whole_rule(3, hv, sig, cs);
+    PsfNode3 &T = nodes[j];
+    if (lane == 0) T.np = np;
+    switch (np) {
+    case 3: psf_node_entry<3>(R, hv, lane, T.w); break;
+    case 4: psf_node_entry<4>(R, hv, lane, T.w); break;
+    case 5: psf_node_entry<5>(R, hv, lane, T.w); break;
+    case 6: psf_node_entry<6>(R, hv, lane, T.w); break;
+    default: break;
+    }
+}
+
+template <int NP> __device__ inline float psf_voxel_nodes(smem<float> *w, float t0, float t1, float t2)
+{
+    constexpr int M = PsfNodes<NP>::M;
+    constexpr bool ODD = PsfNodes<NP>::ODD;
+    float Xe[M], Xo[M], Ye[M], Yo[M], Ze[M], Zo[M];
+    psf_axis<NP>(t0, Xe, Xo);
+    psf_axis<NP>(t1, Ye, Yo);
+    psf_axis<NP>(t2, Ze, Zo);
+    float s = 0.0f;
+#pragma unroll
+    for (int m0 = 0; m0 < M; m0++) {
+        float se = 0.0f, so = 0.0f;
+#pragma unroll
+        for (int m1 = 0; m1 < M; m1++) {
+            float a = 0.0f, b = 0.0f, c = 0.0f, d = 0.0f;
+#pragma unroll
+            for (int m2 = 0; m2 < M; m2++) {
+                smem<float> *q = w + ((m0 * M + m1) * M + m2) * 4;
+                const bool z0 = ODD && m0 == 0, z1 = ODD && m1 == 0, z2 = ODD && m2 == 0;
+                if (z2)
+                    a = q[0];
+                else
+                    a = fmaf(q[0], Ze[m2], a);
+                if (!z1 && !z2) b = fmaf(q[1], Zo[m2], b);
+                if (!z0 && !z2) c = fmaf(q[2], Zo[m2], c);
+                if (!z0 && !z1) {
+                    if (z2)
+                        d = q[3];
+                    else
+                        d = fmaf(q[3], Ze[m2], d);
+                }
+            }
+            if (ODD && m1 == 0) {
+                se += a;
+                so += c;
+            } else {
+                se = fmaf(Ye[m1], a, fmaf(Yo[m1], b, se));
+                so = fmaf(Ye[m1], c, fmaf(Yo[m1], d, so));
+            }
+        }
+        if (ODD && m0 == 0)
+            s += se;
+        else
+            s = fmaf(Xe[m0], se, fmaf(Xo[m0], so, s));
+    }
+    return s;
+}
+
+// The 3D render with voxel integrals.  Block = brick of 4 x 8 x 8 voxels, four
+// cubes of 4 x 4 x 4 (lane = voxel), PX_GROUPS waves per cube that take every
+// PX_GROUPS-th record of the cube's list; bricks nearest the volume centre
+// first.  A thread tests one record against the four cubes: index box, then
+// the plane through the cube's centre across the exponent's gradient g there
+// (the support reaches |v| rho along it, v = U'(yc - x), rho^2 = -kappa; the
+// cube comes as near as |v|^2 - sum |g_c| extent_c).  Records and node tables are
+// read into scalar registers; four records' values are summed in FP32 and
+// added to an FP64 total, the groups' totals in group order.  Bound by VALU
+// issue: a voxel costs 7 to 19 exponentials instead of 27 to 216, and the cube
+// test drops what the boxes of slanted ellipsoids keep; 1000 atoms on 64^3:
+// 1.75 -> 0.16 ms.
+constexpr int PX_GROUPS = 4, PX_CUBES = 4, PX_WAVES = PX_GROUPS * PX_CUBES, PX_THREADS = 64 * PX_WAVES;
+
+template <int NP>
+__device__ inline float psf_cell_value(smem<float> *w, const float *g, const float *hv, float e)
+{
+    const float n = psf_voxel_nodes<NP>(w, -2.0f * g[0] * hv[0], -2.0f * g[1] * hv[1], -2.0f * g[2] * hv[2]);
+    return e > PSF_CELL_MIN ? __builtin_amdgcn_exp2f(e) * n : 0.0f;
+}
+
+__global__ __launch_bounds__(PX_THREADS) void psf_voxels_kernel(const PsfVolRec *__restrict__ recs,
+                                                                const PsfNode3 *__restrict__ nodes, int N, gt_vol V,
+                                                                float *__restrict__ u, int e0, int e1, int e2)
+{
+    __shared__ alignas(8) unsigned short wl[PX_CUBES][PX_THREADS];
+    __shared__ int cnt[PX_CUBES][PX_WAVES];
+    __shared__ int wlen[PX_CUBES];
+    static_assert(sizeof(wl) >= PX_THREADS * sizeof(double), "reduction buffer");
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int cube = wave & (PX_CUBES - 1), grp = wave / PX_CUBES;
+    const int nb0 = (V.m0 + 3) / 4, nb1 = (V.m1 + 7) / 8, nb2 = (V.m2 + 7) / 8;
+    const int e[3] = {e0, e1, e2};
+    int tb[3];
+    morton_ranks(blockIdx.x, e, tb);
+    if (tb[0] >= nb0 || tb[1] >= nb1 || tb[2] >= nb2) return;  // whole block
+    const int b0 = centre_out(tb[0], nb0) * 4, b1 = centre_out(tb[1], nb1) * 8, b2 = centre_out(tb[2], nb2) * 8;
+    const int i0 = b0 + (lane >> 4), i1 = b1 + 4 * (cube >> 1) + ((lane >> 2) & 3), i2 = b2 + 4 * (cube & 1) + (lane & 3);
+    const bool valid = i0 < V.m0 && i1 < V.m1 && i2 < V.m2;
+    const float yc[3] = {V.y0[min(i0, V.m0 - 1)], V.y1[min(i1, V.m1 - 1)], V.y2[min(i2, V.m2 - 1)]};
+    const float hv[3] = {psf_cell_half(V.y0), psf_cell_half(V.y1), psf_cell_half(V.y2)};
+    // centre and half extent (voxels included) of the brick's cubes per axis
+    float cc[3][2], ce[3][2];
+    {
+        const float *y[3] = {V.y0, V.y1, V.y2};
+        const int b[3] = {b0, b1, b2}, m[3] = {V.m0, V.m1, V.m2};
+#pragma unroll
+        for (int c = 0; c < 3; c++)
+#pragma unroll
+            for (int h = 0; h < (c == 0 ? 1 : 2); h++) {
+                const float ya = y[c][min(b[c] + 4 * h, m[c] - 1)], yb = y[c][min(b[c] + 4 * h + 3, m[c] - 1)];
+                cc[c][h] = 0.5f * (ya + yb);
+                ce[c][h] = 0.5f * (yb - ya) + hv[c];
+            }
+    }
+    double s = 0.0;
+    for (int base = 0; base < N; base += PX_THREADS) {
+        unsigned mask = 0;
+        const int j = base + (int)threadIdx.x;
+        if (j < N) {
+            const PsfVolRec &r = recs[j];
+            if (r.lo[0] <= b0 + 3 && r.hi[0] >= b0 && r.lo[1] <= b1 + 7 && r.hi[1] >= b1 && r.lo[2] <= b2 + 7 &&
+                r.hi[2] >= b2) {
+                const float d0 = (cc[0][0] - r.xh[0]) - r.xl[0];
+#pragma unroll
+                for (int c = 0; c < PX_CUBES; c++) {
+                    const int h1 = c >> 1, h2 = c & 1, c1 = b1 + 4 * h1, c2 = b2 + 4 * h2;
+                    const float d1 = (cc[1][h1] - r.xh[1]) - r.xl[1], d2 = (cc[2][h2] - r.xh[2]) - r.xl[2];
+                    const float v0 = fmaf(r.u[0], d0, fmaf(r.u[3], d1, r.u[5] * d2));
+                    const float v1 = fmaf(r.u[1], d1, r.u[4] * d2), v2 = r.u[2] * d2;
+                    const float n2 = fmaf(v0, v0, fmaf(v1, v1, v2 * v2));
+                    const float g0 = r.u[0] * v0, g1 = fmaf(r.u[3], v0, r.u[1] * v1);
+                    const float g2 = fmaf(r.u[5], v0, fmaf(r.u[4], v1, r.u[2] * v2));
+                    const float reach = fmaf(fabsf(g0), ce[0][0], fmaf(fabsf(g1), ce[1][h1], fabsf(g2) * ce[2][h2]));
+                    // NaN keeps the record
+                    const bool apart = n2 * (1.0f - 1e-4f) - reach > ((float)PSF_SQRT_NEG_KAPPA + 1e-2f) * sqrtf(n2);
+                    if (r.lo[1] <= c1 + 3 && r.hi[1] >= c1 && r.lo[2] <= c2 + 3 && r.hi[2] >= c2 && !apart)
+                        mask |= 1u << c;
+                }
+            }
+        }
+        wave_lists<PX_WAVES, PX_CUBES>(mask, wl, cnt, wlen);
+        const int len = __builtin_amdgcn_readfirstlane(wlen[cube]);
+        float part = 0.0f;
+        int n4 = 0;
+        for (int k = grp; k < len; k += PX_GROUPS) {
+            const int jj = base + __builtin_amdgcn_readfirstlane((int)wl[cube][k]);
+            smem<PsfVolRec> *r = scalar_ptr(recs) + jj;
+            smem<PsfNode3> *nd = scalar_ptr(nodes) + jj;
+            smem<float> *w = nd->w;
+            const float u0 = r->u[0], u1 = r->u[1], u2 = r->u[2], u3 = r->u[3], u4 = r->u[4], u5 = r->u[5];
+            const float d0 = (yc[0] - r->xh[0]) - r->xl[0], d1 = (yc[1] - r->xh[1]) - r->xl[1],
+                        d2 = (yc[2] - r->xh[2]) - r->xl[2];
+            const float v0 = fmaf(u0, d0, fmaf(u3, d1, u5 * d2)), v1 = fmaf(u1, d1, u4 * d2), v2 = u2 * d2;
+            const float g[3] = {u0 * v0, fmaf(u3, v0, u1 * v1), fmaf(u5, v0, fmaf(u4, v1, u2 * v2))};
+            const float ex = -fmaf(v0, v0, fmaf(v1, v1, v2 * v2));
+            float v;
+            switch (nd->np) {
+            case 3: v = psf_cell_value<3>(w, g, hv, ex); break;
+            case 4: v = psf_cell_value<4>(w, g, hv, ex); break;
+            case 5: v = psf_cell_value<5>(w, g, hv, ex); break;
+            case 6: v = psf_cell_value<6>(w, g, hv, ex); break;
+            default: v = psf_voxel<3>(recs[jj], yc, hv);
+            }
+            part += v;
+            if ((++n4 & 3) == 0) {
+                s += (double)part;
+                part = 0.0f;
+            }
+        }
+        s += (double)part;
+        __syncthreads();
+    }
+    double *red = reinterpret_cast<double *>(&wl[0][0]);
+    red[threadIdx.x] = s;
+    __syncthreads();
+    if (grp == 0 && valid) {
+        double t = 0.0;
+        for (int g = 0; g < PX_GROUPS; g++) t += red[(g * PX_CUBES + cube) * 64 + lane];
+        u[((size_t)i0 * V.m1 + i1) * V.m2 + i2] = (float)t;
+    }
+}
+
+// The other renders (sampled rule, 2D):
 // Block = brick of 4 x 8 x 8 voxels (3D) or 16 x 16 (2D), thread = voxel,
 // PV_GROUPS groups of 256 threads on the same brick: group g takes every
 // PV_GROUPS-th staged record, and the groups' compensated sums are added in
@@ -1595,7 +1853,8 @@ extern "C" size_t gt_psf_volume_workspace(const gt_atoms *atoms, const gt_vol *v
 {
     (void)vol;
     if (!atoms) return 0;
-    return align_up((size_t)atoms->n * sizeof(PsfVolRec));
+    return align_up((size_t)atoms->n * sizeof(PsfVolRec)) +
+           (atoms->dim == 3 ? align_up((size_t)atoms->n * sizeof(PsfNode3)) : 0);
 }
 
 extern "C" int gt_psf_volume_rule(const gt_atoms *atoms, const gt_vol *vol, int rule, float *u, void *ws,
@@ -1632,7 +1891,12 @@ extern "C" int gt_psf_volume_rule(const gt_atoms *atoms, const gt_vol *vol, int 
     const dim3 sg((unsigned)((atoms->n + 255) / 256));
     // bricks numbered by Morton index over 2^e0 x 2^e1 x 2^e2 centre-out ranks
     int nb[3];
-    if (vol->dim == 3) {
+    const bool whole = vol->dim == 3 && rule == GT_PSF_EXACT;
+    PsfNode3 *nodes = (PsfNode3 *)((char *)ws + align_up((size_t)atoms->n * sizeof(PsfVolRec)));
+    if (whole) {
+        hipLaunchKernelGGL(psf_voxel_setup_kernel, dim3((unsigned)atoms->n), dim3(64), 0, st, *atoms, *vol, recs, nodes);
+        nb[0] = (vol->m0 + 3) / 4, nb[1] = (vol->m1 + 7) / 8, nb[2] = (vol->m2 + 7) / 8;
+    } else if (vol->dim == 3) {
         hipLaunchKernelGGL(psf_vol_setup_kernel<3>, sg, dim3(256), 0, st, *atoms, *vol, recs, rule);
         nb[0] = (vol->m0 + 3) / 4, nb[1] = (vol->m1 + 7) / 8, nb[2] = (vol->m2 + 7) / 8;
     } else {
@@ -1643,13 +1907,12 @@ extern "C" int gt_psf_volume_rule(const gt_atoms *atoms, const gt_vol *vol, int 
     GT_CHECK_ARG(e[0] + e[1] + e[2] <= 30, "gt_psf_volume: grid too large");
     const unsigned blocks = 1u << (e[0] + e[1] + e[2]);
     prof_begin(st, GT_K_VOLUME);
-    if (vol->dim == 3) {
-        if (rule == GT_PSF_SAMPLED)
-            hipLaunchKernelGGL((psf_volume_kernel<3, GT_PSF_SAMPLED>), dim3(blocks), dim3(PV_THREADS), 0, st, recs,
-                               atoms->n, *vol, u, e[0], e[1], e[2]);
-        else
-            hipLaunchKernelGGL((psf_volume_kernel<3, GT_PSF_EXACT>), dim3(blocks), dim3(PV_THREADS), 0, st, recs,
-                               atoms->n, *vol, u, e[0], e[1], e[2]);
+    if (whole) {
+        hipLaunchKernelGGL(psf_voxels_kernel, dim3(blocks), dim3(PX_THREADS), 0, st, recs, (const PsfNode3 *)nodes,
+                           atoms->n, *vol, u, e[0], e[1], e[2]);
+    } else if (vol->dim == 3) {
+        hipLaunchKernelGGL((psf_volume_kernel<3, GT_PSF_SAMPLED>), dim3(blocks), dim3(PV_THREADS), 0, st, recs,
+                           atoms->n, *vol, u, e[0], e[1], e[2]);
     } else {
         if (rule == GT_PSF_SAMPLED)
             hipLaunchKernelGGL((psf_volume_kernel<2, GT_PSF_SAMPLED>), dim3(blocks), dim3(PV_THREADS), 0, st, recs,

@@ -50,3 +50,18 @@ def test_project(gt, oracle, cuda, ratio, n0, n1, n):
     P = psf.forward(atoms, space).cpu().numpy()
     og = oracle.Geometry(f32(space.orientations), tuple(f32(o) for o in space.ortho), [f32(q) for q in det])
     assert _rel(P, oracle.psf_radproj(f32(I), f32(x), f32(r), og, 24)) < TOL
+
+
+@pytest.mark.parametrize("ratio", [0.45, 0.95, 1.35, 1.9, 2.6])
+@pytest.mark.parametrize("shape,n", [((2, 3, 5), 3), ((4, 8, 8), 4), ((5, 9, 17), 5), ((11, 4, 7), 1100)])
+def test_render(gt, oracle, cuda, ratio, shape, n):
+    psf = importlib.import_module("2018_dictionary_tomography_amd.psf")
+    rng = np.random.default_rng(int(100 * ratio) + shape[0])
+    cell = 2.0 / 33
+    y = [cell * (np.arange(m) - 0.5 * (m - 1)) for m in shape]
+    I, x, r = _atoms(rng, n, cell, ratio, 0.2)
+    x[1:] *= 0.5 * cell * np.array(shape)
+    x[0] = 0.5 * cell * np.array(shape) * (1, 0, 0)  # on a face
+    atoms = gt.AtomElement(gt.AtomSpace(3, isotropic=False), x, r, I, device=cuda)
+    u = psf.volume(atoms, gt.VolSpace(y)).cpu().numpy()
+    assert _rel(u, oracle.psf_volproj(f32(I), f32(x), f32(r), [f32(v) for v in y], 12)) < TOL
