@@ -310,8 +310,9 @@ __device__ inline int wave_max_i32(int v)
 // concave quadratic in one variable, maximised at its clamped vertex)
 // reaches the cutoff, widened by SPAN_SLACK.  A record whose quadratic is
 // not strictly concave (rounded) is always kept.  f1, f2: the record's
-// floats 4..11, (c_lo1, q0, q1, q2) and (q3, q4, q5, pad).
-__host__ __device__ inline bool support_meets_rect(const float4 &f1, const float4 &f2, float xa, float xb, float ya, float yb)
+// floats 4..11, (c_lo1, q0, q1, q2) and (q3, q4, q5, pad).  kappa: the cutoff.
+__host__ __device__ inline bool support_meets_rect(const float4 &f1, const float4 &f2, float xa, float xb, float ya,
+                                                   float yb, float kappa = (float)KAPPA)
 {
     const float q0 = f1.y, q1 = f1.z, q2 = f1.w, q3 = f2.x, q4 = f2.y, q5 = f2.z;
     if (!(q0 < 0.0f) || !(q2 < 0.0f) || !(q1 * q1 < 4.0f * q0 * q2)) return true;
@@ -331,7 +332,7 @@ __host__ __device__ inline bool support_meets_rect(const float4 &f1, const float
         const float xx = fminf(fmaxf(lin2 * i0, xa), xb);
         best = fmaxf(best, fmaf(fmaf(q0, xx, lin2), xx, fmaf(fmaf(q2, yy, q4), yy, q5)));
     }
-    return best >= (float)KAPPA - SPAN_SLACK;
+    return best >= kappa - SPAN_SLACK;
 }
 
 // One pixel of the moments walks, branch-free.  xp = (x, x^2, x^3, x^4).

@@ -1511,9 +1511,9 @@ __global__ __launch_bounds__(PX_THREADS) void psf_voxels_kernel(const PsfVolRec 
         unsigned mask = 0;
         const int j = base + (int)threadIdx.x;
         if (j < N) {
-            const PsfVolRec &r = recs[j];
-            if (r.lo[0] <= b0 + 3 && r.hi[0] >= b0 && r.lo[1] <= b1 + 7 && r.hi[1] >= b1 && r.lo[2] <= b2 + 7 &&
-                r.hi[2] >= b2) {
+            const PsfVolRec r = recs[j];
+            if ((int)(r.lo[0] <= b0 + 3) & (int)(r.hi[0] >= b0) & (int)(r.lo[1] <= b1 + 7) & (int)(r.hi[1] >= b1) &
+                (int)(r.lo[2] <= b2 + 7) & (int)(r.hi[2] >= b2)) {
                 const float d0 = (cc[0][0] - r.xh[0]) - r.xl[0];
 #pragma unroll
                 for (int c = 0; c < PX_CUBES; c++) {
