@@ -1,11 +1,12 @@
-// gt_ftpatch.h -- per-patch culling of the Fourier grid evaluation.
+// gt_ftpatch.h -- culling of the Fourier grid and plane evaluations.
 //
 // An FT-space atom contributes I exp(-|U^T k|^2 / 2) exp(-i x . k) where
 // |U^T k|^2 < 30 (GaussDictCode/bin/FTGaussian3D.py:95-110, 151-164): its
 // support is an ellipsoid about k = 0.  ft_patch_min bounds |U^T k|^2 from
 // below over a rectangle of (k1, k2) at fixed k0, so that a patch of samples
-// the support cannot reach is skipped.  Host-callable for the brute-force
-// check in tests/native.
+// the support cannot reach is skipped; ft_box_meets does the same for a box, and
+// kp_row_range bounds the rows of a sample plane that an ellipse reaches.
+// Host-callable for the brute-force checks in tests/native.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -50,6 +51,47 @@ __host__ __device__ inline float ft_patch_min(const FtL &r, float k0, float a1, 
         best = fminf(best, fmaf(p1, p1, p2 * p2));
     }
     return fmaf(v0, v0, best);
+}
+
+// Can the support {|U^T k| < rho} (scaled as FtRec.u, upper-triangular form) reach the box of half
+// extents x about the centre m?  Tested on the plane through the centre across
+// the gradient g = U v of |v|^2 / 2, v = U^T m: the support reaches rho |v| along g,
+// the box comes as near as |v|^2 - sum |g_c| x_c (relative slack 1e-3; NaN keeps).
+__host__ __device__ inline bool ft_box_meets(const FtL &r, float m0, float m1, float m2, float x0, float x1, float x2,
+                                             float rho)
+{
+    const float v0 = r.u[0] * m0, v1 = fmaf(r.u[1], m1, r.u[3] * m0);
+    const float v2 = fmaf(r.u[4], m1, fmaf(r.u[5], m0, r.u[2] * m2));
+    const float n2 = fmaf(v0, v0, fmaf(v1, v1, v2 * v2));
+    const float g0 = fmaf(r.u[0], v0, fmaf(r.u[3], v1, r.u[5] * v2));
+    const float g1 = fmaf(r.u[1], v1, r.u[4] * v2), g2 = r.u[2] * v2;
+    const float reach = fmaf(fabsf(g0), x0, fmaf(fabsf(g1), x1, fabsf(g2) * x2));
+    return !(n2 * (1.0f - 1e-4f) - reach > rho * (1.0f + 1e-3f) * sqrtf(n2));
+}
+
+// The rows [xlo, xhi] that the ellipse {q0 x^2 + q1 x y + q2 y^2 >= cut} (cut <
+// 0) has in the band ya <= y <= yb: its convex part in the band spans from the
+// least to the largest x, each at the ellipse's own extreme point when that
+// lies in the band, else on the nearer band edge.  Widened by a relative 1e-3;
+// everything for a form that is not strictly concave; empty (xlo > xhi) when
+// the band misses the ellipse.
+__host__ __device__ inline void kp_row_range(float q0, float q1, float q2, float cut, float ya, float yb, float &xlo,
+                                             float &xhi)
+{
+    xlo = -3.0e38f;
+    xhi = 3.0e38f;
+    const float det = 4.0f * q0 * q2 - q1 * q1;
+    if (!(q0 < 0.0f) || !(q2 < 0.0f) || !(det > 1e-6f * q0 * q2)) return;
+    const float hw = sqrtf(4.0f * cut * q2 / det);  // half-width in x
+    const float ys = -0.5f * q1 / q2 * hw;          // y of the point x = hw (x = -hw: -ys)
+    const float yr = fminf(fmaxf(ys, ya), yb), yl = fminf(fmaxf(-ys, ya), yb);
+    // q0 x^2 + q1 y x + q2 y^2 - cut = 0 at y = yr (larger root) and y = yl (smaller root)
+    const float dr = q1 * yr * q1 * yr - 4.0f * q0 * (q2 * yr * yr - cut);
+    const float dl = q1 * yl * q1 * yl - 4.0f * q0 * (q2 * yl * yl - cut);
+    const float tol = 1e-3f * hw;
+    const float i2 = -0.5f / q0;
+    xhi = fmaf(q1, yr, sqrtf(fmaxf(dr, 0.0f))) * i2 + tol;
+    xlo = fmaf(q1, yl, -sqrtf(fmaxf(dl, 0.0f))) * i2 - tol;
 }
 
 }  // namespace gt

@@ -29,6 +29,7 @@
 // the even moments of |E|^2, are needed: 24 FP32 moments per (atom, angle),
 // accumulated column by column, then contracted in FP64 by the wave.  The
 // isotropic 3D form is L = Id / r with the chain rule over the diagonal slots.
+#include "gt_ftpatch.h"
 #include "gt_pixel.h"
 
 namespace gt {
@@ -295,31 +296,6 @@ __global__ __launch_bounds__(256) void kp_eval_kernel(const KpRec<R> *__restrict
 static_assert(sizeof(KpRec<float>) == 48, "KpRec<float>: amp, q[3] | ch[2], cl[2] | lo[2], hi[2]");
 constexpr int KE_WAVES = 8, KE_ROWS = 16, KE_COLS = 32, KE_R = KE_ROWS / 2;
 constexpr int KE_GROUP = 8;
-
-// The rows [xlo, xhi] that the ellipse {q0 x^2 + q1 x y + q2 y^2 >= cut} (cut <
-// 0) has in the band ya <= y <= yb: its convex part in the band spans from the
-// least to the largest x, each at the ellipse's own extreme point when that
-// lies in the band, else on the nearer band edge.  Widened by a relative 1e-3;
-// everything for a form that is not strictly concave; empty (xlo > xhi) when
-// the band misses the ellipse.
-__host__ __device__ inline void kp_row_range(float q0, float q1, float q2, float cut, float ya, float yb, float &xlo,
-                                             float &xhi)
-{
-    xlo = -3.0e38f;
-    xhi = 3.0e38f;
-    const float det = 4.0f * q0 * q2 - q1 * q1;
-    if (!(q0 < 0.0f) || !(q2 < 0.0f) || !(det > 1e-6f * q0 * q2)) return;
-    const float hw = sqrtf(4.0f * cut * q2 / det);  // half-width in x
-    const float ys = -0.5f * q1 / q2 * hw;          // y of the point x = hw (x = -hw: -ys)
-    const float yr = fminf(fmaxf(ys, ya), yb), yl = fminf(fmaxf(-ys, ya), yb);
-    // q0 x^2 + q1 y x + q2 y^2 - cut = 0 at y = yr (larger root) and y = yl (smaller root)
-    const float dr = q1 * yr * q1 * yr - 4.0f * q0 * (q2 * yr * yr - cut);
-    const float dl = q1 * yl * q1 * yl - 4.0f * q0 * (q2 * yl * yl - cut);
-    const float tol = 1e-3f * hw;
-    const float i2 = -0.5f / q0;
-    xhi = fmaf(q1, yr, sqrtf(fmaxf(dr, 0.0f))) * i2 + tol;
-    xlo = fmaf(q1, yl, -sqrtf(fmaxf(dl, 0.0f))) * i2 - tol;
-}
 
 __global__ __launch_bounds__(64 * KE_WAVES) void kp_rect_kernel(const KpRec<float> *__restrict__ recs, int N,
                                                                 KpDev<float> P, float cutlog, float2 *__restrict__ out,
