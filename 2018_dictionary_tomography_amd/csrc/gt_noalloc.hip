@@ -21,6 +21,13 @@
 
 namespace gt {
 
+// gt_projector.hip
+int forward_derivs(const gt_atoms *atoms, const gt_geom *geom, const float *data, int order, float *R, double *f,
+                   double *g, double *H, void *ws, bool tiles, hipStream_t st);
+int check_forward_derivs(const gt_atoms *atoms, const gt_geom *geom, const float *data, int order, const float *R,
+                         const double *g);
+size_t forward_derivs_least(const gt_atoms *atoms, const gt_geom *geom);
+
 static __device__ __align__(256) unsigned char scratch[GT_NOALLOC_SCRATCH_BYTES];
 
 constexpr int NOALLOC_MAX_DEVICES = 64;
@@ -59,14 +66,17 @@ extern "C" int gt_forward_derivs_noalloc(const gt_atoms *atoms, const gt_geom *g
 {
     int rc;
     if ((rc = check_atoms(atoms)) || (rc = check_geom(geom, atoms->dim))) return rc;
-    const size_t need = gt_derivs_workspace(atoms, geom, GT_MODE_RESID);
+    const size_t need = forward_derivs_least(atoms, geom);
     if (need > GT_NOALLOC_SCRATCH_BYTES) {
         set_error("gt_forward_derivs_noalloc: %d atoms x %d angles need %zu bytes of scratch, above the %zu-byte "
                   "limit; call gt_forward_derivs with a workspace",
                   atoms->n, geom->nA, need, (size_t)GT_NOALLOC_SCRATCH_BYTES);
         return GT_EWORKSPACE;
     }
+    if ((rc = check_forward_derivs(atoms, geom, data, order, R, g))) return rc;
     void *ws = nullptr;
     if ((rc = scratch_address(&ws))) return rc;
-    return gt_forward_derivs(atoms, geom, data, order, R, f, g, H, ws, GT_NOALLOC_SCRATCH_BYTES, stream);
+    // f from the forward's tile sums where they fit as well
+    const bool tiles = gt_derivs_workspace(atoms, geom, GT_MODE_RESID) <= GT_NOALLOC_SCRATCH_BYTES;
+    return forward_derivs(atoms, geom, data, order, R, f, g, H, ws, tiles, (hipStream_t)stream);
 }

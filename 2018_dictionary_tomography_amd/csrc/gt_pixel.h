@@ -18,7 +18,9 @@ constexpr int MOMW = 32;  // floats per moment record
 //   MODE 1 (L2):     w1 = (aE - C) E, w2 = E^2, acc[30] += (aE-C)^2, acc[31] += C^2
 //   MODE 2 (resid):  w1 = C E, w2 = E^2
 // acc[15 + m] holds the w2 moments.  Ca points at this angle's [n0][n1] slab.
-template <int K, int MODE>
+// DEG: the highest degree taken; a gradient needs 2, a Hessian 4 and the w2
+// moments.  The sums that both take are formed in the same order.
+template <int K, int MODE, int DEG = 4>
 __device__ inline void pair_moments(const PairRec &rec, const float *__restrict__ p0, const float *__restrict__ p1,
                                     const float *__restrict__ Ca, int n1, int lane, float *acc)
 {
@@ -47,6 +49,8 @@ __device__ inline void pair_moments(const PairRec &rec, const float *__restrict_
             } else {
                 w1 = cv * E;
             }
+            constexpr bool W2 = MODE != GT_MODE_LINEAR && DEG == 4;
+            constexpr int NM = K == 2 ? (DEG + 1) * (DEG + 2) / 2 : DEG + 1;
             const float w2 = E * E;
             if (K == 2) {
                 const float x1 = dp0, y1 = dp1;
@@ -54,19 +58,19 @@ __device__ inline void pair_moments(const PairRec &rec, const float *__restrict_
                 const float mono[15] = {1.0f,    x1,      y1,      x2,      xy,      y2,      x2 * x1, x2 * y1,
                                         x1 * y2, y2 * y1, x2 * x2, x2 * xy, x2 * y2, xy * y2, y2 * y2};
 #pragma unroll
-                for (int m = 0; m < 15; m++) acc[m] = fmaf(w1, mono[m], acc[m]);
-                if (MODE != GT_MODE_LINEAR) {
+                for (int m = 0; m < NM; m++) acc[m] = fmaf(w1, mono[m], acc[m]);
+                if (W2) {
 #pragma unroll
-                    for (int m = 0; m < 15; m++) acc[15 + m] = fmaf(w2, mono[m], acc[15 + m]);
+                    for (int m = 0; m < NM; m++) acc[15 + m] = fmaf(w2, mono[m], acc[15 + m]);
                 }
             } else {
                 const float x1 = dp0, x2 = x1 * x1;
                 const float mono[5] = {1.0f, x1, x2, x2 * x1, x2 * x2};
 #pragma unroll
-                for (int m = 0; m < 5; m++) acc[m] = fmaf(w1, mono[m], acc[m]);
-                if (MODE != GT_MODE_LINEAR) {
+                for (int m = 0; m < NM; m++) acc[m] = fmaf(w1, mono[m], acc[m]);
+                if (W2) {
 #pragma unroll
-                    for (int m = 0; m < 5; m++) acc[15 + m] = fmaf(w2, mono[m], acc[15 + m]);
+                    for (int m = 0; m < NM; m++) acc[15 + m] = fmaf(w2, mono[m], acc[15 + m]);
                 }
             }
         }
@@ -222,18 +226,31 @@ __device__ inline float grid_step(const float *p, int n, int lane)
     return __ballot(!ok) == 0ull ? dx : 0.0f;
 }
 
+// Powers of a row's offset that a walk of degree DEG reads.
+template <int DEG> struct RowPow;
+template <> struct RowPow<4> {
+    using type = float4;
+    __device__ static inline float4 make(float x)
+    {
+        const float x2 = x * x;
+        return make_float4(x, x2, x2 * x, x2 * x2);
+    }
+};
+template <> struct RowPow<2> {
+    using type = float2;
+    __device__ static inline float2 make(float x) { return make_float2(x, x * x); }
+};
+
 // Row table of one pair over a window of H box rows, in the wave's LDS:
-// tab[r] = (x, x^2, x^3, x^4), x = dp0 of row row0 + r (the same FP32
-// expressions a pixel would evaluate).  Returns the spacing dx of a uniform
+// tab[r] = (x, x^2, x^3, x^4) (DEG 2: (x, x^2)), x = dp0 of row row0 + r (the same
+// FP32 expressions a pixel would evaluate).  Returns the spacing dx of a uniform
 // grid x(r) = x(0) + r dx that every row matches to within dx / 4, or 0 if
 // the rows are not such a grid (then no row span is derived from it).
-__device__ inline float row_table(const PairRec &rec, const float *p0, int row0, int H, int lane, float4 *tab)
+template <int DEG>
+__device__ inline float row_table(const PairRec &rec, const float *p0, int row0, int H, int lane,
+                                  typename RowPow<DEG>::type *tab)
 {
-    for (int r = lane; r < H; r += 64) {
-        const float x = (p0[row0 + r] - rec.c_hi[0]) - rec.c_lo[0];
-        const float x2 = x * x;
-        tab[r] = make_float4(x, x2, x2 * x, x2 * x2);
-    }
+    for (int r = lane; r < H; r += 64) tab[r] = RowPow<DEG>::make((p0[row0 + r] - rec.c_hi[0]) - rec.c_lo[0]);
     wave_sync();
     if (H < 2) return 0.0f;
     const float x0 = tab[0].x, dx = (tab[H - 1].x - x0) / (float)(H - 1);
@@ -343,9 +360,9 @@ __host__ __device__ inline bool support_meets_rect(const float4 &f1, const float
 // cut-off; what that adds is below 1e-13 of the sums, under their FP32
 // resolution.  The L2 energy terms, which do not vanish outside the support,
 // are taken for pixels inside it only.
-template <int MODE>
-__device__ inline void moment_pixel(const PairRec &rec, float cv, float4 xp, float rowlin, float colt, float *A,
-                                    float *B, float *acc)
+template <int MODE, int DEG>
+__device__ inline void moment_pixel(const PairRec &rec, float cv, typename RowPow<DEG>::type xp, float rowlin,
+                                    float colt, float *A, float *B, float *acc)
 {
     const float x = xp.x;
     const float q = fmaf(fmaf(rec.q[0], x, rowlin), x, colt);
@@ -363,15 +380,17 @@ __device__ inline void moment_pixel(const PairRec &rec, float cv, float4 xp, flo
     A[0] += w1;
     A[1] = fmaf(w1, xp.x, A[1]);
     A[2] = fmaf(w1, xp.y, A[2]);
-    A[3] = fmaf(w1, xp.z, A[3]);
-    A[4] = fmaf(w1, xp.w, A[4]);
-    if (MODE != GT_MODE_LINEAR) {
-        const float w2 = E * E;
-        B[0] += w2;
-        B[1] = fmaf(w2, xp.x, B[1]);
-        B[2] = fmaf(w2, xp.y, B[2]);
-        B[3] = fmaf(w2, xp.z, B[3]);
-        B[4] = fmaf(w2, xp.w, B[4]);
+    if constexpr (DEG == 4) {
+        A[3] = fmaf(w1, xp.z, A[3]);
+        A[4] = fmaf(w1, xp.w, A[4]);
+        if (MODE != GT_MODE_LINEAR) {
+            const float w2 = E * E;
+            B[0] += w2;
+            B[1] = fmaf(w2, xp.x, B[1]);
+            B[2] = fmaf(w2, xp.y, B[2]);
+            B[3] = fmaf(w2, xp.z, B[3]);
+            B[4] = fmaf(w2, xp.w, B[4]);
+        }
     }
 }
 
@@ -380,10 +399,10 @@ __device__ inline void moment_pixel(const PairRec &rec, float cv, float4 xp, flo
 // offset of its row and its row-table entry advance once per group of UNR
 // rows; the rows of a group sit at wave-uniform distances (u step rows) from
 // them, which the residual loads take as their scalar offsets.
-template <int MODE, int UNR, int RS>
+template <int MODE, int UNR, int RS, int DEG>
 __device__ inline void moment_rows(const PairRec &rec, __amdgpu_buffer_rsrc_t crs, unsigned off, unsigned rowb,
-                                   const float4 *trow, int step_, int r0, int he, float rowlin, float colt, float *A,
-                                   float *B, float *acc)
+                                   const typename RowPow<DEG>::type *trow, int step_, int r0, int he, float rowlin,
+                                   float colt, float *A, float *B, float *acc)
 {
     const int step = RS > 0 ? RS : step_;
     const unsigned gstep = (unsigned)step * rowb;
@@ -391,7 +410,7 @@ __device__ inline void moment_rows(const PairRec &rec, __amdgpu_buffer_rsrc_t cr
     const int last = he - (UNR - 1) * step;
     for (; r0 <= last; r0 += UNR * step) {
         float cv[UNR];
-        float4 xp[UNR];
+        typename RowPow<DEG>::type xp[UNR];
 #pragma unroll
         for (int u = 0; u < UNR; u++) {
             cv[u] = buffer_load_f32(crs, off, (unsigned)u * gstep);
@@ -400,12 +419,12 @@ __device__ inline void moment_rows(const PairRec &rec, __amdgpu_buffer_rsrc_t cr
         off += UNR * gstep;
         trow += UNR * step;
 #pragma unroll
-        for (int u = 0; u < UNR; u++) moment_pixel<MODE>(rec, cv[u], xp[u], rowlin, colt, A, B, acc);
+        for (int u = 0; u < UNR; u++) moment_pixel<MODE, DEG>(rec, cv[u], xp[u], rowlin, colt, A, B, acc);
     }
     // remaining rows one at a time (same row order)
     for (; r0 <= he; r0 += step) {
         const float cv = buffer_load_f32(crs, off, 0u);
-        moment_pixel<MODE>(rec, cv, *trow, rowlin, colt, A, B, acc);
+        moment_pixel<MODE, DEG>(rec, cv, *trow, rowlin, colt, A, B, acc);
         off += gstep;
         trow += step;
     }
@@ -429,9 +448,10 @@ constexpr int MOM_CHUNK = 32;
 // of it: the pixels left out are outside the support, where the full walk
 // adds exact zeros, so the sums are those of walking the whole box.  UNR rows are loaded per step (more rows in flight
 // hide load latency when few waves share a SIMD).
-template <int MODE, int UNR, int TROWS>
+template <int MODE, int UNR, int TROWS, int DEG = 4>
 __device__ inline void pair_moments_rows(const PairRec &rec, const float *p0, const float *p1,
-                                         const float *__restrict__ Ca, int n1, int lane, float *acc, float4 *tab)
+                                         const float *__restrict__ Ca, int n1, int lane, float *acc,
+                                         typename RowPow<DEG>::type *tab)
 {
     const int W = rec.hi[1] - rec.lo[1] + 1;
     const int Hbox = rec.hi[0] - rec.lo[0] + 1;
@@ -445,7 +465,7 @@ __device__ inline void pair_moments_rows(const PairRec &rec, const float *p0, co
         const int H = min(TROWS, Hbox - w0);
         const int row0 = rec.lo[0] + w0;
         if (w0 > 0) wave_sync();  // the previous window's table is no longer read
-        const float dx = row_table(rec, p0, row0, H, lane, tab);
+        const float dx = row_table<DEG>(rec, p0, row0, H, lane, tab);
         const float x0 = tab[0].x, inv_dx = span_inv_dx(dx), inv2a = span_inv2a(rec);
         for (int cb = 0; cb < W; cb += MOM_CHUNK) {
             ColChunk cc;
@@ -468,18 +488,18 @@ __device__ inline void pair_moments_rows(const PairRec &rec, const float *p0, co
             // two row phases (chunks of 32 columns, the common case): the
             // row-table reads of a group take immediate offsets
             if (cc.R == 2)
-                moment_rows<MODE, UNR, 2>(rec, crs, off, rowb, tab + r0, 2, r0, he, rowlin, colt, A, B, acc);
+                moment_rows<MODE, UNR, 2, DEG>(rec, crs, off, rowb, tab + r0, 2, r0, he, rowlin, colt, A, B, acc);
             else
-                moment_rows<MODE, UNR, 0>(rec, crs, off, rowb, tab + r0, cc.R, r0, he, rowlin, colt, A, B, acc);
+                moment_rows<MODE, UNR, 0, DEG>(rec, crs, off, rowb, tab + r0, cc.R, r0, he, rowlin, colt, A, B, acc);
             const float y2 = dp1 * dp1;
             const float yp[5] = {1.0f, dp1, y2, y2 * dp1, y2 * y2};
 #pragma unroll
-            for (int i = 0; i <= 4; i++)
+            for (int i = 0; i <= DEG; i++)
 #pragma unroll
-                for (int j = 0; i + j <= 4; j++) {
+                for (int j = 0; i + j <= DEG; j++) {
                     const int m = (i + j) * (i + j + 1) / 2 + j;
                     acc[m] = fmaf(A[i], yp[j], acc[m]);
-                    if (MODE != GT_MODE_LINEAR) acc[15 + m] = fmaf(B[i], yp[j], acc[15 + m]);
+                    if (MODE != GT_MODE_LINEAR && DEG == 4) acc[15 + m] = fmaf(B[i], yp[j], acc[15 + m]);
                 }
         }
     }
@@ -524,9 +544,9 @@ __device__ inline void pair_moments_box(const PairRec &rec, const float *p0, con
             const int r0 = cc.ro;
             const unsigned off = 4u * ((unsigned)(row0 + r0) * (unsigned)n1 + (unsigned)i1);
             if (cc.R == 2)
-                moment_rows<MODE, UNR, 2>(rec, crs, off, rowb, tab + r0, 2, r0, H - 1, rowlin, colt, A, B, acc);
+                moment_rows<MODE, UNR, 2, 4>(rec, crs, off, rowb, tab + r0, 2, r0, H - 1, rowlin, colt, A, B, acc);
             else
-                moment_rows<MODE, UNR, 0>(rec, crs, off, rowb, tab + r0, cc.R, r0, H - 1, rowlin, colt, A, B, acc);
+                moment_rows<MODE, UNR, 0, 4>(rec, crs, off, rowb, tab + r0, cc.R, r0, H - 1, rowlin, colt, A, B, acc);
             const float y2 = dp1 * dp1;
             const float yp[5] = {1.0f, dp1, y2, y2 * dp1, y2 * y2};
 #pragma unroll

@@ -17,6 +17,8 @@
 // __RadProj (NewtonBases2D.py:284-296), __L2derivs_RadProj_aniso_3D and
 // __derivs_RadProj_aniso_3D (NewtonBases.py:792-870, 993-1069) and their 2D
 // versions (NewtonBases2D.py:329-401, 444-515).
+#include <algorithm>
+
 #include "gt_pixel.h"
 
 namespace gt {
@@ -26,7 +28,6 @@ constexpr int CHUNK = 256;
 constexpr int MOM_STRIDE = 32;  // floats per (atom, angle) moment record
 constexpr int MOM_TROWS = 512;  // rows of a moments wave's row table
 constexpr int MOM_WAVES = 1;    // waves (pairs) per moments block
-static_assert(MOM_TROWS * 16 <= 64 * (MOM_STRIDE + 1) * 4, "row table must fit the reduction slab");
 constexpr int MODE_LINEAR = GT_MODE_LINEAR, MODE_L2 = GT_MODE_L2, MODE_RESID = GT_MODE_RESID;
 
 __device__ inline void kahan_add(float &s, float &c, float v)
@@ -213,11 +214,12 @@ __device__ inline void f3_values(const float4 &f0, const float4 &f1, const float
     vB = f0.x * eB;
 }
 
-__global__ __launch_bounds__(F3_WAVES * 64) void forward3_kernel(const PairRec *__restrict__ recs, int N, int nA,
+// (at most 64 VGPRs: eight waves per SIMD)
+__global__ __launch_bounds__(F3_WAVES * 64) __attribute__((amdgpu_waves_per_eu(8))) void forward3_kernel(const PairRec *__restrict__ recs, int N, int nA,
                                                                  int n0, int n1, const float *__restrict__ p0,
                                                                  const float *__restrict__ p1, float *__restrict__ R,
                                                                  const float *__restrict__ sub, int e0, int e1,
-                                                                 int sorted)
+                                                                 int sorted, double *__restrict__ part)
 {
     __shared__ PairRec list[F3_CHUNK];
     __shared__ alignas(16) unsigned short wl[F3_WAVES][F3_CHUNK];  // 8-byte reads of 4 indices
@@ -291,11 +293,17 @@ __global__ __launch_bounds__(F3_WAVES * 64) void forward3_kernel(const PairRec *
         __syncthreads();
     }
     // R = projection, or projection - sub (the residual) when sub is given
+    float vA = 0.0f, vB = 0.0f;
     if (i1 < n1) {
         const size_t oA = ((size_t)a * n0 + rA) * n1 + i1, oB = ((size_t)a * n0 + rB) * n1 + i1;
-        if (rA < n0) R[oA] = sub ? (float)sA - sub[oA] : (float)sA;
-        if (rB < n0) R[oB] = sub ? (float)sB - sub[oB] : (float)sB;
+        if (rA < n0) R[oA] = vA = sub ? (float)sA - sub[oA] : (float)sA;
+        if (rB < n0) R[oB] = vB = sub ? (float)sB - sub[oB] : (float)sB;
     }
+    if (!part) return;
+    // sum of squares of the wave's rectangle, for the l2 value of the residual
+    const double q = wave_sum_f64((double)vA * vA + (double)vB * vB);
+    if (lane == 0)
+        part[(((size_t)a * tilesR + row0 / TILE_ROWS) * tilesC + col0 / TILE_COLS) * F3_WAVES + wave] = q;
 }
 
 // ---------------------------------------------------------------------------
@@ -303,7 +311,7 @@ __global__ __launch_bounds__(F3_WAVES * 64) void forward3_kernel(const PairRec *
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void forward2_kernel(const PairRec *__restrict__ recs, int N, int n0,
                                                        const float *__restrict__ p0, float *__restrict__ R,
-                                                       const float *__restrict__ sub)
+                                                       const float *__restrict__ sub, double *__restrict__ part)
 {
     __shared__ PairRec list[CHUNK];
     __shared__ int wcnt[4];
@@ -328,59 +336,110 @@ __global__ __launch_bounds__(256) void forward2_kernel(const PairRec *__restrict
         }
         __syncthreads();
     }
-    if (i0 < n0) R[(size_t)a * n0 + i0] = sub ? s - sub[(size_t)a * n0 + i0] : s;
+    float v = 0.0f;
+    if (i0 < n0) R[(size_t)a * n0 + i0] = v = sub ? s - sub[(size_t)a * n0 + i0] : s;
+    if (!part) return;
+    const double q2 = wave_sum_f64((double)v * v);
+    if ((threadIdx.x & 63) == 0) part[((size_t)a * gridDim.x + blockIdx.x) * 4 + wave] = q2;
 }
 
 // ---------------------------------------------------------------------------
 // moments
 // ---------------------------------------------------------------------------
+// f = 1/2 sum of the forward's n partial sums of squares, in a fixed order: one
+// wave of the moments grid adds PART_CHUNK of them in place (16 loads in flight
+// per lane), one block the n / PART_CHUNK results.
+constexpr int PART_CHUNK = 1024;
+__device__ inline void chunk_sum(double *__restrict__ part, size_t n, size_t chunk, int lane)
+{
+    double *p = part + chunk * PART_CHUNK;
+    const int m = (int)(n - chunk * PART_CHUNK < PART_CHUNK ? n - chunk * PART_CHUNK : PART_CHUNK);
+    double v[16];
+#pragma unroll
+    for (int u = 0; u < 16; u++) v[u] = p[std::min(lane + 64 * u, m - 1)];
+    double s[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int u = 0; u < 16; u++) s[u & 3] += lane + 64 * u < m ? v[u] : 0.0;
+    const double t = wave_sum_f64((s[0] + s[1]) + (s[2] + s[3]));
+    if (lane == 0) p[0] = t;  // read by this wave only, before
+}
+__device__ inline void half_sum(const double *__restrict__ sums, size_t n, size_t stride, double *__restrict__ f,
+                                int nthr, double *red)
+{
+    double s = 0.0;
+    for (size_t i = threadIdx.x; i < n; i += nthr) s += sums[i * stride];
+    const double t = wave_sum_f64(s);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = t;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double v = 0.0;
+        for (int w = 0; w < nthr / 64; w++) v += red[w];
+        f[0] = 0.5 * v;
+    }
+}
+__global__ __launch_bounds__(64) void chunk_sum_kernel(double *__restrict__ part, size_t n)
+{
+    chunk_sum(part, n, blockIdx.x, threadIdx.x);
+}
+__global__ __launch_bounds__(512) void half_sum_kernel(const double *__restrict__ sums, size_t n, size_t stride,
+                                                       double *__restrict__ f)
+{
+    __shared__ double red[8];
+    half_sum(sums, n, stride, f, 512, red);
+}
+
 // Layout of one moment record (32 floats): [0, NM) sum w1 mono, [15, 15+NM)
-// sum E^2 mono, [30] sum_fp (alpha E - C)^2, [31] sum_fp C^2 (L2 mode).
-template <int K, int MODE>
-__global__ __launch_bounds__(64 * MOM_WAVES) void moments_kernel(const PairRec *__restrict__ recs, int N, int nA,
+// sum E^2 mono, [30] sum_fp (alpha E - C)^2, [31] sum_fp C^2 (L2 mode).  Order 1
+// takes the degrees up to 2 of the first only (the rest is zero): a gradient
+// needs 6 of the 30 moments (3 of 10 on a 1D detector).  5000 atoms, 90 x 256^2,
+// linear mode: 2.08 -> 1.58 ms, the last 0.12 of it from 64 registers instead of
+// 86 (eight waves per SIMD; order 2's reduction slab allows five).
+template <int K, int MODE, int ORDER>
+__global__ __launch_bounds__(64 * MOM_WAVES, ORDER == 1 ? 8 : 1) void moments_kernel(const PairRec *__restrict__ recs, int N, int nA,
                                                                  int n0, int n1, const float *__restrict__ p0,
                                                                  const float *__restrict__ p1,
-                                                                 const float *__restrict__ C, float *__restrict__ mom)
+                                                                 const float *__restrict__ C, float *__restrict__ mom,
+                                                                 double *__restrict__ part, size_t nparts)
 {
+    constexpr int NV = ORDER == 2 ? MOM_STRIDE : 8, DEG = ORDER == 2 ? 4 : 2;  // values summed, highest degree
+    using Row = typename RowPow<DEG>::type;
     // the reduction slab of a wave doubles as its row table while it walks
-    // its pair (MOM_TROWS float4 = 8 KiB of the 8.25 KiB slab)
-    __shared__ alignas(16) float red[MOM_WAVES][64][MOM_STRIDE + 1];
+    // its pair (order 2: 8 KiB of the 8.25 KiB slab; order 1: 4 KiB)
+    constexpr size_t SLAB = std::max(64 * (NV + 1) * sizeof(float), MOM_TROWS * sizeof(Row));
+    __shared__ alignas(16) char slab[MOM_WAVES][SLAB];
     // the wave index is uniform: scalar pair index, record and slab base
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const long pair = (long)blockIdx.x * MOM_WAVES + wave;
     const bool valid = pair < (long)N * nA;
+    if (!valid) {  // the waves past the pairs: f's partial sums
+        const size_t chunk = (size_t)(pair - (long)N * nA);
+        if (chunk * PART_CHUNK < nparts) chunk_sum(part, nparts, chunk, lane);
+        return;
+    }
     float acc[MOM_STRIDE];
 #pragma unroll
     for (int v = 0; v < MOM_STRIDE; v++) acc[v] = 0.0f;
-    if (valid) {
-        const PairRec rec = recs[pair];
-        const int a = (int)(pair / N);
-        if (K == 2)
-            pair_moments_rows<MODE, 4, MOM_TROWS>(rec, p0, p1, C + (size_t)a * n0 * n1, n1, lane, acc,
-                                                  reinterpret_cast<float4 *>(&red[wave][0][0]));
-        else
-            pair_moments<K, MODE>(rec, p0, p1, C + (size_t)a * n0 * n1, n1, lane, acc);
-    }
+    const PairRec rec = recs[pair];
+    const int a = (int)(pair / N);
+    if (K == 2)
+        pair_moments_rows<MODE, 4, MOM_TROWS, DEG>(rec, p0, p1, C + (size_t)a * n0 * n1, n1, lane, acc,
+                                                   reinterpret_cast<Row *>(slab[wave]));
+    else
+        pair_moments<K, MODE, DEG>(rec, p0, p1, C + (size_t)a * n0 * n1, n1, lane, acc);
     // each wave reduces its own slab: no block barrier, so a wave whose pair
     // is done does not wait for the others of its block
+    float (*red)[NV + 1] = reinterpret_cast<float (*)[NV + 1]>(slab[wave]);
 #pragma unroll
-    for (int v = 0; v < MOM_STRIDE; v++) red[wave][lane][v] = acc[v];
+    for (int v = 0; v < NV; v++) red[lane][v] = acc[ORDER == 2 || v < 6 ? v : 24 + v];
     wave_sync();
-    if (valid) {
-        const int col = lane & 31, half = lane >> 5;
-        float s = 0.0f;
-        for (int i = 0; i < 32; i++) s += red[wave][half * 32 + i][col];
-        s += __shfl_xor(s, 32);
-        if (lane < 32) mom[pair * MOM_STRIDE + lane] = s;
-    }
-}
-
-// f = 1/2 sum over angles of the per-angle FP64 sums of squares (one thread).
-__global__ void half_total_kernel(const double *__restrict__ per, int n, double *__restrict__ f)
-{
-    double s = 0.0;
-    for (int a = 0; a < n; a++) s += per[a];
-    f[0] = 0.5 * s;
+    // (the same order of additions for both orders: equal gradients)
+    const int col = lane & 31, half = lane >> 5;
+    const int v = ORDER == 2 || col < 6 ? col : col - 24;  // its value's slot (order 1: 0..5, 30, 31)
+    float s = 0.0f;
+    if (v >= 0 && v < NV && (ORDER == 2 || col < 6 || col >= 30))
+        for (int i = 0; i < 32; i++) s += red[half * 32 + i][v];
+    s += __shfl_xor(s, 32);
+    if (half == 0) mom[pair * MOM_STRIDE + col] = s;
 }
 
 // FP64 sum of C^2 per angle (the L2 value of the pixels outside every footprint).
@@ -405,11 +464,15 @@ __global__ __launch_bounds__(256) void sumsq_kernel(const float *__restrict__ C,
 // ---------------------------------------------------------------------------
 // finish
 // ---------------------------------------------------------------------------
+// With part given, one block more, the first: f from the forward's partial sums.
+// One kernel for both orders, so that the gradient is formed by the same
+// instructions and an order-1 call returns the bits of an order-2 one.
 template <int D, int MODE>
 __global__ __launch_bounds__(64) void finish_kernel(gt_atoms A, gt_geom G, const PairRec *__restrict__ recs,
                                                     const float *__restrict__ mom, const double *__restrict__ sumC2,
                                                     int want_hess, double *__restrict__ fo, double *__restrict__ go,
-                                                    double *__restrict__ Ho)
+                                                    double *__restrict__ Ho, const double *__restrict__ part,
+                                                    size_t nparts, double *__restrict__ ftotal)
 {
     using Dm = Dims<D>;
     constexpr int P = Dm::P, NM = Dm::NM, NH = P * (P + 1) / 2, NV = 1 + P + NH;
@@ -417,8 +480,12 @@ __global__ __launch_bounds__(64) void finish_kernel(gt_atoms A, gt_geom G, const
     // accumulates its pairs' Hessian entries there directly (a P x P array
     // per lane in registers would spill)
     __shared__ double red[64][NV + 1];
-    const int j = blockIdx.x, lane = threadIdx.x;
+    const int j = (int)blockIdx.x - (part ? 1 : 0), lane = threadIdx.x;
     const int N = A.n;
+    if (j < 0) {
+        half_sum(part, (nparts + PART_CHUNK - 1) / PART_CHUNK, PART_CHUNK, ftotal, 64, &red[0][0]);
+        return;
+    }
     double grad[P], F = 0.0;
     for (int i = 0; i < P; i++) grad[i] = 0.0;
     double *row = red[lane];
@@ -560,8 +627,15 @@ __global__ void negate_kernel(float *__restrict__ R, const float *__restrict__ s
 
 // Forward projection from precomputed records (used by the fitters too);
 // with sub != NULL the result is the residual projection - sub.
+// part (with n > 0): receives the forward_parts() sums of squares, one per wave.
+static size_t forward_parts(const gt_geom *G)
+{
+    if (G->dim == 3)
+        return (size_t)F3_WAVES * G->nA * ((G->n0 + TILE_ROWS - 1) / TILE_ROWS) * ((G->n1 + TILE_COLS - 1) / TILE_COLS);
+    return (size_t)4 * G->nA * ((G->n0 + 255) / 256);
+}
 int launch_forward(const gt_atoms *A, const gt_geom *G, const PairRec *recs, float *R, hipStream_t st,
-                   const float *sub)
+                   const float *sub, double *part)
 {
     const size_t nout = (size_t)G->nA * G->n0 * G->n1;
     if (A->n == 0) {
@@ -578,32 +652,36 @@ int launch_forward(const gt_atoms *A, const gt_geom *G, const PairRec *recs, flo
         GT_CHECK_ARG(blocks < (1ull << 31), "forward: too many detector tiles (%d x %d, %d angles)", G->n0, G->n1,
                      G->nA);
         launch_timed(GT_K_FORWARD, forward3_kernel, dim3((unsigned)blocks), dim3(F3_WAVES * 64), 0, st, recs, A->n,
-                     G->nA, G->n0, G->n1, G->p0, G->p1, R, sub, e0, e1, G->sorted);
+                     G->nA, G->n0, G->n1, G->p0, G->p1, R, sub, e0, e1, G->sorted, part);
     } else {
         const int tiles = (G->n0 + 255) / 256;
         launch_timed(GT_K_FORWARD, forward2_kernel, dim3(tiles, G->nA), dim3(256), 0, st, recs, A->n, G->n0, G->p0, R,
-                     sub);
+                     sub, part);
     }
     GT_HIP(hipGetLastError());
     return 0;
 }
 
-template <int D, int MODE>
+template <int D, int MODE, int ORDER>
 static void launch_deriv_kernels(const gt_atoms *A, const gt_geom *G, const PairRec *recs, float *mom,
-                                 const double *sumC2, const float *C, int want_hess, double *f, double *g, double *H,
-                                 hipStream_t st)
+                                 const double *sumC2, const float *C, double *f, double *g, double *H,
+                                 double *part, double *ftotal, hipStream_t st)
 {
     constexpr int K = D - 1;
     const long pairs = (long)A->n * G->nA;
-    launch_timed(GT_K_MOMENTS, moments_kernel<K, MODE>, dim3((unsigned)((pairs + MOM_WAVES - 1) / MOM_WAVES)),
+    const size_t nparts = part ? forward_parts(G) : 0;
+    const size_t waves = (size_t)pairs + (nparts + PART_CHUNK - 1) / PART_CHUNK;
+    launch_timed(GT_K_MOMENTS, moments_kernel<K, MODE, ORDER>, dim3((unsigned)((waves + MOM_WAVES - 1) / MOM_WAVES)),
                  dim3(64 * MOM_WAVES), 0, st, recs,
-                 A->n, G->nA, G->n0, G->n1, G->p0, G->p1, C, mom);
-    launch_timed(GT_K_FINISH, finish_kernel<D, MODE>, dim3(A->n), dim3(64), 0, st, *A, *G, recs, mom, sumC2, want_hess,
-                 f, g, H);
+                 A->n, G->nA, G->n0, G->n1, G->p0, G->p1, C, mom, part, nparts);
+    launch_timed(GT_K_FINISH, finish_kernel<D, MODE>, dim3(A->n + (part ? 1 : 0)), dim3(64), 0, st, *A, *G, recs,
+                 mom, sumC2, ORDER == 2 ? 1 : 0, f, g, H, part, nparts, ftotal);
 }
 
+// part, ftotal (residual mode): the forward's partial sums and where f goes.
 int launch_derivs(const gt_atoms *A, const gt_geom *G, const PairRec *recs, float *mom, double *sumC2,
-                  const float *C, int mode, int want_hess, double *f, double *g, double *H, hipStream_t st)
+                  const float *C, int mode, int want_hess, double *f, double *g, double *H, hipStream_t st,
+                  double *part = nullptr, double *ftotal = nullptr)
 {
     if (A->n == 0) return 0;
     GT_CHECK_ARG((long)A->n * G->nA / 4 < (1L << 31), "too many (atom, angle) pairs for one launch");
@@ -611,10 +689,14 @@ int launch_derivs(const gt_atoms *A, const gt_geom *G, const PairRec *recs, floa
         hipLaunchKernelGGL(sumsq_kernel, dim3(G->nA), dim3(256), 0, st, C, (long)G->n0 * G->n1, sumC2);
     }
     const int D = G->dim;
-#define GT_DISPATCH(DD, MM)                                                                             \
-    if (D == DD && mode == MM)                                                                          \
-        launch_deriv_kernels<DD, MM>(A, G, recs, mom, sumC2, C, want_hess, (mode == MODE_RESID) ? nullptr : f, g, \
-                                     H, st);
+    if (mode == MODE_RESID) f = nullptr;
+#define GT_DISPATCH(DD, MM)                                                                               \
+    if (D == DD && mode == MM) {                                                                          \
+        if (want_hess)                                                                                    \
+            launch_deriv_kernels<DD, MM, 2>(A, G, recs, mom, sumC2, C, f, g, H, part, ftotal, st);        \
+        else                                                                                              \
+            launch_deriv_kernels<DD, MM, 1>(A, G, recs, mom, sumC2, C, f, g, nullptr, part, ftotal, st);  \
+    }
     GT_DISPATCH(3, MODE_LINEAR)
     GT_DISPATCH(3, MODE_L2)
     GT_DISPATCH(3, MODE_RESID)
@@ -622,6 +704,32 @@ int launch_derivs(const gt_atoms *A, const gt_geom *G, const PairRec *recs, floa
     GT_DISPATCH(2, MODE_L2)
     GT_DISPATCH(2, MODE_RESID)
 #undef GT_DISPATCH
+    GT_HIP(hipGetLastError());
+    return 0;
+}
+
+// Residual projection - data in R and, when f is given, f = 1/2 |R|^2: its sums
+// of squares per tile go to part (forward_parts() doubles); without room for
+// them (part NULL) or without atoms, per angle to sumC2, by a pass of their own.
+// total: also add them up; else the moments and finish kernels do (only with
+// part and atoms).
+static int launch_residual(const gt_atoms *A, const gt_geom *G, const PairRec *recs, const float *data, float *R,
+                           double *f, double *part, double *sumC2, bool total, hipStream_t st)
+{
+    int rc;
+    const bool tiles = f && part && A->n > 0;
+    if ((rc = launch_forward(A, G, recs, R, st, data, tiles ? part : nullptr))) return rc;
+    if (!f) return 0;
+    if (tiles) {
+        if (total) {
+            const size_t n = forward_parts(G), chunks = (n + PART_CHUNK - 1) / PART_CHUNK;
+            hipLaunchKernelGGL(chunk_sum_kernel, dim3((unsigned)chunks), dim3(64), 0, st, part, n);
+            hipLaunchKernelGGL(half_sum_kernel, dim3(1), dim3(512), 0, st, part, chunks, (size_t)PART_CHUNK, f);
+        }
+    } else {
+        hipLaunchKernelGGL(sumsq_kernel, dim3(G->nA), dim3(256), 0, st, R, (long)G->n0 * G->n1, sumC2);
+        hipLaunchKernelGGL(half_sum_kernel, dim3(1), dim3(512), 0, st, sumC2, (size_t)G->nA, (size_t)1, f);
+    }
     GT_HIP(hipGetLastError());
     return 0;
 }
@@ -651,14 +759,17 @@ extern "C" int gt_forward(const gt_atoms *atoms, const gt_geom *geom, float *R, 
     hipStream_t st = (hipStream_t)stream;
     PairRec *recs = (PairRec *)ws;
     if ((rc = launch_setup(atoms, geom, recs, st))) return rc;
-    return launch_forward(atoms, geom, recs, R, st, nullptr);
+    return launch_forward(atoms, geom, recs, R, st, nullptr, nullptr);
 }
+
+static size_t ang_bytes(const gt_geom *G) { return align_up((size_t)G->nA * sizeof(double)); }
+static size_t part_bytes(const gt_geom *G) { return align_up(forward_parts(G) * sizeof(double)); }
+static size_t derivs_bytes(const gt_atoms *A, const gt_geom *G) { return rec_bytes(A, G) + mom_bytes(A, G) + ang_bytes(G); }
 
 extern "C" size_t gt_derivs_workspace(const gt_atoms *atoms, const gt_geom *geom, int mode)
 {
-    (void)mode;
     if (!atoms || !geom) return 0;
-    return rec_bytes(atoms, geom) + mom_bytes(atoms, geom) + align_up((size_t)geom->nA * sizeof(double));
+    return derivs_bytes(atoms, geom) + (mode == GT_MODE_RESID ? part_bytes(geom) : 0);
 }
 
 extern "C" int gt_derivs(const gt_atoms *atoms, const gt_geom *geom, const float *C, int mode, int order, double *f,
@@ -686,8 +797,25 @@ extern "C" int gt_derivs(const gt_atoms *atoms, const gt_geom *geom, const float
     return launch_derivs(atoms, geom, recs, mom, sumC2, C, mode, order > 1, f, g, H, st);
 }
 
-extern "C" int gt_forward_derivs(const gt_atoms *atoms, const gt_geom *geom, const float *data, int order, float *R,
-                                 double *f, double *g, double *H, void *ws, size_t ws_bytes, void *stream)
+namespace gt {
+// gt_forward_derivs with a workspace of derivs_bytes() or, with the tile sums of
+// f (`tiles`), of gt_derivs_workspace() bytes.
+int forward_derivs(const gt_atoms *atoms, const gt_geom *geom, const float *data, int order, float *R, double *f,
+                   double *g, double *H, void *ws, bool tiles, hipStream_t st)
+{
+    int rc;
+    char *w = (char *)ws;
+    PairRec *recs = (PairRec *)w;
+    float *mom = (float *)(w + rec_bytes(atoms, geom));
+    double *sumC2 = (double *)(w + rec_bytes(atoms, geom) + mom_bytes(atoms, geom));
+    double *part = tiles && f && atoms->n > 0 ? (double *)(w + derivs_bytes(atoms, geom)) : nullptr;
+    if ((rc = launch_setup(atoms, geom, recs, st))) return rc;
+    if ((rc = launch_residual(atoms, geom, recs, data, R, f, part, sumC2, false, st))) return rc;
+    return launch_derivs(atoms, geom, recs, mom, sumC2, R, GT_MODE_RESID, order > 1, nullptr, g, H, st, part, f);
+}
+
+int check_forward_derivs(const gt_atoms *atoms, const gt_geom *geom, const float *data, int order, const float *R,
+                         const double *g)
 {
     int rc;
     if ((rc = check_atoms(atoms)) || (rc = check_geom(geom, atoms->dim))) return rc;
@@ -696,23 +824,22 @@ extern "C" int gt_forward_derivs(const gt_atoms *atoms, const gt_geom *geom, con
     GT_CHECK_ARG(R != nullptr, "gt_forward_derivs: R is NULL");
     GT_CHECK_ARG(g != nullptr || atoms->n == 0, "gt_forward_derivs: g is NULL");
     GT_CHECK_ARG(R != data, "gt_forward_derivs: R must not alias data");
+    return 0;
+}
+
+size_t forward_derivs_least(const gt_atoms *atoms, const gt_geom *geom) { return derivs_bytes(atoms, geom); }
+}  // namespace gt
+
+extern "C" int gt_forward_derivs(const gt_atoms *atoms, const gt_geom *geom, const float *data, int order, float *R,
+                                 double *f, double *g, double *H, void *ws, size_t ws_bytes, void *stream)
+{
+    int rc;
+    if ((rc = check_forward_derivs(atoms, geom, data, order, R, g))) return rc;
     const size_t need = gt_derivs_workspace(atoms, geom, GT_MODE_RESID);
     if (need > ws_bytes || (need > 0 && ws == nullptr)) {
         set_error("gt_forward_derivs: workspace of %zu bytes given, %zu needed", ws_bytes, need);
         return GT_EWORKSPACE;
     }
     GT_CHECK_ARG(((uintptr_t)ws & 63) == 0, "gt_forward_derivs: workspace must be 64-byte aligned");
-    hipStream_t st = (hipStream_t)stream;
-    char *w = (char *)ws;
-    PairRec *recs = (PairRec *)w;
-    float *mom = (float *)(w + rec_bytes(atoms, geom));
-    double *sumC2 = (double *)(w + rec_bytes(atoms, geom) + mom_bytes(atoms, geom));
-    if ((rc = launch_setup(atoms, geom, recs, st))) return rc;
-    if ((rc = launch_forward(atoms, geom, recs, R, st, data))) return rc;
-    if (f) {
-        hipLaunchKernelGGL(sumsq_kernel, dim3(geom->nA), dim3(256), 0, st, R, (long)geom->n0 * geom->n1, sumC2);
-        hipLaunchKernelGGL(half_total_kernel, dim3(1), dim3(1), 0, st, sumC2, geom->nA, f);
-        GT_HIP(hipGetLastError());
-    }
-    return launch_derivs(atoms, geom, recs, mom, sumC2, R, GT_MODE_RESID, order > 1, nullptr, g, H, st);
+    return forward_derivs(atoms, geom, data, order, R, f, g, H, ws, true, (hipStream_t)stream);
 }

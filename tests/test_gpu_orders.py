@@ -1,0 +1,72 @@
+"""Gradient-only derivatives and the l2 value from the forward's partial sums.
+
+order=1 takes fewer moments per (atom, angle) pair than order=2 and adds the
+ones it takes in the same order, so the gradient has the same bits.  f is the
+FP64 sum of squares of the float32 residual that the call returns: n positive
+FP64 terms, so any order of additions is within n eps of any other."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+EPS = 2.0 ** -52
+
+# (dim, detector, angles, atoms, isotropic): one partial tile, ragged tiles, a
+# detector of more rows than the row table holds, 2.5D; partial sums below one
+# chunk of 1024, exactly one (256 angles x 4 waves) and one and a remainder
+CASES = [
+    ("2d", (5,), 1, 1, True),
+    ("2d", (100,), 256, 3, True),
+    ("2d", (257,), 257, 4, False),
+    ("2d", (1300,), 65, 2, True),
+    ("3d", (7, 5), 2, 3, True),
+    ("3d", (33, 65), 67, 5, False),
+    ("3d", (640, 24), 3, 2, False),
+    ("2.5d", (40, 31), 9, 6, False),
+]
+
+
+def _problem(gt, case, dev):
+    kind, det, nA, N, iso = case
+    rng = np.random.default_rng(N + nA)
+    D = 2 if kind == "2d" else 3
+    axes = tuple(gt.cell_centres(-1.1, 1.1, n) for n in det)
+    if kind == "3d":
+        from importlib import import_module
+
+        T, ortho, _ = import_module("2018_dictionary_tomography_amd.workloads").tilt_series(nA, 60.0, det=16)
+        space = gt.ProjSpace(orientations=T, ortho=ortho, detector=axes)
+    else:
+        space = gt.ProjSpace(angles=np.linspace(0, np.pi, nA, endpoint=False), detector=axes)
+    P = 1 if iso else D * (D + 1) // 2
+    r = np.full((N, P), 3.0)
+    if not iso:
+        r[:] = rng.normal(scale=0.5, size=r.shape)
+        r[:, :D] = 2.0 + rng.random((N, D)) * 4.0
+    r[0, :D] = 1.0  # one wide atom
+    atoms = gt.AtomElement(gt.AtomSpace(D, isotropic=iso), rng.uniform(-0.6, 0.6, (N, D)), r,
+                           rng.uniform(0.5, 2.0, N), device=dev)
+    data = torch.as_tensor(rng.normal(size=(nA,) + tuple(det)), dtype=torch.float32, device=dev)
+    return atoms, space, data
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(map(str, c[:4])))
+def test_orders_and_value(gt, cuda, case):
+    atoms, space, data = _problem(gt, case, cuda)
+    for mode in ("linear", "L2", "resid"):
+        f1, g1, H1 = gt.ops.derivs(atoms, space, data, mode, order=1)
+        f2, g2, _ = gt.ops.derivs(atoms, space, data, mode, order=2)
+        assert H1 is None and torch.equal(g1, g2)
+        assert (f1 is None and f2 is None) or torch.equal(f1, f2)
+    R = gt.ops.forward(atoms, space)
+    got = [gt.ops.forward_derivs(atoms, space, data, order=o) for o in (1, 2)]
+    got += [gt.ops.forward_derivs_noalloc(atoms, space, data, order=2)]
+    for resid, f, g, _ in got:
+        assert torch.equal(resid, R - data)
+        want = 0.5 * float((resid.double() ** 2).sum())
+        assert abs(float(f) - want) <= resid.numel() * EPS * want
+        assert torch.equal(f, got[0][1]) and torch.equal(g, got[0][2])
+    assert torch.equal(got[0][2], gt.ops.derivs(atoms, space, got[0][0], "resid", order=1)[1])
+    resid, f, g, _ = gt.ops.forward_derivs(atoms, space, data, want_f=False)
+    assert f is None and torch.equal(g, got[0][2])
