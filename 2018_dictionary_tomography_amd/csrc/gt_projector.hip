@@ -346,10 +346,13 @@ __global__ __launch_bounds__(256) void forward2_kernel(const PairRec *__restrict
 // ---------------------------------------------------------------------------
 // moments
 // ---------------------------------------------------------------------------
-// f = 1/2 sum of the forward's n partial sums of squares, in a fixed order: one
-// wave of the moments grid adds PART_CHUNK of them in place (16 loads in flight
-// per lane), one block the n / PART_CHUNK results.
-constexpr int PART_CHUNK = 1024;
+// f = 1/2 sum of the forward's n partial sums of squares, in a fixed order.  With
+// a moments grid to follow, one wave of it adds PART_CHUNK of them in place and
+// one block of the finish grid the n / PART_CHUNK results; without, one block of
+// half_sum_kernel adds up to HALF_SUM_MAX itself (46080 of 5000 atoms' 90 x
+// 256^2: 8 us) and more after a launch that folds the chunks.  16 loads in
+// flight per lane.
+constexpr int PART_CHUNK = 1024, HALF_SUM_MAX = 65536;
 __device__ inline void chunk_sum(double *__restrict__ part, size_t n, size_t chunk, int lane)
 {
     double *p = part + chunk * PART_CHUNK;
@@ -363,17 +366,33 @@ __device__ inline void chunk_sum(double *__restrict__ part, size_t n, size_t chu
     const double t = wave_sum_f64((s[0] + s[1]) + (s[2] + s[3]));
     if (lane == 0) p[0] = t;  // read by this wave only, before
 }
+template <int NTHR>
 __device__ inline void half_sum(const double *__restrict__ sums, size_t n, size_t stride, double *__restrict__ f,
-                                int nthr, double *red)
+                                double *red)
 {
     double s = 0.0;
-    for (size_t i = threadIdx.x; i < n; i += nthr) s += sums[i * stride];
+    size_t i = threadIdx.x;
+    for (; i + 15 * NTHR < n; i += 16 * NTHR) {
+        double v[16];
+#pragma unroll
+        for (int u = 0; u < 16; u++) v[u] = sums[(i + u * NTHR) * stride];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] += v[u + 8];
+        s += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+    }
+    if (i < n) {
+        double v[16];
+#pragma unroll
+        for (int u = 0; u < 16; u++) v[u] = sums[std::min(i + u * NTHR, n - 1) * stride];
+#pragma unroll
+        for (int u = 0; u < 16; u++) s += i + u * NTHR < n ? v[u] : 0.0;
+    }
     const double t = wave_sum_f64(s);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = t;
     __syncthreads();
     if (threadIdx.x == 0) {
         double v = 0.0;
-        for (int w = 0; w < nthr / 64; w++) v += red[w];
+        for (int w = 0; w < NTHR / 64; w++) v += red[w];
         f[0] = 0.5 * v;
     }
 }
@@ -381,11 +400,11 @@ __global__ __launch_bounds__(64) void chunk_sum_kernel(double *__restrict__ part
 {
     chunk_sum(part, n, blockIdx.x, threadIdx.x);
 }
-__global__ __launch_bounds__(512) void half_sum_kernel(const double *__restrict__ sums, size_t n, size_t stride,
-                                                       double *__restrict__ f)
+__global__ __launch_bounds__(1024) void half_sum_kernel(const double *__restrict__ sums, size_t n, size_t stride,
+                                                        double *__restrict__ f)
 {
-    __shared__ double red[8];
-    half_sum(sums, n, stride, f, 512, red);
+    __shared__ double red[16];
+    half_sum<1024>(sums, n, stride, f, red);
 }
 
 // Layout of one moment record (32 floats): [0, NM) sum w1 mono, [15, 15+NM)
@@ -483,7 +502,7 @@ __global__ __launch_bounds__(64) void finish_kernel(gt_atoms A, gt_geom G, const
     const int j = (int)blockIdx.x - (part ? 1 : 0), lane = threadIdx.x;
     const int N = A.n;
     if (j < 0) {
-        half_sum(part, (nparts + PART_CHUNK - 1) / PART_CHUNK, PART_CHUNK, ftotal, 64, &red[0][0]);
+        half_sum<64>(part, (nparts + PART_CHUNK - 1) / PART_CHUNK, PART_CHUNK, ftotal, &red[0][0]);
         return;
     }
     double grad[P], F = 0.0;
@@ -722,13 +741,18 @@ static int launch_residual(const gt_atoms *A, const gt_geom *G, const PairRec *r
     if (!f) return 0;
     if (tiles) {
         if (total) {
-            const size_t n = forward_parts(G), chunks = (n + PART_CHUNK - 1) / PART_CHUNK;
-            hipLaunchKernelGGL(chunk_sum_kernel, dim3((unsigned)chunks), dim3(64), 0, st, part, n);
-            hipLaunchKernelGGL(half_sum_kernel, dim3(1), dim3(512), 0, st, part, chunks, (size_t)PART_CHUNK, f);
+            size_t n = forward_parts(G), stride = 1;
+            if (n > HALF_SUM_MAX) {
+                const size_t chunks = (n + PART_CHUNK - 1) / PART_CHUNK;
+                hipLaunchKernelGGL(chunk_sum_kernel, dim3((unsigned)chunks), dim3(64), 0, st, part, n);
+                n = chunks;
+                stride = PART_CHUNK;
+            }
+            hipLaunchKernelGGL(half_sum_kernel, dim3(1), dim3(1024), 0, st, part, n, stride, f);
         }
     } else {
         hipLaunchKernelGGL(sumsq_kernel, dim3(G->nA), dim3(256), 0, st, R, (long)G->n0 * G->n1, sumC2);
-        hipLaunchKernelGGL(half_sum_kernel, dim3(1), dim3(512), 0, st, sumC2, (size_t)G->nA, (size_t)1, f);
+        hipLaunchKernelGGL(half_sum_kernel, dim3(1), dim3(1024), 0, st, sumC2, (size_t)G->nA, (size_t)1, f);
     }
     GT_HIP(hipGetLastError());
     return 0;
@@ -842,4 +866,31 @@ extern "C" int gt_forward_derivs(const gt_atoms *atoms, const gt_geom *geom, con
     }
     GT_CHECK_ARG(((uintptr_t)ws & 63) == 0, "gt_forward_derivs: workspace must be 64-byte aligned");
     return forward_derivs(atoms, geom, data, order, R, f, g, H, ws, true, (hipStream_t)stream);
+}
+
+extern "C" size_t gt_residual_workspace(const gt_atoms *atoms, const gt_geom *geom)
+{
+    if (!atoms || !geom) return 0;
+    return rec_bytes(atoms, geom) + std::max(part_bytes(geom), ang_bytes(geom));
+}
+
+extern "C" int gt_residual(const gt_atoms *atoms, const gt_geom *geom, const float *data, float *R, double *f, void *ws,
+                           size_t ws_bytes, void *stream)
+{
+    int rc;
+    if ((rc = check_atoms(atoms)) || (rc = check_geom(geom, atoms->dim))) return rc;
+    GT_CHECK_ARG(data != nullptr, "gt_residual: data is NULL");
+    GT_CHECK_ARG(R != nullptr, "gt_residual: R is NULL");
+    GT_CHECK_ARG(R != data, "gt_residual: R must not alias data");
+    const size_t need = gt_residual_workspace(atoms, geom);
+    if (need > ws_bytes || (need > 0 && ws == nullptr)) {
+        set_error("gt_residual: workspace of %zu bytes given, %zu needed", ws_bytes, need);
+        return GT_EWORKSPACE;
+    }
+    GT_CHECK_ARG(((uintptr_t)ws & 63) == 0, "gt_residual: workspace must be 64-byte aligned");
+    hipStream_t st = (hipStream_t)stream;
+    PairRec *recs = (PairRec *)ws;
+    double *sums = (double *)((char *)ws + rec_bytes(atoms, geom));
+    if ((rc = launch_setup(atoms, geom, recs, st))) return rc;
+    return launch_residual(atoms, geom, recs, data, R, f, sums, sums, true, st);
 }

@@ -182,6 +182,25 @@ def forward_derivs(atoms, space, data, order=2, out=None, want_f=True):
     return out, f, g, H
 
 
+def residual(atoms, space, data):
+    """(resid, f): resid = forward(atoms) - data and f = 1/2||resid||^2 (0-d FP64).
+    data: contiguous float32 tensor on the atoms' device, of the space's shape."""
+    lib = load()
+    dev = atoms.I.device
+    geom = device_geometry(space, dev)
+    a = atoms_struct(atoms)
+    if tuple(data.shape) != tuple(geom.shape) or data.dtype != torch.float32 or data.device != dev \
+            or not data.is_contiguous():
+        raise ValueError(f"data must be a contiguous float32 tensor of shape {geom.shape} on {dev}")
+    resid = torch.empty(geom.shape, dtype=torch.float32, device=dev)
+    f = torch.empty((), dtype=torch.float64, device=dev)
+    need = lib.gt_residual_workspace(ctypes.byref(a), ctypes.byref(geom.struct))
+    ws = _ws.get(need, dev)
+    check(lib.gt_residual(ctypes.byref(a), ctypes.byref(geom.struct), _ptr(data), _ptr(resid), _ptr(f), _ptr(ws),
+                          ws.numel(), stream_handle(dev)), "gt_residual")
+    return resid, f
+
+
 def forward_derivs_noalloc(atoms, space, data, order=2, out=None, want_f=True):
     """forward_derivs through gt_forward_derivs_noalloc: the library takes
     the workspace from its per-GPU scratch array (at most

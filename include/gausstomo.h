@@ -135,6 +135,13 @@ int gt_derivs(const gt_atoms *atoms, const gt_geom *geom, const float *C, int mo
 int gt_forward_derivs(const gt_atoms *atoms, const gt_geom *geom, const float *data, int order, float *R,
                       double *f, double *g, double *H, void *ws, size_t ws_bytes, void *stream);
 
+/* The projection half of gt_forward_derivs: R = RadProj(atoms) - data and, if f
+ * is not NULL, f[0] = 1/2 ||R||^2 in FP64 (transport_loss.l2_squared_loss,
+ * transport_loss.py:567-585).  R and data must not overlap. */
+size_t gt_residual_workspace(const gt_atoms *atoms, const gt_geom *geom);
+int gt_residual(const gt_atoms *atoms, const gt_geom *geom, const float *data, float *R, double *f, void *ws,
+                size_t ws_bytes, void *stream);
+
 /* No counterpart in the reference: gt_forward_derivs without a workspace, for
  * callers that cannot allocate device memory (code under HIP graph capture,
  * serving loops, harnesses that forbid hipMalloc).  The workspace is a
