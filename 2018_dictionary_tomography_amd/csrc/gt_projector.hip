@@ -103,12 +103,23 @@ __device__ inline int stage_chunk(const PairRec *__restrict__ ra, int base, int 
 // Block tile TILE_ROWS x TILE_COLS = 8 x 64 pixels, F3_WAVES = 4 waves; wave
 // w owns the 8 x 16 rectangle rows 8 (w / 4) .. +7, columns 16 (w % 4) ..
 // +15, and lane l column l % 16 of it, rows l / 16 and l / 16 + 4 (2 pixels
-// per lane).  Staging keeps the records that touch the tile in LDS and, for
-// every wave, the list of those that touch its rectangle (both in atom
-// order, so each pixel's summation order is fixed): a wave then walks only
-// records that reach its pixels.  (8 x 64 tiles of 4 waves measured 138 us
+// per lane).  Staging keeps the records that reach a rectangle in LDS and, for
+// every wave, the list of those that reach its own (in atom order, so each
+// pixel's summation order is fixed).  (8 x 64 tiles of 4 waves measured 138 us
 // against 155 us for 16 x 64 tiles of 8 waves: twice the blocks, so the
 // centre-first dispatch balances finer.)
+//
+// Vector issue and LDS bandwidth bound it together (80% of the LDS cycles and
+// one vector instruction per cycle and CU).  A wave takes four records at a
+// time: lane (u, k) works out what record u's exponent takes from column k and
+// row k % 8 of the rectangle, once for the 8 rows and 16 columns that share it,
+// and the pixels read the two from LDS: 15 vector instructions and 12 LDS
+// cycles per record and wave against 23 and 17 with each lane working on the
+// records (three 16-byte broadcast reads each) by itself.  The record itself
+// comes as one word per lane and is passed around its row of 16 lanes.  5000
+// atoms, 90 x 256^2: 2.02 -> 1.76 ms; 1000, 61 x 128^2: 98.8 -> 88.8 us; 300,
+// 45 x 96 x 83: 26.0 -> 22.4 us.  (Records through scalar loads: 102 us of the
+// second, their waits are shared with LDS.)
 constexpr int F3_WAVES = 4, F3_CHUNK = F3_WAVES * 64;
 static_assert(TILE_ROWS == 8 * ((F3_WAVES + 3) / 4) && TILE_COLS == 16 * (F3_WAVES < 4 ? F3_WAVES : 4),
               "the tile is the union of the waves' 8 x 16 rectangles");
@@ -122,109 +133,64 @@ constexpr int F3_RX = 2 * ((F3_WAVES + 3) / 4), F3_CY = 2 * (F3_WAVES < 4 ? F3_W
 // angles of one tile together (block b: angle b % nA, tile rank b / nA), so
 // the heavy tiles start first and the light ones fill the tail.
 
-__device__ inline int stage_rects(const PairRec *__restrict__ ra, int base, int N, int row0, int col0, int thi0,
-                                  int thi1, PairRec *list, unsigned short (*wl)[F3_CHUNK], int (*cnt)[F3_WAVES],
-                                  int *wlen, bool exact, const float (&rx)[F3_RX], const float (&cy)[F3_CY])
+__device__ inline void stage_rects(const PairRec *__restrict__ ra, int base, int N, int row0, int col0, PairRec *list,
+                                   unsigned short (*wl)[F3_CHUNK], int (*cnt)[F3_WAVES], int *wlen, bool exact,
+                                   const float (&rx)[F3_RX], const float (&cy)[F3_CY])
 {
-    const int lane = threadIdx.x & 63, hw = threadIdx.x >> 6;
     const int j = base + (int)threadIdx.x;
-    int4 v0 = make_int4(0, 0, 0, 0), v1 = v0, v2 = v0, v3 = v0;
-    bool hit = false;
     unsigned mask = 0;
     if (j < N) {
         const int4 *src = reinterpret_cast<const int4 *>(ra + j);
-        v0 = src[0];
-        v1 = src[1];
-        v2 = src[2];
-        v3 = src[3];
+        const int4 v0 = src[0], v1 = src[1], v2 = src[2], v3 = src[3];
         // v3 = (lo[0], lo[1], hi[0], hi[1])
-        hit = v3.x <= thi0 && v3.z >= row0 && v3.y <= thi1 && v3.w >= col0;
-        if (hit) {
-            // f0 = (alpha, c_hi0, c_hi1, c_lo0), f1 = (c_lo1, q0, q1, q2), f2 = (q3, q4, q5, pad)
-            const float4 f0 = *reinterpret_cast<const float4 *>(&v0), f1 = *reinterpret_cast<const float4 *>(&v1);
-            const float4 f2 = *reinterpret_cast<const float4 *>(&v2);
+        // f0 = (alpha, c_hi0, c_hi1, c_lo0), f1 = (c_lo1, q0, q1, q2), f2 = (q3, q4, q5, pad)
+        const float4 f0 = *reinterpret_cast<const float4 *>(&v0), f1 = *reinterpret_cast<const float4 *>(&v1);
+        const float4 f2 = *reinterpret_cast<const float4 *>(&v2);
 #pragma unroll
-            for (int w = 0; w < F3_WAVES; w++) {
-                const int r = row0 + 8 * (w >> 2), c = col0 + 16 * (w & 3);
-                if (v3.x <= r + 7 && v3.z >= r && v3.y <= c + 15 && v3.w >= c &&
-                    (!exact || support_meets_rect(f1, f2, (rx[2 * (w >> 2)] - f0.y) - f0.w,
-                                               (rx[2 * (w >> 2) + 1] - f0.y) - f0.w, (cy[2 * (w & 3)] - f0.z) - f1.x,
-                                               (cy[2 * (w & 3) + 1] - f0.z) - f1.x)))
-                    mask |= 1u << w;
-            }
+        for (int w = 0; w < F3_WAVES; w++) {
+            const int r = row0 + 8 * (w >> 2), c = col0 + 16 * (w & 3);
+            if (v3.x <= r + 7 && v3.z >= r && v3.y <= c + 15 && v3.w >= c &&
+                (!exact || support_meets_rect(f1, f2, (rx[2 * (w >> 2)] - f0.y) - f0.w,
+                                           (rx[2 * (w >> 2) + 1] - f0.y) - f0.w, (cy[2 * (w & 3)] - f0.z) - f1.x,
+                                           (cy[2 * (w & 3) + 1] - f0.z) - f1.x)))
+                mask |= 1u << w;
+        }
+        if (mask) {
+            float4 *dst = reinterpret_cast<float4 *>(list + threadIdx.x);
+            dst[0] = f0;
+            dst[1] = f1;
+            dst[2] = f2;
         }
     }
-    // cnt[k][hw]: hits of this hardware wave, k = 0 the tile list, k = 1 + w wave w's list
-    const unsigned long long below = (1ull << lane) - 1ull;
-    const unsigned long long mt = __ballot(hit);
-    if (lane == 0) cnt[0][hw] = __popcll(mt);
-    unsigned long long mw[F3_WAVES];
-#pragma unroll
-    for (int w = 0; w < F3_WAVES; w++) {
-        mw[w] = __ballot((mask >> w) & 1u);
-        if (lane == 0) cnt[1 + w][hw] = __popcll(mw[w]);
-    }
-    __syncthreads();
-    int off = 0, total = 0;
-#pragma unroll
-    for (int h = 0; h < F3_WAVES; h++) {
-        if (h < hw) off += cnt[0][h];
-        total += cnt[0][h];
-    }
-    const int pos = off + __popcll(mt & below);
-    if (hit) {
-        int4 *dst = reinterpret_cast<int4 *>(list + pos);
-        dst[0] = v0;
-        dst[1] = v1;
-        dst[2] = v2;
-        dst[3] = v3;
-    }
-#pragma unroll
-    for (int w = 0; w < F3_WAVES; w++) {
-        int o = 0, t = 0;
-#pragma unroll
-        for (int h = 0; h < F3_WAVES; h++) {
-            if (h < hw) o += cnt[1 + w][h];
-            t += cnt[1 + w][h];
-        }
-        if ((mask >> w) & 1u) wl[w][o + __popcll(mw[w] & below)] = (unsigned short)pos;
-        if (threadIdx.x == 0) wlen[w] = t;
-    }
-    __syncthreads();
-    return total;
+    wave_lists<F3_WAVES, F3_WAVES>(mask, wl, cnt, wlen);
 }
 
-// One record's values at a lane's two pixels.  The record arrives as its
-// first 48 bytes (alpha, c_hi, c_lo, q): f0 = (alpha, c_hi0, c_hi1, c_lo0),
-// f1 = (c_lo1, q0, q1, q2), f2 = (q3, q4, q5, pad).  No cut-off test: every
-// record in a wave's list reaches its rectangle, and the values at pixels of
-// the rectangle outside the support are below e^-30 of the record's peak.
-__device__ inline void f3_values(const float4 &f0, const float4 &f1, const float4 &f2, float pc, float prA,
-                                 float prB, float &vA, float &vB)
+// the value of lane K of each row of 16 lanes, in the whole row
+template <int K> __device__ inline float row_bcast(float v)
 {
-    const float dp1 = (pc - f0.z) - f1.x;
-    const float rowlin = fmaf(f1.z, dp1, f2.x);
-    const float col = fmaf(fmaf(f1.w, dp1, f2.y), dp1, f2.z);
-    const float dA = (prA - f0.y) - f0.w;
-    const float dB = (prB - f0.y) - f0.w;
-    const float qA = fmaf(fmaf(f1.y, dA, rowlin), dA, col);
-    const float qB = fmaf(fmaf(f1.y, dB, rowlin), dB, col);
-    const float eA = __builtin_amdgcn_exp2f(qA), eB = __builtin_amdgcn_exp2f(qB);
-    vA = f0.x * eA;
-    vB = f0.x * eB;
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + K, 0xf, 0xf, true));
 }
+// A group of four records as the pixels read it: per column (the terms linear
+// and constant in the row, q0, alpha), per row the offset from the centre.  No
+// cut-off test: every record in a wave's list reaches its rectangle, and the
+// values at pixels of the rectangle outside the support are below e^-30 of the
+// record's peak.
+struct F3Tab {
+    float4 c[4][16];
+    float r[4][8];  // rows 0, 4, 1, 5, ...: a lane's two side by side
+};
 
 // (at most 64 VGPRs: eight waves per SIMD)
-__global__ __launch_bounds__(F3_WAVES * 64) __attribute__((amdgpu_waves_per_eu(8))) void forward3_kernel(const PairRec *__restrict__ recs, int N, int nA,
-                                                                 int n0, int n1, const float *__restrict__ p0,
-                                                                 const float *__restrict__ p1, float *__restrict__ R,
-                                                                 const float *__restrict__ sub, int e0, int e1,
-                                                                 int sorted, double *__restrict__ part)
+__global__ __launch_bounds__(F3_WAVES * 64) __attribute__((amdgpu_waves_per_eu(8))) void forward3_kernel(
+    const PairRec *__restrict__ recs, int N, int nA, int n0, int n1, const float *__restrict__ p0,
+    const float *__restrict__ p1, float *__restrict__ R, const float *__restrict__ sub, int e0, int e1, int sorted,
+    double *__restrict__ part)
 {
-    __shared__ PairRec list[F3_CHUNK];
-    __shared__ alignas(16) unsigned short wl[F3_WAVES][F3_CHUNK];  // 8-byte reads of 4 indices
-    __shared__ int cnt[F3_WAVES + 1][F3_WAVES];
+    __shared__ PairRec list[F3_CHUNK];  // (their first 48 bytes)
+    __shared__ unsigned short wl[F3_WAVES][F3_CHUNK];
+    __shared__ int cnt[F3_WAVES][F3_WAVES];
     __shared__ int wlen[F3_WAVES];
+    __shared__ F3Tab tab[F3_WAVES];
     const int tilesR = (n0 + TILE_ROWS - 1) / TILE_ROWS, tilesC = (n1 + TILE_COLS - 1) / TILE_COLS;
     const int a = (int)(blockIdx.x % (unsigned)nA);
     const int e[3] = {e0, e1, 0};
@@ -236,9 +202,9 @@ __global__ __launch_bounds__(F3_WAVES * 64) __attribute__((amdgpu_waves_per_eu(8
     const int wr0 = row0 + 8 * (wave >> 2), wc0 = col0 + 16 * (wave & 3);
     const int i1 = wc0 + (lane & 15);
     const int rA = wr0 + (lane >> 4), rB = rA + 4;
-    const int thi0 = min(row0 + TILE_ROWS - 1, n0 - 1), thi1 = min(col0 + TILE_COLS - 1, n1 - 1);
     const float pc = p1[min(i1, n1 - 1)];
-    const float prA = p0[min(rA, n0 - 1)], prB = p0[min(rB, n0 - 1)];
+    const float pr8 = p0[min(wr0 + (lane & 7), n0 - 1)];
+    const int u16 = lane >> 4;
     double sA = 0.0, sB = 0.0;
     // detector coordinates bounding each wave rectangle (first and last
     // row / column), for the exact cull of an ascending detector
@@ -255,40 +221,60 @@ __global__ __launch_bounds__(F3_WAVES * 64) __attribute__((amdgpu_waves_per_eu(8
     }
     const PairRec *ra = recs + (size_t)a * N;
     for (int base = 0; base < N; base += F3_CHUNK) {
-        stage_rects(ra, base, N, row0, col0, thi0, thi1, list, wl, cnt, wlen, sorted != 0, rx, cy);
+        stage_rects(ra, base, N, row0, col0, list, wl, cnt, wlen, sorted != 0, rx, cy);
         const int len = wlen[wave];
         const unsigned short *wlw = wl[wave];
-        int e = 0;
-        // 4 records per step: their list indices (one 8-byte read) and records
-        // (three 16-byte reads each) are all read before any is used; the
-        // pixel sums still take the records in list order
-        for (; e + 4 <= len; e += 4) {
-            const uint2 iv = *reinterpret_cast<const uint2 *>(wlw + e);
-            const int idx[4] = {(int)(iv.x & 0xffffu), (int)(iv.x >> 16), (int)(iv.y & 0xffffu), (int)(iv.y >> 16)};
-            float4 f0[4], f1[4], f2[4];
+        if (len > 0) {
+            // lane (u, k): record u of the group at column k and row k % 8
+            F3Tab &T = tab[wave];
+            float vA[4], vB[4];
+            const float *lf = reinterpret_cast<const float *>(list) + (lane & 15);
+            float w = lf[16 * wlw[min(u16, len - 1)]];
+            int nidx = wlw[min(4 + u16, len - 1)];
+            const auto group = [&](int e) {
+                // words of a record: 0 alpha, 1-2 c_hi, 3-4 c_lo, 5-10 q
+                const float dp1 = (pc - row_bcast<2>(w)) - row_bcast<4>(w);
+                T.c[u16][lane & 15] =
+                    make_float4(fmaf(row_bcast<6>(w), dp1, row_bcast<8>(w)),
+                                fmaf(fmaf(row_bcast<7>(w), dp1, row_bcast<9>(w)), dp1, row_bcast<10>(w)),
+                                row_bcast<5>(w), row_bcast<0>(w));
+                T.r[u16][2 * (lane & 3) + ((lane >> 2) & 1)] = (pr8 - row_bcast<1>(w)) - row_bcast<3>(w);
+                wave_sync();
+                float4 c[4];
+                float2 d[4];
 #pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const float4 *rp = reinterpret_cast<const float4 *>(list + idx[u]);
-                f0[u] = rp[0];
-                f1[u] = rp[1];
-                f2[u] = rp[2];
-            }
+                for (int u = 0; u < 4; u++) {
+                    c[u] = T.c[u][lane & 15];
+                    d[u] = *reinterpret_cast<const float2 *>(&T.r[u][2 * u16]);
+                }
+                w = lf[16 * nidx];
+                nidx = wlw[min(e + 8 + u16, len - 1)];
+                wave_sync();
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    vA[u] = c[u].w * __builtin_amdgcn_exp2f(fmaf(fmaf(c[u].z, d[u].x, c[u].x), d[u].x, c[u].y));
+                    vB[u] = c[u].w * __builtin_amdgcn_exp2f(fmaf(fmaf(c[u].z, d[u].y, c[u].x), d[u].y, c[u].y));
+                }
+            };
+            int e = 0;
             // the four values of a pixel are summed in FP32 in list order and
             // that sum is added to the pixel's FP64 total: an error of at most
             // 3u times the sum of the four magnitudes, for one conversion and
             // one FP64 add per four records
-            float vA[4], vB[4];
+            for (; e + 4 <= len; e += 4) {
+                group(e);
+                sA += (double)(((vA[0] + vA[1]) + vA[2]) + vA[3]);
+                sB += (double)(((vB[0] + vB[1]) + vB[2]) + vB[3]);
+            }
+            if (e < len) {
+                group(e);
 #pragma unroll
-            for (int u = 0; u < 4; u++) f3_values(f0[u], f1[u], f2[u], pc, prA, prB, vA[u], vB[u]);
-            sA += (double)(((vA[0] + vA[1]) + vA[2]) + vA[3]);
-            sB += (double)(((vB[0] + vB[1]) + vB[2]) + vB[3]);
-        }
-        for (; e < len; e++) {
-            const float4 *rp = reinterpret_cast<const float4 *>(list + wlw[e]);
-            float vA, vB;
-            f3_values(rp[0], rp[1], rp[2], pc, prA, prB, vA, vB);
-            sA += (double)vA;
-            sB += (double)vB;
+                for (int u = 0; u < 3; u++)
+                    if (e + u < len) {
+                        sA += (double)vA[u];
+                        sB += (double)vB[u];
+                    }
+            }
         }
         __syncthreads();
     }
