@@ -36,7 +36,12 @@
 // same decisions from the same numbers and the result does not depend on G.
 // The members meet at two device-wide barriers per atom update (after the
 // per-angle contractions and after the per-angle energy changes); a barrier
-// wait is bounded in time.  The solve and the accept logic run redundantly in
+// wait is bounded in time.  An update is one latency chain: 300 atoms, 61 x
+// 96^2, 66 us at G = 4 (4 setup, 14 moments and contraction, 14 meeting and
+// sums over angles, 7 solve, 3 + 15 the proposal's setup and energy, 2 accept,
+// 7 commit); 69 us with a barrier word that the last arrival resets and
+// releases, per-angle records read a line per lane, and the atom, its step
+// size and its place in the order read one after the other.  The solve and the accept logic run redundantly in
 // every member; member 0 writes the progress fields back at the end.
 //
 // Pixel phases give one (atom, angle) pair to each wave.  A wave contracts
@@ -55,7 +60,7 @@ constexpr int FIT_WAVES = FIT_THREADS / 64;
 constexpr int NAMAX = GT_FIT_MAX_ANGLES;
 static_assert(NAMAX % 64 == 0, "per-angle sums take whole waves of angles");
 constexpr int DETMAX = GT_FIT_MAX_DETECTOR;
-constexpr int NVS = 65;                          // stride of a per-angle gradient/Hessian record
+constexpr int NVS = 65;                          // entries of a per-angle gradient/Hessian record
 constexpr int FIT_UNR = 8;                       // detector rows in flight per lane in the pixel passes
 constexpr int FIT_TROWS = 192;                   // rows of a wave's row table (moments, energy and commit passes)
 constexpr int FIT_BOXW = 64;                     // columns per chunk of the moments walk
@@ -63,8 +68,9 @@ constexpr double FIT_EPS = 1e-4;                 // NewtonGaussian.py:21
 constexpr double GD_EPS = 1e-8;                  // GD_lib.py:96
 constexpr long long FIT_WAIT_TICKS = 200000000;  // barrier wait limit: 2 s of the 100 MHz clock
 
-// Slot scratch layout (bytes): per-angle records double[nA][NVS] | per-angle
-// energy changes double[nA] | barrier words.
+// Slot scratch layout (bytes): per-angle gradient/Hessian entries
+// double[NVS][nA] (an entry's angles side by side: the sums over angles read
+// whole lines) | per-angle energy changes double[nA] | barrier words.
 __host__ __device__ inline size_t fit_off_dE(int nA) { return align_up((size_t)nA * NVS * sizeof(double)); }
 __host__ __device__ inline size_t fit_off_bar(int nA) { return fit_off_dE(nA) + align_up((size_t)nA * sizeof(double)); }
 __host__ __device__ inline size_t fit_scratch_size(int nA) { return fit_off_bar(nA) + ALIGN; }
@@ -99,8 +105,10 @@ template <int D> struct FitLDS {
     double rv_old, rv_new;    // regulariser terms of the current atom and of the proposal
     double dxnorm, hj;
     FitCtl c;
-    unsigned gen;
+    unsigned arrivals;  // barrier count the next meeting waits for, less G
     int accept, j, stop, abort_, skip, moved;
+    long lin;  // place of the current atom in the order (-1: none yet), its and the next one's number
+    int jcur, jnext;
     int next[3];  // next own-angle number of the moments, energy and commit passes
 };
 
@@ -511,31 +519,37 @@ __device__ inline void wait_all_memory() { __builtin_amdgcn_s_waitcnt(0); }
 
 // Device-wide barrier of the G workgroups of one slot, called by thread 0 of
 // each after every thread of its workgroup has completed its xput stores.
-// bar[0] counts arrivals, bar[1] is the generation, bar[2] the abort flag.
-// The wait is bounded: after FIT_WAIT_TICKS the slot is aborted.  Returns
-// false if aborted.
-__device__ inline bool group_barrier(unsigned *bar, int G, unsigned &gen)
+// bar[0] counts arrivals, bar[2] is the abort flag.  The count runs on through
+// a launch (the k-th barrier is passed at k G arrivals) and the waiters read it
+// directly, so a barrier is one arrival and the reads that see the last one:
+// nothing is reset and no word of release is written in between.  The wait is
+// bounded: after FIT_WAIT_TICKS the slot is aborted.  Returns false if aborted.
+__device__ inline bool group_barrier(unsigned *bar, int G, unsigned &target)
 {
-    if (xgetu(bar + 2) != 0u) return false;
-    const unsigned target = gen + 1u;
-    const unsigned old = __hip_atomic_fetch_add(bar, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (old == (unsigned)G - 1u) {
-        xputu(bar, 0u);
-        wait_all_memory();  // the reset lands before anyone can pass and arrive again
-        xputu(bar + 1, target);
-    } else {
-        const long long t0 = wall_clock64();
-        while (xgetu(bar + 1) != target) {
-            if (xgetu(bar + 2) != 0u) return false;
-            if (wall_clock64() - t0 > FIT_WAIT_TICKS) {
-                xputu(bar + 2, 1u);
-                return false;
-            }
-            __builtin_amdgcn_s_sleep(2);
+    target += (unsigned)G;
+    __hip_atomic_fetch_add(bar, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const long long t0 = wall_clock64();
+    for (;;) {
+        const unsigned n = xgetu(bar), aborted = xgetu(bar + 2);
+        if ((int)(n - target) >= 0) return true;
+        if (aborted != 0u) return false;
+        if (wall_clock64() - t0 > FIT_WAIT_TICKS) {
+            xputu(bar + 2, 1u);
+            return false;
         }
+        __builtin_amdgcn_s_sleep(1);
     }
-    gen = target;
-    return true;
+}
+
+// The end of a launch: the last member to leave (none waits any more) clears
+// the count for the next launch, whose group may have another size.
+__device__ inline void group_leave(unsigned *bar, int G)
+{
+    wait_all_memory();
+    if (__hip_atomic_fetch_add(bar + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)G - 1u) {
+        xputu(bar, 0u);
+        xputu(bar + 1, 0u);
+    }
 }
 
 // Advance the loop position after an update (or after a skipped block):
@@ -610,7 +624,14 @@ __global__ __launch_bounds__(FIT_THREADS) void fit_kernel(gt_fit_slot *__restric
     const gt_geom Gm = slot_geom(S, D);
     const int N = S.N, nA = S.nA, n1 = S.n1;
     const size_t slab = (size_t)S.n0 * S.n1;
-    const float *det[2] = {S.p0, S.p1};
+    // (local copies: the slot's own fields would be read again after every store)
+    float *const aI = S.I, *const ax = S.x, *const ar = S.r;
+    double *const ah = S.h;
+    const int *const perm = S.perm;
+    const long nperm = (long)S.max_outer * N;
+    gmem<float> *const resid = (gmem<float> *)S.resid;
+    const int rk = S.reg_kind;
+    const float *det[2] = {L.p0, L.p1};  // the detector coordinates in LDS
     const int nd[2] = {S.n0, S.n1};
     char *scr = (char *)S.scratch;
     double *prec = (double *)scr;
@@ -644,7 +665,8 @@ __global__ __launch_bounds__(FIT_THREADS) void fit_kernel(gt_fit_slot *__restric
         c.ninf = S.ninf;
         c.F = S.F;
         c.Rsum = S.Rsum;
-        L.gen = (G > 1) ? xgetu(bar + 1) : 0u;
+        L.arrivals = 0u;
+        L.lin = -1;
         L.abort_ = 0;
     }
     __syncthreads();
@@ -663,7 +685,7 @@ __global__ __launch_bounds__(FIT_THREADS) void fit_kernel(gt_fit_slot *__restric
     wait_all_memory();                                                         \
     __syncthreads();                                                           \
     if (G > 1) {                                                               \
-        if (tid == 0 && !group_barrier(bar, G, L.gen)) L.abort_ = 1;           \
+        if (tid == 0 && !group_barrier(bar, G, L.arrivals)) L.abort_ = 1;           \
         __syncthreads();                                                       \
         if (L.abort_) break;                                                   \
     }
@@ -671,23 +693,38 @@ __global__ __launch_bounds__(FIT_THREADS) void fit_kernel(gt_fit_slot *__restric
     const int my_budget = quota > 0 ? min(budget, quota) : (S.quota > 0 ? min(budget, S.quota) : budget);
     for (int step = 0; step < my_budget; step++) {
         // ---- choose the atom, load its parameters -----------------------
-        if (tid == 0) {
-            FitCtl &c = L.c;
-            L.skip = 0;
-            L.stop = c.done != 0 || c.it >= S.max_outer || c.pos >= N;
-            if (!L.stop) {
-                const int j = S.perm[(size_t)c.it * N + c.pos];
-                if (j < 0 || j >= N) {
-                    L.stop = 1;
-                    c.done = 2;
+        if (wave == 0) {
+            const FitCtl &c = L.c;
+            bool stop = c.done != 0 || c.it >= S.max_outer || c.pos >= N;
+            int j = 0, jn = -1;
+            if (!stop) {
+                // the next entry of the order is read along with this one's atom
+                const long lin = (long)c.it * N + c.pos;
+                j = lin == L.lin ? L.jcur : (L.lin >= 0 && lin == L.lin + 1 ? L.jnext : perm[lin]);
+                const bool bad = j < 0 || j >= N;
+                if (!bad) {
+                    const float *src = lane == 0 ? aI + j : (lane <= D ? ax + (size_t)j * D + lane - 1
+                                                                       : ar + (size_t)j * NRs + lane - 1 - D);
+                    if (lane < 1 + D + NRs) L.th_old[lane] = *src;
+                    // h: the other members write the values of the updates
+                    // before this one that this member has written itself
+                    if (lane == 0) L.hj = ah[(size_t)c.blk * N + j];
                 }
+                if (lin + 1 < nperm) jn = perm[lin + 1];
+                wave_sync();
+                if (lane == 0) {
+                    L.lin = lin;
+                    L.jcur = j;
+                    L.jnext = jn;
+                    if (bad) L.c.done = 2;
+                }
+                stop = bad;
+            }
+            if (lane == 0) {
+                L.skip = 0;
+                L.stop = stop;
                 L.j = j;
                 L.next[0] = L.next[1] = L.next[2] = 0;
-                if (!L.stop) {
-                    L.th_old[0] = S.I[j];
-                    for (int i = 0; i < D; i++) L.th_old[1 + i] = S.x[(size_t)j * D + i];
-                    for (int k = 0; k < NRs; k++) L.th_old[1 + D + k] = S.r[(size_t)j * NRs + k];
-                }
             }
         }
         __syncthreads();
@@ -712,7 +749,7 @@ __global__ __launch_bounds__(FIT_THREADS) void fit_kernel(gt_fit_slot *__restric
                 float acc[MOMW];
 #pragma unroll
                 for (int v = 0; v < MOMW; v++) acc[v] = 0.0f;
-                const gmem<float> *Ra = (gmem<float> *)S.resid + (size_t)a * slab;
+                const gmem<float> *Ra = resid + (size_t)a * slab;
                 if (K == 2)
                     pair_moments_box<GT_MODE_RESID, FIT_UNR, FIT_TROWS, FIT_BOXW>(rec, L.p0, L.p1, Ra, n1, lane,
                                                                                   acc, L.tab[wave]);
@@ -756,7 +793,7 @@ __global__ __launch_bounds__(FIT_THREADS) void fit_kernel(gt_fit_slot *__restric
                     const int e = q == NV ? 0 : q;
                     int i = e, l = e;
                     if (e >= P) upper_ij(e - P, P, i, l);
-                    xput(prec + (size_t)a * NVS + e, (e < P) ? fin_grad<D>(W.F, e) : fin_hess<D>(W.F, i, l));
+                    xput(prec + (size_t)e * nA + a, (e < P) ? fin_grad<D>(W.F, e) : fin_hess<D>(W.F, i, l));
                 }
                 wave_sync();  // W is reused by the wave's next angle
             }
@@ -776,7 +813,7 @@ __global__ __launch_bounds__(FIT_THREADS) void fit_kernel(gt_fit_slot *__restric
                 if (e < NV) {
 #pragma unroll
                     for (int u = 0; u < NAMAX / 64; u++)
-                        if (lane + 64 * u < nA) t += xget(prec + (size_t)(lane + 64 * u) * NVS + e);
+                        if (lane + 64 * u < nA) t += xget(prec + (size_t)e * nA + lane + 64 * u);
                 }
                 v[q] = t;
             }
@@ -799,14 +836,12 @@ __global__ __launch_bounds__(FIT_THREADS) void fit_kernel(gt_fit_slot *__restric
         __syncthreads();
         GT_FIT_TICK(2);
         // ---- phase D: damped Newton system, solve, projections ------------
-        // h is read here, between the two barriers of this update: other
-        // members write its new value only after the second one
-        const int rk = S.reg_kind;
-        if (tid == 0) {
-            L.hj = S.h[(size_t)L.c.blk * N + j];
-            L.rv_old = rk != GT_REG_NULL ? reg_eval<D>(rk, S.reg_p, iso, L.th_old, L.rg, L.rH) : 0.0;
+        if (rk != GT_REG_NULL) {
+            if (tid == 0) L.rv_old = reg_eval<D>(rk, S.reg_p, iso, L.th_old, L.rg, L.rH);
+            __syncthreads();
+        } else if (tid == 0) {
+            L.rv_old = 0.0;
         }
-        __syncthreads();
         // (H + reg'' + I/h) dx = -(g + reg') over the solve's parameters
         // (NewtonGaussian.py:61-74 and :147-152)
         if (tid < PI * PI) {
@@ -961,7 +996,7 @@ __global__ __launch_bounds__(FIT_THREADS) void fit_kernel(gt_fit_slot *__restric
         // ---- phase F: per-angle FP64 energy changes -----------------------
         for (int k = next_angle(&L.next[1], lane); k < nOwn; k = next_angle(&L.next[1], lane)) {
             const int a = member + G * k;
-            gmem<float> *Ra = (gmem<float> *)S.resid + (size_t)a * slab;
+            gmem<float> *Ra = resid + (size_t)a * slab;
             float2 *dt = reinterpret_cast<float2 *>(L.tab[wave]);
             double acc = stage ? pair_delta4<K, 2>(L.rec_old[k], L.rec_new[k], L.p0, L.p1, Ra,
                                                    stage + (size_t)a * slab, n1, lane, dt)
@@ -1021,12 +1056,12 @@ __global__ __launch_bounds__(FIT_THREADS) void fit_kernel(gt_fit_slot *__restric
                     h *= S.block == 2 ? 1.1 : (S.block ? 1.3 : 2.0);
                     // every member writes the same values: its own later reads
                     // of atom j then never depend on another member's timing
-                    S.I[j] = (float)L.th_new[0];
-                    for (int i = 0; i < D; i++) S.x[(size_t)j * D + i] = (float)L.th_new[1 + i];
-                    for (int k = 0; k < NRs; k++) S.r[(size_t)j * NRs + k] = (float)L.th_new[1 + D + k];
+                    aI[j] = (float)L.th_new[0];
+                    for (int i = 0; i < D; i++) ax[(size_t)j * D + i] = (float)L.th_new[1 + i];
+                    for (int k = 0; k < NRs; k++) ar[(size_t)j * NRs + k] = (float)L.th_new[1 + D + k];
                     c.accepted++;
                 }
-                S.h[(size_t)c.blk * N + j] = S.block == 2 ? fmax(h, GD_EPS) : fmin(fmax(h, FIT_EPS), 1.0 / FIT_EPS);
+                ah[(size_t)c.blk * N + j] = S.block == 2 ? fmax(h, GD_EPS) : fmin(fmax(h, FIT_EPS), 1.0 / FIT_EPS);
                 c.jj++;
                 if (S.Ehist && member == 0) S.Ehist[c.jj] = c.E;
                 c.updates++;
@@ -1041,7 +1076,7 @@ __global__ __launch_bounds__(FIT_THREADS) void fit_kernel(gt_fit_slot *__restric
         if (stage ? !L.accept : L.accept) {
             for (int k = next_angle(&L.next[2], lane); k < nOwn; k = next_angle(&L.next[2], lane)) {
                 const int a = member + G * k;
-                gmem<float> *Ra = (gmem<float> *)S.resid + (size_t)a * slab;
+                gmem<float> *Ra = resid + (size_t)a * slab;
                 if (stage)
                     pair_restore<K>(L.rec_old[k], L.rec_new[k], Ra, stage + (size_t)a * slab, n1, lane);
                 else
@@ -1057,6 +1092,7 @@ __global__ __launch_bounds__(FIT_THREADS) void fit_kernel(gt_fit_slot *__restric
 #undef GT_FIT_MEET
 #undef GT_FIT_TICK
     if (tid == 0) {
+        if (G > 1) group_leave(bar, G);
         const bool failed = L.abort_ || (G > 1 && xgetu(bar + 2) != 0u);
         if (member == 0) {
             const FitCtl &c = L.c;

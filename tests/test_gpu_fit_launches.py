@@ -1,0 +1,41 @@
+"""A fit advanced in launches of a few updates with another group size each
+time, against one launch of a single workgroup: the same bits.  Sizes at which
+the order of atoms is read ahead across (one atom, repeated inner iterations,
+the ends of outer iterations) and groups with more members than angles per
+member."""
+import importlib
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,nA,iters,block", [(1, 3, [4, 1], False), (2, 17, [3, 2], False), (5, 20, [2, 3], True),
+                                              (9, 33, [2, 1], False)])
+def test_launches_and_groups(gt, cuda, n, nA, iters, block):
+    F = importlib.import_module("2018_dictionary_tomography_amd.fit")
+    W = importlib.import_module("2018_dictionary_tomography_amd.workloads")
+    rng = np.random.default_rng(n)
+    I, x, r, _ = W.draw_aniso3(n, rng, rho=(0.05, 0.1))
+    T, ortho, dv = W.tilt_series(nA, 60.0, det=33)
+    space = gt.ProjSpace(orientations=T, ortho=ortho, detector=dv)
+    aspace = gt.AtomSpace(3, isotropic=False)
+    data = gt.ops.forward(gt.AtomElement(aspace, x, r, I, device=cuda), space)
+    start = gt.AtomElement(aspace, x + rng.normal(0, 0.02, x.shape), r, I * 0.8, device=cuda)
+    one, s1 = F.newton_fit(start, space, data, iters, tol=1e-9, group=1, block=block)
+    req = F.FitRequest(start, space, data, iters, tol=1e-9, block=block)
+    table = torch.as_tensor(np.frombuffer(req.slot_bytes(), dtype=np.uint8).copy(), device=cuda)
+    groups, k = [min(g, F.max_blocks()) for g in (3, 1, nA, 2, 8)], 0
+    while True:
+        g = groups[k % len(groups)]
+        F.run_blocks(table, 1, torch.as_tensor(F.block_table([g]), device=cuda), g, req.dim, 1 + k % 3)
+        s = F.read_slots(table, 1)[0]
+        k += 1
+        assert k < 200
+        if s.done:
+            break
+    assert (s.done, s.jj, s.accepted, s.E) == (s1.done, s1.jj, s1.accepted, s1.E)
+    for a, b in ((req.I, one.I), (req.x, one.x), (req.r, one.r), (req.resid, one.resid), (req.h, one.h)):
+        assert torch.equal(a, b)
