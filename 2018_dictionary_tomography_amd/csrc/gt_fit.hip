@@ -37,9 +37,10 @@
 // The members meet at two device-wide barriers per atom update (after the
 // per-angle contractions and after the per-angle energy changes); a barrier
 // wait is bounded in time.  An update is one latency chain: 300 atoms, 61 x
-// 96^2, 66 us at G = 4 (4 setup, 14 moments and contraction, 14 meeting and
-// sums over angles, 7 solve, 3 + 15 the proposal's setup and energy, 2 accept,
-// 7 commit); 69 us with a barrier word that the last arrival resets and
+// 96^2, 63 us at G = 4 (14 moments and contraction, 14 meeting and sums over
+// angles, 7 solve, 3 + 14 the proposal's setup and energy, 2 accept, 9 commit
+// beside the next atom's setup); 66 us with that setup after the commit, 69 us
+// with a barrier word that the last arrival resets and
 // releases, per-angle records read a line per lane, and the atom, its step
 // size and its place in the order read one after the other.  The solve and the accept logic run redundantly in
 // every member; member 0 writes the progress fields back at the end.
@@ -691,11 +692,18 @@ __global__ __launch_bounds__(FIT_THREADS) void fit_kernel(gt_fit_slot *__restric
     }
 
     const int my_budget = quota > 0 ? min(budget, quota) : (S.quota > 0 ? min(budget, S.quota) : budget);
-    for (int step = 0; step < my_budget; step++) {
+    // The residual of an update is committed (phase H) at the top of the next
+    // one, beside the choice and the set-up of the next atom: wave 0 does those
+    // (one latency chain of FP64, 4 us of 60) while the others commit.  The
+    // records of the next atom wait in the contraction's LDS, which is idle.
+    bool pending = false;
+    PairRec *const rec_next = reinterpret_cast<PairRec *>(L.wc);
+    static_assert(sizeof(L.wc) >= sizeof(L.rec_old), "the next atom's records fit the contraction's LDS");
+    for (int step = 0;; step++) {
         // ---- choose the atom, load its parameters -----------------------
         if (wave == 0) {
             const FitCtl &c = L.c;
-            bool stop = c.done != 0 || c.it >= S.max_outer || c.pos >= N;
+            bool stop = step >= my_budget || c.done != 0 || c.it >= S.max_outer || c.pos >= N;
             int j = 0, jn = -1;
             if (!stop) {
                 // the next entry of the order is read along with this one's atom
@@ -724,20 +732,46 @@ __global__ __launch_bounds__(FIT_THREADS) void fit_kernel(gt_fit_slot *__restric
                 L.skip = 0;
                 L.stop = stop;
                 L.j = j;
-                L.next[0] = L.next[1] = L.next[2] = 0;
+                L.next[0] = L.next[1] = 0;
+            }
+            wave_sync();
+        }
+        if (!pending) __syncthreads();
+        // ---- phase A: detector Gaussians of the current atom (own angles) --
+        // all threads, or wave 0 beside the commit
+        const int nset = pending ? 64 : FIT_THREADS;
+        if (tid < nset && !L.stop) {
+            PairRec *const dst = pending ? rec_next : L.rec_old;
+            for (int k = tid; k < nOwn; k += nset) {
+                PairGeom<D> g;
+                atom_from_theta<D>(L.th_old, iso, g);
+                angle_from_stash<D>(L.geo[k], Gm.lenT, g);
+                pair_setup<D>(g, det, nd, S.sorted, dst[k]);
             }
         }
+        // ---- phase H: commit the last update's residual, own angles ---------
+        // with a staging slab the energy pass already committed: undo on
+        // reject; without one, commit on accept
+        if (pending)
+            for (int k = next_angle(&L.next[2], lane); k < nOwn; k = next_angle(&L.next[2], lane)) {
+                const int a = member + G * k;
+                gmem<float> *Ra = resid + (size_t)a * slab;
+                if (stage)
+                    pair_restore<K>(L.rec_old[k], L.rec_new[k], Ra, stage + (size_t)a * slab, n1, lane);
+                else
+                    pair_delta4<K, 1>(L.rec_old[k], L.rec_new[k], L.p0, L.p1, Ra, nullptr, n1, lane,
+                                      reinterpret_cast<float2 *>(L.tab[wave]));
+            }
         __syncthreads();
+        GT_FIT_TICK(7);
         if (L.stop) break;
-        const int j = L.j;
-        // ---- phase A: detector Gaussians of the current atom (own angles) --
-        for (int k = tid; k < nOwn; k += FIT_THREADS) {
-            PairGeom<D> g;
-            atom_from_theta<D>(L.th_old, iso, g);
-            angle_from_stash<D>(L.geo[k], Gm.lenT, g);
-            pair_setup<D>(g, det, nd, S.sorted, L.rec_old[k]);
+        if (pending) {
+            for (int i = tid; i < 4 * nOwn; i += FIT_THREADS)
+                reinterpret_cast<int4 *>(L.rec_old)[i] = reinterpret_cast<const int4 *>(rec_next)[i];
+            __syncthreads();
         }
-        __syncthreads();
+        pending = false;
+        const int j = L.j;
         GT_FIT_TICK(0);
         // ---- phase B+C: per-angle pixel moments, then that angle's FP64
         //      gradient/Hessian record, both by the wave that took the angle --
@@ -980,8 +1014,8 @@ __global__ __launch_bounds__(FIT_THREADS) void fit_kernel(gt_fit_slot *__restric
         GT_FIT_TICK(3);
         if (L.stop) break;
         if (L.skip) {  // block variant: nothing to try for this block
+            __syncthreads();  // (the flag is cleared with the next choice)
             if (tid == 0) fit_advance(L.c, S, true);
-            __syncthreads();
             continue;
         }
         // ---- phase E: detector Gaussians of the proposal -------------------
@@ -1066,28 +1100,14 @@ __global__ __launch_bounds__(FIT_THREADS) void fit_kernel(gt_fit_slot *__restric
                 if (S.Ehist && member == 0) S.Ehist[c.jj] = c.E;
                 c.updates++;
                 L.accept = accept;
+                L.next[2] = 0;
+                // loop control (NewtonGaussian.py:50-98, :131-222)
+                fit_advance(c, S, false);
             }
         }
         __syncthreads();
         GT_FIT_TICK(6);
-        // ---- phase H: commit the residual of the own angles ----------------
-        // with a staging slab the energy pass already committed: undo on
-        // reject; without one, commit on accept
-        if (stage ? !L.accept : L.accept) {
-            for (int k = next_angle(&L.next[2], lane); k < nOwn; k = next_angle(&L.next[2], lane)) {
-                const int a = member + G * k;
-                gmem<float> *Ra = resid + (size_t)a * slab;
-                if (stage)
-                    pair_restore<K>(L.rec_old[k], L.rec_new[k], Ra, stage + (size_t)a * slab, n1, lane);
-                else
-                    pair_delta4<K, 1>(L.rec_old[k], L.rec_new[k], L.p0, L.p1, Ra, nullptr, n1, lane,
-                                      reinterpret_cast<float2 *>(L.tab[wave]));
-            }
-        }
-        // ---- loop control (NewtonGaussian.py:50-98, :131-222) ---------------
-        if (tid == 0) fit_advance(L.c, S, false);
-        __syncthreads();
-        GT_FIT_TICK(7);
+        pending = stage ? !L.accept : L.accept;
     }
 #undef GT_FIT_MEET
 #undef GT_FIT_TICK
