@@ -66,7 +66,7 @@ class gt_fit_block(ctypes.Structure):
 
 
 BLOCK_BYTES = ctypes.sizeof(gt_fit_block)
-ANGLES_PER_MEMBER = 16  # one angle per wave of a 16-wave workgroup
+ANGLES_PER_MEMBER = 4  # see default_group
 
 
 def _declare():
@@ -74,8 +74,13 @@ def _declare():
 
 
 def default_group(nA):
-    """Workgroups that advance one fit together: enough that each holds about
-    one angle per wave, at most 8."""
+    """Workgroups that advance one fit together: one per 4 angles, at most 8 (a
+    group's workgroups wait for each other and must all be on the device, so
+    concurrent fits share its 256).  An update at 16 angles per workgroup and
+    at 4, microseconds: 30 angles x 64^2 49.7 and 42.6, 61 x 96^2 63.0 and
+    56.7, 61 x 160^2 99.0 and 88.5, 2D 60 x 128 29.8 and 27.3; more than 4 per
+    workgroup leaves the waves of a SIMD in each other's way, fewer gains 4 to
+    10% more for twice the workgroups."""
     return max(1, min(8, -(-int(nA) // ANGLES_PER_MEMBER)))
 
 
