@@ -42,12 +42,11 @@ class GaussTomo:
     # -- derivatives -----------------------------------------------------
     def _derivs(self, atoms, C, order, mode):
         C = C.data if hasattr(C, "data") and not isinstance(C, torch.Tensor) else C
-        f, g, H = ops.derivs(atoms, self.range, C, mode, order)
-        f = f.cpu().numpy().reshape(-1, 1)
-        g = g.cpu().numpy()
+        f, g, H = ops.derivs_host(atoms, self.range, C, mode, order)
+        f = f.reshape(-1, 1)
         if order == 1:
             return f, g
-        return f, g, H.cpu().numpy()
+        return f, g, H
 
     def derivs(self, atoms, C, order=2):
         """Per atom: R(a_i).C, its gradient and Hessian (atomFuncs.py:130-142).

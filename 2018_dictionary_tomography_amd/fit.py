@@ -130,7 +130,7 @@ class FitRequest:
     fit alone or 256 at once)."""
 
     def __init__(self, atoms, space, data, max_iter, tol=1e-4, min_iter=1, seed=1, record=True, device=None,
-                 reg=None, block=False, perm=None, h=None, stage=False, gd_dims=None):
+                 reg=None, block=False, perm=None, h=None, stage=False, gd_dims=None, settle=True):
         dev = device or atoms.I.device
         self.reg = as_regulariser(reg)
         # variant: 0 Newton, 1 block Newton, 2 block gradient descent over gd_dims
@@ -151,47 +151,41 @@ class FitRequest:
         if max(self.geom.n0, self.geom.n1) > MAX_DETECTOR:
             raise ValueError(f"the fitter supports detectors up to {MAX_DETECTOR} pixels per axis")
         self.dim = self.geom.dim
+        n = int(atoms.I.numel())
+        if perm is None:
+            perm = permutations(n, self.max_outer, seed)
+        else:
+            perm = np.asarray(perm, dtype=np.int32).reshape(-1, n)
+            if perm.shape[0] < self.max_outer or not all(np.array_equal(np.sort(p), np.arange(n)) for p in perm):
+                raise ValueError("perm must hold max_outer permutations of range(N)")
+        if h is None:
+            h = np.full(nblk * n, 1e-2 if self.mode == 2 else 1.0)  # GD_lib.py:99, NewtonGaussian.py:25,119
+        else:
+            h = np.ascontiguousarray(h, dtype=np.float64).reshape(-1)
+            if h.size != nblk * n:
+                raise ValueError(f"h must hold {nblk * n} step sizes")
+        # slot scratch (zeros), step sizes and atom order in one upload
+        lib = _declare()
+        ns, nh = lib.gt_fit_scratch_bytes(self.geom.nA), 8 * h.size
+        up = np.zeros(ns + nh + 4 * self.max_outer * n, dtype=np.uint8)
+        up[ns:ns + nh] = h.view(np.uint8)
+        up[ns + nh:] = np.ascontiguousarray(perm[: self.max_outer], dtype=np.int32).reshape(-1).view(np.uint8)
+        up = torch.as_tensor(up, device=dev)
+        self.scratch = up[:ns]
+        self.h = up[ns:ns + nh].view(torch.float64)
+        self.perm = up[ns + nh:].view(torch.int32).view(self.max_outer, n)
         self.I = atoms.I.detach().to(dev, torch.float32).clone().contiguous()
         self.x = atoms.x.detach().to(dev, torch.float32).clone().contiguous()
         self.r = atoms.r.detach().to(dev, torch.float32).clone().contiguous()
-        self.N = int(self.I.numel())
+        self.N = n
         self.iso = int(self.r.shape[1] == 1)
         data = data.data if hasattr(data, "data") and not isinstance(data, torch.Tensor) else data
         self.data = torch.as_tensor(data, device=dev).to(torch.float32).reshape(self.geom.shape).contiguous()
-        self.resid = ops.forward(self, space).sub_(self.data)
-        r64 = self.resid.double()
-        self.F0 = float(0.5 * (r64 * r64).sum())
-        # E = F + reg(recon) (NewtonGaussian.py:28-30): the sum of the finite
-        # per-atom terms and the count of the others
-        self.ninf0, self.Rsum0 = 0, 0.0
-        if self.reg.kind != 0 and self.N > 0:
-            val = self.reg.terms(self, 0)[0]
-            fin = torch.isfinite(val)
-            self.ninf0 = int((~fin).sum())
-            self.Rsum0 = float(val[fin].sum())
-        self.E0 = self.F0 + (float("inf") if self.ninf0 else self.Rsum0)
-        if perm is None:
-            perm = permutations(self.N, self.max_outer, seed)
-        perm = np.asarray(perm, dtype=np.int32).reshape(-1, self.N)
-        if perm.shape[0] < self.max_outer or not all(np.array_equal(np.sort(p), np.arange(self.N)) for p in perm):
-            raise ValueError("perm must hold max_outer permutations of range(N)")
-        self.perm = torch.as_tensor(perm[: self.max_outer].copy(), device=dev).contiguous()
-        if h is None:
-            h0 = 1e-2 if self.mode == 2 else 1.0  # GD_lib.py:99, NewtonGaussian.py:25,119
-            self.h = torch.full((nblk * self.N,), h0, dtype=torch.float64, device=dev)
-        else:
-            h = np.asarray(h, dtype=np.float64).reshape(-1)
-            if h.size != nblk * self.N:
-                raise ValueError(f"h must hold {nblk * self.N} step sizes")
-            self.h = torch.as_tensor(h.copy(), device=dev)
+        self.data = self.data.detach().resolve_neg()
+        self.resid, self.start_energy = ops.residual(self, space, self.data)
         nh = nblk * self.max_outer * self.max_inner * self.N + 1
         self.Ehist = torch.zeros(nh, dtype=torch.float64, device=dev) if record else None
         self.Fhist = torch.zeros(nh, dtype=torch.float64, device=dev) if record else None
-        if record:
-            self.Ehist[0] = self.E0
-            self.Fhist[0] = self.F0
-        lib = _declare()
-        self.scratch = torch.zeros(lib.gt_fit_scratch_bytes(self.geom.nA), dtype=torch.uint8, device=dev)
         # old residual of the update in flight: lets the energy pass commit at once
         self.stage = torch.empty(self.geom.shape, dtype=torch.float32, device=dev) if stage else None
         g = self.geom
@@ -203,13 +197,33 @@ class FitRequest:
             I=self.I.data_ptr(), x=self.x.data_ptr(), r=self.r.data_ptr(), resid=self.resid.data_ptr(),
             h=self.h.data_ptr(), Ehist=self.Ehist.data_ptr() if record else None, scratch=self.scratch.data_ptr(),
             stage=self.stage.data_ptr() if stage else None,
-            it=0, pos=0, inner=0, jj=0, brk0=1, brk1=1, done=0 if self.N > 0 else 1, pad1=0, E=self.E0,
+            it=0, pos=0, inner=0, jj=0, brk0=1, brk1=1, done=0 if self.N > 0 else 1, pad1=0, E=0.0,
             updates=0, accepted=0, block=self.mode, reg_kind=int(self.reg.kind),
-            Fhist=self.Fhist.data_ptr() if record else None, blk=0, ninf=self.ninf0, F=self.F0, Rsum=self.Rsum0,
+            Fhist=self.Fhist.data_ptr() if record else None, blk=0, ninf=0, F=0.0, Rsum=0.0,
             gd_nblk=len(self.gd_blocks))
         self.slot.reg_p[:] = [float(v) for v in self.reg.params()]
         for i, b in enumerate(self.gd_blocks):
             self.slot.gd_blocks[i] = b
+        if settle:
+            self.settle(float(self.start_energy))
+
+    def settle(self, F0):
+        """The start energies, from the fidelity F0 brought over by the caller."""
+        self.F0 = F0
+        # E = F + reg(recon) (NewtonGaussian.py:28-30): the sum of the finite
+        # per-atom terms and the count of the others
+        self.ninf0, self.Rsum0 = 0, 0.0
+        if self.reg.kind != 0 and self.N > 0:
+            val = self.reg.terms(self, 0)[0]
+            fin = torch.isfinite(val)
+            self.ninf0 = int((~fin).sum())
+            self.Rsum0 = float(val[fin].sum())
+        self.E0 = self.F0 + (float("inf") if self.ninf0 else self.Rsum0)
+        if self.Ehist is not None:
+            self.Ehist[0] = self.E0
+            self.Fhist[0] = self.F0
+        s = self.slot
+        s.E, s.F, s.ninf, s.Rsum = self.E0, self.F0, self.ninf0, self.Rsum0
 
     def slot_bytes(self):
         return bytes(self.slot)

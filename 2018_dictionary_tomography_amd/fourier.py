@@ -150,10 +150,25 @@ class DevicePlanes:
     """Device copy of a plane sample set and its gt_kplanes struct."""
 
     def __init__(self, form, k0, k1, w0, w1, device, f64=False):
-        dt = torch.float64 if f64 else torch.float32
-        cv = lambda a: None if a is None else torch.as_tensor(np.ascontiguousarray(
-            a.detach().cpu().numpy() if isinstance(a, torch.Tensor) else a, dtype=np.float64), device=device).to(dt)
-        self.k0, self.k1, self.w0, self.w1 = cv(k0), cv(k1), cv(w0), cv(w1)
+        # converted and checked on the host, brought over in one transfer
+        dt = np.float64 if f64 else np.float32
+        host = []
+        with np.errstate(over="ignore"):
+            for a in (k0, k1, w0, w1):
+                if isinstance(a, torch.Tensor):
+                    a = a.detach().cpu().numpy()
+                host.append(None if a is None else np.ascontiguousarray(a, dtype=np.float64).astype(dt))
+        at, size = [], 0
+        for a in host:
+            at.append(size)
+            size += 0 if a is None else -(-a.size // 64) * 64  # every array on its own 256 bytes
+        packed = np.zeros(size, dtype=dt)
+        for a, o in zip(host, at):
+            if a is not None:
+                packed[o:o + a.size] = a.reshape(-1)
+        buf = torch.as_tensor(packed, device=device)
+        self.k0, self.k1, self.w0, self.w1 = (None if a is None else buf[o:o + a.size].view(a.shape)
+                                              for a, o in zip(host, at))
         self.form, self.f64 = form, f64
         m0 = self.k0.numel()
         if form == _lib.GT_KP_2D_LINE:
@@ -163,8 +178,8 @@ class DevicePlanes:
         else:
             nA, m1 = self.w0.shape[0], self.k1.numel()
         self.nA, self.m0, self.m1 = int(nA), int(m0), int(m1)
-        asc = lambda t: t is None or ops._ascending(t.cpu().numpy())
-        sorted_ = int(asc(self.k0) and (form == _lib.GT_KP_2D_LINE or asc(self.k1)))
+        asc = lambda a: a is None or ops._ascending(a)
+        sorted_ = int(asc(host[0]) and (form == _lib.GT_KP_2D_LINE or asc(host[1])))
         ptr = lambda t: t.data_ptr() if t is not None else None
         cls = _lib.gt_kplanes64 if f64 else _lib.gt_kplanes
         self.struct = cls(form, self.nA, self.m0, self.m1, sorted_, ptr(self.k0), ptr(self.k1), ptr(self.w0),

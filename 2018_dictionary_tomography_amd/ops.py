@@ -132,9 +132,8 @@ def n_params(dim, iso):
     return 1 + dim + (1 if iso else dim * (dim + 1) // 2)
 
 
-def derivs(atoms, space, C, mode="L2", order=2, want_f=True):
-    """Per-atom (f, g, H) in FP64 on the device.  mode: 'linear', 'L2' or 'resid'."""
-    lib = load()
+def _derivs_args(atoms, space, C, mode):
+    """(mode, atoms struct, geometry, C on the device, parameters per atom)."""
     mode = MODES[mode]
     dev = atoms.I.device
     geom = device_geometry(space, dev)
@@ -143,16 +142,40 @@ def derivs(atoms, space, C, mode="L2", order=2, want_f=True):
     C = torch.as_tensor(C, device=dev).to(torch.float32).contiguous()
     if tuple(C.shape) != tuple(geom.shape):
         raise ValueError(f"C must have shape {geom.shape}, got {tuple(C.shape)}")
-    P = n_params(a.dim, a.iso)
-    n = a.n
-    f = torch.zeros(n, dtype=torch.float64, device=dev) if (want_f and mode != GT_MODE_RESID) else None
-    g = torch.empty((n, P), dtype=torch.float64, device=dev)
-    H = torch.empty((n, P, P), dtype=torch.float64, device=dev) if order > 1 else None
+    return mode, a, geom, C, n_params(a.dim, a.iso)
+
+
+def _derivs_run(a, geom, C, mode, order, f, g, H, dev):
+    lib = load()
     need = lib.gt_derivs_workspace(ctypes.byref(a), ctypes.byref(geom.struct), mode)
     ws = _ws.get(need, dev)
     check(lib.gt_derivs(ctypes.byref(a), ctypes.byref(geom.struct), _ptr(C), mode, order, _ptr(f), _ptr(g), _ptr(H),
                         _ptr(ws), ws.numel(), stream_handle(dev)), "gt_derivs")
+
+
+def derivs(atoms, space, C, mode="L2", order=2, want_f=True):
+    """Per-atom (f, g, H) in FP64 on the device.  mode: 'linear', 'L2' or 'resid'."""
+    mode, a, geom, C, P = _derivs_args(atoms, space, C, mode)
+    dev, n = atoms.I.device, a.n
+    f = torch.empty(n, dtype=torch.float64, device=dev) if (want_f and mode != GT_MODE_RESID) else None
+    g = torch.empty((n, P), dtype=torch.float64, device=dev)
+    H = torch.empty((n, P, P), dtype=torch.float64, device=dev) if order > 1 else None
+    _derivs_run(a, geom, C, mode, order, f, g, H, dev)
     return f, g, H
+
+
+def derivs_host(atoms, space, C, mode="L2", order=2):
+    """derivs ('linear' or 'L2') as host arrays: f, g and H side by side on the
+    device and brought over in one transfer."""
+    mode, a, geom, C, P = _derivs_args(atoms, space, C, mode)
+    dev, n = atoms.I.device, a.n
+    buf = torch.empty(n * (1 + P + (P * P if order > 1 else 0)), dtype=torch.float64, device=dev)
+    g = buf[n:n + n * P]
+    H = buf[n + n * P:] if order > 1 else None
+    _derivs_run(a, geom, C, mode, order, buf[:n], g, H, dev)
+    out = buf.cpu().numpy()
+    return (out[:n], out[n:n + n * P].reshape(n, P),
+            out[n + n * P:].reshape(n, P, P) if order > 1 else None)
 
 
 def forward_derivs(atoms, space, data, order=2, out=None, want_f=True):

@@ -240,8 +240,9 @@ class FitServer:
         self.graph.replay()
 
     def _write_slot(self, i, slot):
-        b = torch.frombuffer(bytearray(bytes(slot)), dtype=torch.uint8)
-        self.table[i * F.SLOT_BYTES:(i + 1) * F.SLOT_BYTES].copy_(b.to(self.dev))
+        """Slot i of the host's table, which a launch's read-back keeps current
+        and the next plan uploads whole."""
+        self.host.numpy()[i * F.SLOT_BYTES:(i + 1) * F.SLOT_BYTES] = np.frombuffer(bytes(slot), dtype=np.uint8)
 
     def _read_active(self):
         """(index, gt_fit_slot) of every occupied slot, read back after a launch."""
@@ -251,7 +252,9 @@ class FitServer:
                 for i in range(self.max_slots) if self.slots[i] is not None]
 
     def _plan(self, progress):
-        """Rewrite the block table: groups and quotas of the active slots."""
+        """Upload the slot table and rewrite the block table: groups and quotas
+        of the active slots.  (Neither host buffer is written again before the
+        launch that follows has been waited for.)"""
         act = [i for i in range(self.max_slots) if self.slots[i] is not None]
         specs = [self.slots[i][0] for i in act]
         remaining = []
@@ -267,7 +270,8 @@ class FitServer:
                 rows[b] = (i, m, g, q)
                 b += 1
         self.blocks_host.copy_(torch.from_numpy(rows))
-        self.blocks.copy_(self.blocks_host)
+        self.blocks.copy_(self.blocks_host, non_blocking=True)
+        self.table.copy_(self.host, non_blocking=True)
         self.used_blocks = b
         return dict(zip(act, groups))
 
@@ -287,6 +291,7 @@ class FitServer:
         progress_map = {}
         # the empty table must not be left with stale slots
         self.table.zero_()
+        self.host.zero_()
         torch.cuda.synchronize(self.dev)
         dirty = True
         next_note = progress_every
@@ -303,18 +308,23 @@ class FitServer:
             # admit FIFO while a slot and memory are free
             free = [i for i in range(self.max_slots) if self.slots[i] is None]
             ta = time.perf_counter()
+            new = []
             while queue and free and reserved + queue[0].footprint_bytes() <= self.hbm_budget:
                 spec = queue.pop(0)
                 i = free.pop(0)
                 start, space, data = payloads[spec.rid] if payloads else build_request(spec, self.dev)
                 req = F.FitRequest(start, space, data, [spec.max_iter, 1], record=False,
-                                   stage=spec.N <= self.stage_max_atoms)
-                self._write_slot(i, req.slot)
+                                   stage=spec.N <= self.stage_max_atoms, settle=False)
+                new.append((i, req))
                 self.slots[i] = (spec, req, time.perf_counter() - t0)
                 progress_map[i] = 0
                 reserved += spec.footprint_bytes()
                 active += 1
                 dirty = True
+            if new:  # all their start energies in one transfer
+                for (i, req), F0 in zip(new, torch.stack([req.start_energy for _, req in new]).tolist()):
+                    req.settle(F0)
+                    self._write_slot(i, req.slot)
             st.admit_s += time.perf_counter() - ta
             st.admitted_bytes_peak = max(st.admitted_bytes_peak, reserved)
             if active == 0:
@@ -350,7 +360,7 @@ class FitServer:
                 st.failed += int(s.done == 3)
                 st.singular += int(s.done == 2)
                 if self.keep_results:
-                    st.results[spec.rid] = (req.I.clone(), req.x.clone(), req.r.clone(), s.E, s.done, s.updates)
+                    st.results[spec.rid] = (req.I, req.x, req.r, s.E, s.done, s.updates)
                 reserved -= spec.footprint_bytes()
                 active -= 1
                 self.slots[i] = None

@@ -39,3 +39,30 @@ def test_launches_and_groups(gt, cuda, n, nA, iters, block):
     assert (s.done, s.jj, s.accepted, s.E) == (s1.done, s1.jj, s1.accepted, s1.E)
     for a, b in ((req.I, one.I), (req.x, one.x), (req.r, one.r), (req.resid, one.resid), (req.h, one.h)):
         assert torch.equal(a, b)
+
+
+def test_request_inputs(gt, cuda):
+    """What a request holds on the device, from the forms its inputs may take:
+    no atoms, step sizes and an order given as strided arrays, data as a view."""
+    F = importlib.import_module("2018_dictionary_tomography_amd.fit")
+    W = importlib.import_module("2018_dictionary_tomography_amd.workloads")
+    rng = np.random.default_rng(3)
+    I, x, r, _ = W.draw_aniso3(4, rng, rho=(0.05, 0.1))
+    T, ortho, dv = W.tilt_series(5, 60.0, det=21)
+    space = gt.ProjSpace(orientations=T, ortho=ortho, detector=dv)
+    aspace = gt.AtomSpace(3, isotropic=False)
+    atoms = gt.AtomElement(aspace, x, r, I, device=cuda)
+    data = torch.as_tensor(rng.normal(size=(5, 21, 21)), dtype=torch.float32, device=cuda)
+    perm, h = rng.permutation(4).astype(np.int64), rng.uniform(0.5, 2.0, 8)[::2]
+    for d in (data, torch.complex(data, -data).conj().imag, data.transpose(1, 2).contiguous().transpose(1, 2),
+              data.cpu(), data.double().reshape(-1)):
+        req = F.FitRequest(atoms, space, d, [1, 1], perm=np.repeat(perm, 2)[None, ::2], h=h)
+        assert torch.equal(req.resid, gt.ops.forward(atoms, space) - data)
+        assert abs(req.F0 - 0.5 * float((req.resid.double() ** 2).sum())) <= data.numel() * 2.0 ** -52 * req.F0
+        assert req.perm.cpu().tolist() == [perm.tolist()] and req.h.cpu().tolist() == h.tolist()
+        assert int(req.scratch.sum()) == 0 and (req.slot.E, req.slot.F) == (req.F0, req.F0)
+    for t in (req.I, req.x, req.r):
+        assert t.data_ptr() not in [a.data_ptr() for a in (atoms.I, atoms.x, atoms.r)]
+    none = F.FitRequest(gt.AtomElement(aspace, np.zeros((0, 3)), np.zeros((0, 6)), np.zeros(0), device=cuda), space,
+                        data, [2, 1])
+    assert none.slot.active == 0 and none.slot.done == 1 and torch.equal(none.resid, -data)
