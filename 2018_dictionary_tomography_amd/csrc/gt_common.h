@@ -157,6 +157,12 @@ __device__ inline void wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// The value of lane K of each row of 16 lanes, in the whole row
+template <int K> __device__ inline float row_bcast(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + K, 0xf, 0xf, true));
+}
+
 // sin(2 pi t) and cos(2 pi t) of a phase t in turns, |t| <= 256: the
 // hardware sine and cosine, whose argument is in turns (quarter-rate, like
 // exp2); measured maximum absolute error 1.25e-7 for |t| <= 1.5 on gfx950.

@@ -165,11 +165,6 @@ __device__ inline void stage_rects(const PairRec *__restrict__ ra, int base, int
     wave_lists<F3_WAVES, F3_WAVES>(mask, wl, cnt, wlen);
 }
 
-// the value of lane K of each row of 16 lanes, in the whole row
-template <int K> __device__ inline float row_bcast(float v)
-{
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + K, 0xf, 0xf, true));
-}
 // A group of four records as the pixels read it: per column (the terms linear
 // and constant in the row, q0, alpha), per row the offset from the centre.  No
 // cut-off test: every record in a wave's list reaches its rectangle, and the

@@ -674,39 +674,63 @@ __device__ inline int psf_stage(const PsfRec *__restrict__ ra, int base, int N, 
     return total;
 }
 
-// The forward of 2D detectors with pixel integrals: block = (angle, 8 x 64
+// The forward of 2D detectors with pixel integrals: block = (angle, 8 x 32
 // pixels) of 4 waves, numbered centre tiles first (block b: angle b % nA, tile
-// of Morton rank b / nA); wave w owns the 8 x 16 pixels of columns 16 w .. 16 w
-// + 15, lane l column l % 16, rows l / 16 and l / 16 + 4.  A thread tests one
-// record against the four rectangles (index box, then the support against the
-// rectangle widened by half a pixel, support_meets_rect); the waves walk their
-// own lists with the record and its node table in scalar registers.  Four
-// records' values are summed in FP32 and added to an FP64 total.  Bound by VALU
-// issue (an exponential counts four): with the node tables a pixel costs 5 to
-// 13 exponentials instead of 9 to 36 and one form evaluation per node; 1000
-// atoms, 61 x 128^2: 1.59 -> 0.43 ms.
-constexpr int PF_WAVES = 4, PF_CHUNK = PF_WAVES * 64, PF_ROWS = 8, PF_COLS = 16 * PF_WAVES;
+// of Morton rank b / nA); waves w and w + 2 own the 8 x 16 pixels of columns 16
+// (w % 2) .. + 15, lane l column l % 16, rows l / 16 and l / 16 + 4.  A thread
+// tests one record against the rectangles (index box, then the support against
+// the rectangle widened by half a pixel, support_meets_rect); the two waves of
+// a rectangle walk its list in turns of four records and add their sums.
+//
+// Vector issue and the evenness of the blocks bound it.  Every exponential of a
+// cell is a factor of its column times a factor of its row (PfTab): a wave forms
+// those of four records at once, 1.5 exponentials per record, lane and node pair
+// instead of 8 (two pixels, two axes, two signs) and a product per pixel.  Four
+// records' values are summed in FP32 and added to an FP64 total.  1000 atoms, 61
+// x 128^2: 1.59 ms with a form per node, 0.45 with the node weights tabulated
+// (8 x 64 pixels per block), 0.39 with the factors tabulated, 0.35 with 8 x 32
+// pixels, 0.34 with two waves per rectangle (four: 0.40).
+constexpr int PF_RECTS = 2, PF_GROUPS = 2, PF_WAVES = PF_RECTS * PF_GROUPS;
+constexpr int PF_CHUNK = PF_WAVES * 64, PF_ROWS = 8, PF_COLS = 16 * PF_RECTS;
 
-template <int NP> __device__ inline float psf_pixel_nodes(smem<float> *w, float t0, float t1)
+// A group of four records as the pixels of a wave's rectangle read it.  Along
+// a row of pixels a record's exponents at the nodes, t_k x_i, are linear in the
+// column, along a column in the row, so every factor 2^(t_k x_i) is one of the
+// column (at the rectangle's fifth row) times one of the row.
+struct PfTab {
+    float4 cn[4][3][16];  // node pair i, column: 2^(t0 x), 2^(-t0 x), 2^(t1 x), 2^(-t1 x)
+    float4 rn[4][3][8];   // the rows' factors of the same
+    float2 c[4][16];      // the centre's exponent: its terms linear and constant in the row
+    float2 r[4][4];       // the offsets of rows r and r + 4
+};
+
+template <int NP>
+__device__ inline float psf_pixel_nodes(smem<float> *w, const float4 (&cn)[NP / 2], const float4 (&rn)[NP / 2])
 {
-    constexpr int M = PsfNodes<NP>::M;
+    constexpr int M = PsfNodes<NP>::M, ODD = PsfNodes<NP>::ODD;
     float Xe[M], Xo[M], Ye[M], Yo[M];
-    psf_axis<NP>(t0, Xe, Xo);
-    psf_axis<NP>(t1, Ye, Yo);
+#pragma unroll
+    for (int i = 0; i < NP / 2; i++) {
+        const float x = cn[i].y * rn[i].y, y = cn[i].w * rn[i].w;
+        Xe[i + ODD] = fmaf(cn[i].x, rn[i].x, x);
+        Xo[i + ODD] = fmaf(cn[i].x, rn[i].x, -x);
+        Ye[i + ODD] = fmaf(cn[i].z, rn[i].z, y);
+        Yo[i + ODD] = fmaf(cn[i].z, rn[i].z, -y);
+    }
     float s = 0.0f;
 #pragma unroll
     for (int m0 = 0; m0 < M; m0++) {
         float a = 0.0f, b = 0.0f;
 #pragma unroll
         for (int m1 = 0; m1 < M; m1++) {
-            const bool z = PsfNodes<NP>::ODD && (m0 == 0 || m1 == 0);
-            if (PsfNodes<NP>::ODD && m1 == 0)
+            const bool z = ODD && (m0 == 0 || m1 == 0);
+            if (ODD && m1 == 0)
                 a = w[m0 * M * 2];
             else
                 a = fmaf(w[(m0 * M + m1) * 2], Ye[m1], a);
             if (!z) b = fmaf(w[(m0 * M + m1) * 2 + 1], Yo[m1], b);
         }
-        if (PsfNodes<NP>::ODD && m0 == 0)
+        if (ODD && m0 == 0)
             s += a;
         else
             s = fmaf(Xe[m0], a, fmaf(Xo[m0], b, s));
@@ -714,34 +738,36 @@ template <int NP> __device__ inline float psf_pixel_nodes(smem<float> *w, float 
     return s;
 }
 
-// One record's integrals over a lane's two pixels.
+// Record u of the group: its integrals over a lane's two pixels.
 template <int NP>
-__device__ inline void psf_two_pixels(smem<PsfRec> *R, smem<float> *w, float pc, float prA, float prB, float &vA,
-                                      float &vB)
+__device__ inline void psf_two_pixels(const PfTab &T, int u, float q0, smem<float> *w, int lane, float &vA, float &vB)
 {
-    const float q0 = R->r.q[0], q1 = R->r.q[1], q2 = R->r.q[2], q3 = R->r.q[3], q4 = R->r.q[4], q5 = R->r.q[5];
-    const float d1 = (pc - R->r.c_hi[1]) - R->r.c_lo[1];
-    const float row = fmaf(q1, d1, q3), col = fmaf(fmaf(q2, d1, q4), d1, q5);
-    const float l1 = fmaf(2.0f * q2, d1, q4);
-    const float dA = (prA - R->r.c_hi[0]) - R->r.c_lo[0], dB = (prB - R->r.c_hi[0]) - R->r.c_lo[0];
-    const float hA = fmaf(q0, dA, row), hB = fmaf(q0, dB, row);
-    const float eA = fmaf(hA, dA, col), eB = fmaf(hB, dB, col);
-    const float s0 = R->s[0], s1 = R->s[1];
-    const float nA = psf_pixel_nodes<NP>(w, fmaf(q0, dA, hA) * s0, fmaf(q1, dA, l1) * s1);
-    const float nB = psf_pixel_nodes<NP>(w, fmaf(q0, dB, hB) * s0, fmaf(q1, dB, l1) * s1);
+    float4 cn[NP / 2], rn[NP / 2];
+    const float2 c = T.c[u][lane & 15], r = T.r[u][lane >> 4];
+#pragma unroll
+    for (int i = 0; i < NP / 2; i++) {
+        cn[i] = T.cn[u][i][lane & 15];
+        rn[i] = T.rn[u][i][lane >> 4];
+    }
+    const float eA = fmaf(fmaf(q0, r.x, c.x), r.x, c.y), eB = fmaf(fmaf(q0, r.y, c.x), r.y, c.y);
+    const float nA = psf_pixel_nodes<NP>(w, cn, rn);
+#pragma unroll
+    for (int i = 0; i < NP / 2; i++) rn[i] = T.rn[u][i][(lane >> 4) + 4];
+    const float nB = psf_pixel_nodes<NP>(w, cn, rn);
     vA = eA > PSF_CELL_MIN ? __builtin_amdgcn_exp2f(eA) * nA : 0.0f;
     vB = eB > PSF_CELL_MIN ? __builtin_amdgcn_exp2f(eB) * nB : 0.0f;
 }
 
-__global__ __launch_bounds__(PF_WAVES * 64) void psf_project_kernel(const PsfRec *__restrict__ recs,
-                                                                    const PsfNode2 *__restrict__ nodes, int N, int nA,
-                                                                    int n0, int n1, const float *__restrict__ p0,
-                                                                    const float *__restrict__ p1,
-                                                                    float *__restrict__ R, int e0, int e1)
+// (96 VGPRs, five waves per SIMD; six: the same time with 72 bytes of spills)
+__global__ __launch_bounds__(PF_WAVES * 64) __attribute__((amdgpu_waves_per_eu(5))) void psf_project_kernel(
+    const PsfRec *__restrict__ recs, const PsfNode2 *__restrict__ nodes, int N, int nA, int n0, int n1,
+    const float *__restrict__ p0, const float *__restrict__ p1, float *__restrict__ R, int e0, int e1)
 {
-    __shared__ unsigned short wl[PF_WAVES][PF_CHUNK];
-    __shared__ int cnt[PF_WAVES][PF_WAVES];
-    __shared__ int wlen[PF_WAVES];
+    __shared__ alignas(16) unsigned short wl[PF_RECTS][PF_CHUNK];  // read four at a time
+    __shared__ int cnt[PF_RECTS][PF_WAVES];
+    __shared__ int wlen[PF_RECTS];
+    __shared__ PfTab tab[PF_WAVES];
+    __shared__ double part[PF_WAVES - PF_RECTS][2][64];
     const int tilesR = (n0 + PF_ROWS - 1) / PF_ROWS, tilesC = (n1 + PF_COLS - 1) / PF_COLS;
     const int a = (int)(blockIdx.x % (unsigned)nA);
     const int e[3] = {e0, e1, 0};
@@ -750,13 +776,18 @@ __global__ __launch_bounds__(PF_WAVES * 64) void psf_project_kernel(const PsfRec
     if (t[0] >= tilesR || t[1] >= tilesC) return;  // whole block: no tile of this rank
     const int row0 = centre_out(t[0], tilesR) * PF_ROWS, col0 = centre_out(t[1], tilesC) * PF_COLS;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int i1 = col0 + 16 * wave + (lane & 15), rA = row0 + (lane >> 4), rB = rA + 4;
+    const int rect = wave % PF_RECTS, grp = wave / PF_RECTS;
+    const int i1 = col0 + 16 * rect + (lane & 15), rA = row0 + (lane >> 4), rB = rA + 4;
     const float pc = p1[min(i1, n1 - 1)], prA = p0[min(rA, n0 - 1)], prB = p0[min(rB, n0 - 1)];
     const float s0 = psf_cell_half(p0), s1 = psf_cell_half(p1);
+    // the rectangle's rows and columns from its fifth row and ninth column on
+    const float pr8 = p0[min(row0 + (lane & 7), n0 - 1)], prc = p0[min(row0 + 4, n0 - 1)];
+    const float pcc = p1[min(col0 + 16 * rect + 8, n1 - 1)];
+    const bool regular = __all(fabsf(pr8 - prc) <= 17.0f * s0 && fabsf(pc - pcc) <= 33.0f * s1);
     const float xa = p0[row0] - s0, xb = p0[min(row0 + PF_ROWS - 1, n0 - 1)] + s0;
-    float cy[2 * PF_WAVES];
+    float cy[2 * PF_RECTS];
 #pragma unroll
-    for (int w = 0; w < PF_WAVES; w++) {
+    for (int w = 0; w < PF_RECTS; w++) {
         cy[2 * w] = p1[min(col0 + 16 * w, n1 - 1)] - s1;
         cy[2 * w + 1] = p1[min(col0 + 16 * w + 15, n1 - 1)] + s1;
     }
@@ -772,7 +803,7 @@ __global__ __launch_bounds__(PF_WAVES * 64) void psf_project_kernel(const PsfRec
             const int4 bx = reinterpret_cast<const int4 *>(ra + j)[3];  // lo[0], lo[1], hi[0], hi[1]
             if (bx.x <= row0 + PF_ROWS - 1 && bx.z >= row0 && bx.y <= col0 + PF_COLS - 1 && bx.w >= col0) {
 #pragma unroll
-                for (int w = 0; w < PF_WAVES; w++) {
+                for (int w = 0; w < PF_RECTS; w++) {
                     const int c = col0 + 16 * w;
                     if (bx.y <= c + 15 && bx.w >= c &&
                         support_meets_rect(f1, f2, (xa - f0.y) - f0.w, (xb - f0.y) - f0.w, (cy[2 * w] - f0.z) - f1.x,
@@ -781,39 +812,116 @@ __global__ __launch_bounds__(PF_WAVES * 64) void psf_project_kernel(const PsfRec
                 }
             }
         }
-        wave_lists<PF_WAVES, PF_WAVES>(mask, wl, cnt, wlen);
-        const int len = __builtin_amdgcn_readfirstlane(wlen[wave]);
-        float gA = 0.0f, gB = 0.0f;
-        for (int k = 0; k < len; k++) {
-            const int jj = base + __builtin_amdgcn_readfirstlane((int)wl[wave][k]);
-            smem<PsfRec> *rec = scalar_ptr(ra) + jj;
-            smem<PsfNode2> *nd = scalar_ptr(na) + jj;
-            smem<float> *w = nd->w;
-            float vA, vB;
-            switch (nd->np) {
-            case 3: psf_two_pixels<3>(rec, w, pc, prA, prB, vA, vB); break;
-            case 4: psf_two_pixels<4>(rec, w, pc, prA, prB, vA, vB); break;
-            case 5: psf_two_pixels<5>(rec, w, pc, prA, prB, vA, vB); break;
-            case 6: psf_two_pixels<6>(rec, w, pc, prA, prB, vA, vB); break;
-            default: {
-                float m[1];
-                psf_pixel<2, 1>(ra[jj], prA, pc, m);
-                vA = rec->r.alpha * m[0];
-                psf_pixel<2, 1>(ra[jj], prB, pc, m);
-                vB = rec->r.alpha * m[0];
-            }
-            }
-            gA += vA;
-            gB += vB;
-            if ((k & 3) == 3) {
+        wave_lists<PF_WAVES, PF_RECTS>(mask, wl, cnt, wlen);
+        const int len = __builtin_amdgcn_readfirstlane(wlen[rect]);
+        bool pieces = !regular;  // records that no rule covers whole
+        if (len > 0 && regular) {
+            // lane (u, k): record u of the group, column k and row k % 8; the
+            // record comes as one word per lane (word(k)) and is passed around
+            // its row of 16 lanes, the next group's while this one is used
+            PfTab &T = tab[wave];
+            const unsigned short *lw = wl[rect];
+            const int u16 = lane >> 4;
+            const auto word = [&](int e) {
+                const int jj = base + (int)lw[min(e + u16, len - 1)];
+                const int k = lane & 15;
+                // np, c_hi, c_lo, q, half-widths
+                const float *src = k == 0 ? reinterpret_cast<const float *>(na + jj)
+                                          : reinterpret_cast<const float *>(ra + jj) + (k <= 10 ? k : min(k, 12) + 11);
+                return *src;
+            };
+            float wd = word(4 * grp);
+            for (int e = 4 * grp; e < len; e += 4 * PF_GROUPS) {
+                const float q0 = row_bcast<5>(wd), q1 = row_bcast<6>(wd), q2 = row_bcast<7>(wd);
+                const float h0 = row_bcast<11>(wd), h1 = row_bcast<12>(wd);
+                const float d1 = (pc - row_bcast<2>(wd)) - row_bcast<4>(wd);
+                const float dc = (prc - row_bcast<1>(wd)) - row_bcast<3>(wd);
+                const float row = fmaf(q1, d1, row_bcast<8>(wd)), q4 = row_bcast<9>(wd);
+                const int np = __float_as_int(row_bcast<0>(wd));
+                const float x0 = np == 3 ? (float)psf_node<3>(1)
+                                         : (np == 4 ? (float)psf_node<4>(0)
+                                                    : (np == 5 ? (float)psf_node<5>(1) : (float)psf_node<6>(0)));
+                const float x1 = np == 4 ? (float)psf_node<4>(1)
+                                         : (np == 5 ? (float)psf_node<5>(2) : (float)psf_node<6>(1));
+                const float x2 = (float)psf_node<6>(2);
+                // column factors: the exponents' slopes along the axes at (fifth row, column)
+                const float t0 = fmaf(2.0f * q0, dc, row) * h0, t1 = fmaf(q1, dc, fmaf(2.0f * q2, d1, q4)) * h1;
+                // row factors: lanes 0-7 along axis 0, lanes 8-15 along axis 1
+                const float tr = (lane & 8 ? q1 * h1 : 2.0f * q0 * h0) * (pr8 - prc);
+                wave_sync();
+                const bool two = __any(np >= 4), three = __any(np == 6);
+#pragma unroll
+                for (int i = 0; i < 3; i++) {
+                    if (i == 1 ? !two : (i == 2 && !three)) continue;
+                    const float x = i == 0 ? x0 : (i == 1 ? x1 : x2);
+                    T.cn[u16][i][lane & 15] =
+                        make_float4(__builtin_amdgcn_exp2f(t0 * x), __builtin_amdgcn_exp2f(-t0 * x),
+                                    __builtin_amdgcn_exp2f(t1 * x), __builtin_amdgcn_exp2f(-t1 * x));
+                    reinterpret_cast<float2 *>(&T.rn[u16][i][lane & 7])[(lane >> 3) & 1] =
+                        make_float2(__builtin_amdgcn_exp2f(tr * x), __builtin_amdgcn_exp2f(-tr * x));
+                }
+                T.c[u16][lane & 15] = make_float2(row, fmaf(fmaf(q2, d1, q4), d1, row_bcast<10>(wd)));
+                reinterpret_cast<float *>(&T.r[u16][lane & 3])[(lane >> 2) & 1] =
+                    (pr8 - row_bcast<1>(wd)) - row_bcast<3>(wd);
+                int nps[4], jjs[4];
+                float q0s[4];
+                const uint2 ids = *reinterpret_cast<const uint2 *>(lw + e);  // (entries past the list: not used)
+                const unsigned i0 = __builtin_amdgcn_readfirstlane(ids.x), i1 = __builtin_amdgcn_readfirstlane(ids.y);
+                jjs[0] = i0 & 0xffffu, jjs[1] = i0 >> 16, jjs[2] = i1 & 0xffffu, jjs[3] = i1 >> 16;
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    nps[u] = __builtin_amdgcn_readlane(__float_as_int(wd), 16 * u);
+                    q0s[u] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wd), 16 * u + 5));
+                }
+                wave_sync();
+                wd = word(e + 4 * PF_GROUPS);
+                float gA = 0.0f, gB = 0.0f;
+#pragma unroll 1
+                for (int u = 0; u < 4 && e + u < len; u++) {
+                    const int jj = base + (u < 2 ? (u == 0 ? jjs[0] : jjs[1]) : (u == 2 ? jjs[2] : jjs[3]));
+                    smem<float> *w = scalar_ptr(na + jj)->w;
+                    const int npu = u < 2 ? (u == 0 ? nps[0] : nps[1]) : (u == 2 ? nps[2] : nps[3]);
+                    const float q0u = u < 2 ? (u == 0 ? q0s[0] : q0s[1]) : (u == 2 ? q0s[2] : q0s[3]);
+                    float vA = 0.0f, vB = 0.0f;
+                    switch (npu) {
+                    case 3: psf_two_pixels<3>(T, u, q0u, w, lane, vA, vB); break;
+                    case 4: psf_two_pixels<4>(T, u, q0u, w, lane, vA, vB); break;
+                    case 5: psf_two_pixels<5>(T, u, q0u, w, lane, vA, vB); break;
+                    case 6: psf_two_pixels<6>(T, u, q0u, w, lane, vA, vB); break;
+                    default: pieces = true;
+                    }
+                    gA += vA;
+                    gB += vB;
+                }
                 sA += (double)gA;
                 sB += (double)gB;
-                gA = gB = 0.0f;
             }
         }
-        sA += (double)gA;
-        sB += (double)gB;
+        if (pieces)
+            for (int k = 0; k < len; k++) {
+                if ((k >> 2) % PF_GROUPS != grp) continue;  // (the wave's own fours)
+                const int jj = base + __builtin_amdgcn_readfirstlane((int)wl[rect][k]);
+                if (regular && scalar_ptr(na + jj)->np != 0) continue;
+                const float alpha = scalar_ptr(ra + jj)->r.alpha;
+                float m[1];
+                psf_pixel<2, 1>(ra[jj], prA, pc, m);
+                sA += (double)(alpha * m[0]);
+                psf_pixel<2, 1>(ra[jj], prB, pc, m);
+                sB += (double)(alpha * m[0]);
+            }
         __syncthreads();
+    }
+    // the groups' sums, in group order
+    if (grp > 0) {
+        part[wave - PF_RECTS][0][lane] = sA;
+        part[wave - PF_RECTS][1][lane] = sB;
+    }
+    __syncthreads();
+    if (grp > 0) return;
+#pragma unroll
+    for (int g = 1; g < PF_GROUPS; g++) {
+        sA += part[(g - 1) * PF_RECTS + rect][0][lane];
+        sB += part[(g - 1) * PF_RECTS + rect][1][lane];
     }
     if (i1 < n1) {
         if (rA < n0) R[((size_t)a * n0 + rA) * n1 + i1] = (float)sA;
