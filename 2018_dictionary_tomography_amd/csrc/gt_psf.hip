@@ -1559,10 +1559,10 @@ template <int NP> __device__ inline float psf_voxel_nodes(smem<float> *w, float 
     return s;
 }
 
-// The 3D render with voxel integrals.  Block = brick of 4 x 8 x 8 voxels, four
+// The 3D render with voxel integrals.  Block = brick of 4 x 4 x 8 voxels, two
 // cubes of 4 x 4 x 4 (lane = voxel), PX_GROUPS waves per cube that take every
 // PX_GROUPS-th record of the cube's list; bricks nearest the volume centre
-// first.  A thread tests one record against the four cubes: index box, then
+// first.  A thread tests one record against the cubes: index box, then
 // the plane through the cube's centre across the exponent's gradient g there
 // (the support reaches |v| rho along it, v = U'(yc - x), rho^2 = -kappa; the
 // cube comes as near as |v|^2 - sum |g_c| extent_c).  Records and node tables are
@@ -1570,8 +1570,10 @@ template <int NP> __device__ inline float psf_voxel_nodes(smem<float> *w, float 
 // added to an FP64 total, the groups' totals in group order.  Bound by VALU
 // issue: a voxel costs 7 to 19 exponentials instead of 27 to 216, and the cube
 // test drops what the boxes of slanted ellipsoids keep; 1000 atoms on 64^3:
-// 1.75 -> 0.16 ms.
-constexpr int PX_GROUPS = 4, PX_CUBES = 4, PX_WAVES = PX_GROUPS * PX_CUBES, PX_THREADS = 64 * PX_WAVES;
+// 1.75 -> 0.165 ms with bricks of 4 x 8 x 8 and 16 waves, 0.146 with 8 waves,
+// 0.135 with bricks of 4 x 4 x 8 and 4 or 2 waves per cube (8 per cube: 0.163):
+// smaller blocks leave less to the last ones.
+constexpr int PX_GROUPS = 4, PX_ROW = 1, PX_CUBES = 2 * PX_ROW, PX_WAVES = PX_GROUPS * PX_CUBES, PX_THREADS = 64 * PX_WAVES;
 
 template <int NP>
 __device__ inline float psf_cell_value(smem<float> *w, const float *g, const float *hv, float e)
@@ -1580,22 +1582,22 @@ __device__ inline float psf_cell_value(smem<float> *w, const float *g, const flo
     return e > PSF_CELL_MIN ? __builtin_amdgcn_exp2f(e) * n : 0.0f;
 }
 
-__global__ __launch_bounds__(PX_THREADS) void psf_voxels_kernel(const PsfVolRec *__restrict__ recs,
-                                                                const PsfNode3 *__restrict__ nodes, int N, gt_vol V,
-                                                                float *__restrict__ u, int e0, int e1, int e2)
+__global__ __launch_bounds__(PX_THREADS) __attribute__((amdgpu_waves_per_eu(5))) void psf_voxels_kernel(
+    const PsfVolRec *__restrict__ recs, const PsfNode3 *__restrict__ nodes, int N, gt_vol V, float *__restrict__ u,
+    int e0, int e1, int e2)
 {
     __shared__ alignas(8) unsigned short wl[PX_CUBES][PX_THREADS];
     __shared__ int cnt[PX_CUBES][PX_WAVES];
     __shared__ int wlen[PX_CUBES];
-    static_assert(sizeof(wl) >= PX_THREADS * sizeof(double), "reduction buffer");
+    __shared__ double red[PX_THREADS];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int cube = wave & (PX_CUBES - 1), grp = wave / PX_CUBES;
-    const int nb0 = (V.m0 + 3) / 4, nb1 = (V.m1 + 7) / 8, nb2 = (V.m2 + 7) / 8;
+    const int nb0 = (V.m0 + 3) / 4, nb1 = (V.m1 + 4 * PX_ROW - 1) / (4 * PX_ROW), nb2 = (V.m2 + 7) / 8;
     const int e[3] = {e0, e1, e2};
     int tb[3];
     morton_ranks(blockIdx.x, e, tb);
     if (tb[0] >= nb0 || tb[1] >= nb1 || tb[2] >= nb2) return;  // whole block
-    const int b0 = centre_out(tb[0], nb0) * 4, b1 = centre_out(tb[1], nb1) * 8, b2 = centre_out(tb[2], nb2) * 8;
+    const int b0 = centre_out(tb[0], nb0) * 4, b1 = centre_out(tb[1], nb1) * 4 * PX_ROW, b2 = centre_out(tb[2], nb2) * 8;
     const int i0 = b0 + (lane >> 4), i1 = b1 + 4 * (cube >> 1) + ((lane >> 2) & 3), i2 = b2 + 4 * (cube & 1) + (lane & 3);
     const bool valid = i0 < V.m0 && i1 < V.m1 && i2 < V.m2;
     const float yc[3] = {V.y0[min(i0, V.m0 - 1)], V.y1[min(i1, V.m1 - 1)], V.y2[min(i2, V.m2 - 1)]};
@@ -1608,7 +1610,7 @@ __global__ __launch_bounds__(PX_THREADS) void psf_voxels_kernel(const PsfVolRec 
 #pragma unroll
         for (int c = 0; c < 3; c++)
 #pragma unroll
-            for (int h = 0; h < (c == 0 ? 1 : 2); h++) {
+            for (int h = 0; h < (c == 0 ? 1 : (c == 1 ? PX_ROW : 2)); h++) {
                 const float ya = y[c][min(b[c] + 4 * h, m[c] - 1)], yb = y[c][min(b[c] + 4 * h + 3, m[c] - 1)];
                 cc[c][h] = 0.5f * (ya + yb);
                 ce[c][h] = 0.5f * (yb - ya) + hv[c];
@@ -1620,7 +1622,7 @@ __global__ __launch_bounds__(PX_THREADS) void psf_voxels_kernel(const PsfVolRec 
         const int j = base + (int)threadIdx.x;
         if (j < N) {
             const PsfVolRec r = recs[j];
-            if ((int)(r.lo[0] <= b0 + 3) & (int)(r.hi[0] >= b0) & (int)(r.lo[1] <= b1 + 7) & (int)(r.hi[1] >= b1) &
+            if ((int)(r.lo[0] <= b0 + 3) & (int)(r.hi[0] >= b0) & (int)(r.lo[1] <= b1 + 4 * PX_ROW - 1) & (int)(r.hi[1] >= b1) &
                 (int)(r.lo[2] <= b2 + 7) & (int)(r.hi[2] >= b2)) {
                 const float d0 = (cc[0][0] - r.xh[0]) - r.xl[0];
 #pragma unroll
@@ -1644,6 +1646,7 @@ __global__ __launch_bounds__(PX_THREADS) void psf_voxels_kernel(const PsfVolRec 
         const int len = __builtin_amdgcn_readfirstlane(wlen[cube]);
         float part = 0.0f;
         int n4 = 0;
+        bool pieces = false;  // records that no rule covers whole
         for (int k = grp; k < len; k += PX_GROUPS) {
             const int jj = base + __builtin_amdgcn_readfirstlane((int)wl[cube][k]);
             smem<PsfVolRec> *r = scalar_ptr(recs) + jj;
@@ -1661,7 +1664,7 @@ __global__ __launch_bounds__(PX_THREADS) void psf_voxels_kernel(const PsfVolRec 
             case 4: v = psf_cell_value<4>(w, g, hv, ex); break;
             case 5: v = psf_cell_value<5>(w, g, hv, ex); break;
             case 6: v = psf_cell_value<6>(w, g, hv, ex); break;
-            default: v = psf_voxel<3>(recs[jj], yc, hv);
+            default: v = 0.0f, pieces = true;
             }
             part += v;
             if ((++n4 & 3) == 0) {
@@ -1670,9 +1673,13 @@ __global__ __launch_bounds__(PX_THREADS) void psf_voxels_kernel(const PsfVolRec 
             }
         }
         s += (double)part;
+        if (pieces)
+            for (int k = grp; k < len; k += PX_GROUPS) {
+                const int jj = base + __builtin_amdgcn_readfirstlane((int)wl[cube][k]);
+                if (scalar_ptr(nodes + jj)->np == 0) s += (double)psf_voxel<3>(recs[jj], yc, hv);
+            }
         __syncthreads();
     }
-    double *red = reinterpret_cast<double *>(&wl[0][0]);
     red[threadIdx.x] = s;
     __syncthreads();
     if (grp == 0 && valid) {
@@ -2003,7 +2010,7 @@ extern "C" int gt_psf_volume_rule(const gt_atoms *atoms, const gt_vol *vol, int 
     PsfNode3 *nodes = (PsfNode3 *)((char *)ws + align_up((size_t)atoms->n * sizeof(PsfVolRec)));
     if (whole) {
         hipLaunchKernelGGL(psf_voxel_setup_kernel, dim3((unsigned)atoms->n), dim3(64), 0, st, *atoms, *vol, recs, nodes);
-        nb[0] = (vol->m0 + 3) / 4, nb[1] = (vol->m1 + 7) / 8, nb[2] = (vol->m2 + 7) / 8;
+        nb[0] = (vol->m0 + 3) / 4, nb[1] = (vol->m1 + 4 * PX_ROW - 1) / (4 * PX_ROW), nb[2] = (vol->m2 + 7) / 8;
     } else if (vol->dim == 3) {
         hipLaunchKernelGGL(psf_vol_setup_kernel<3>, sg, dim3(256), 0, st, *atoms, *vol, recs, rule);
         nb[0] = (vol->m0 + 3) / 4, nb[1] = (vol->m1 + 7) / 8, nb[2] = (vol->m2 + 7) / 8;
