@@ -308,12 +308,24 @@ __global__ __launch_bounds__(256) void forward2_kernel(const PairRec *__restrict
     const float kap = (float)KAPPA;
     for (int base = 0; base < N; base += CHUNK) {
         const int total = stage_chunk<4>(ra, base, N, row0, thi, 0, 0, list, wcnt);
-        for (int e = 0; e < total; e++) {
-            const PairRec &q = list[e];
-            if (q.lo[0] > w1 || q.hi[0] < w0) continue;
-            const float dp0 = (pr - q.c_hi[0]) - q.c_lo[0];
-            const float qq = fmaf(fmaf(q.q[0], dp0, q.q[3]), dp0, q.q[5]);
-            if (qq >= kap) kahan_add(s, c, q.alpha * __builtin_amdgcn_exp2f(qq));
+        // four records at a time: their values first, then the compensated sum
+        // takes them in list order (a few waves per CU: one at a time, every
+        // record's LDS reads and exponential were waited for: 51 atoms, 180 angles
+        // 12.0 us, now 10.4)
+        for (int e = 0; e < total; e += 4) {
+            float v[4];
+            bool in[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const PairRec &q = list[min(e + u, total - 1)];
+                const float dp0 = (pr - q.c_hi[0]) - q.c_lo[0];
+                const float qq = fmaf(fmaf(q.q[0], dp0, q.q[3]), dp0, q.q[5]);
+                in[u] = e + u < total && !(q.lo[0] > w1 || q.hi[0] < w0) && qq >= kap;
+                v[u] = q.alpha * __builtin_amdgcn_exp2f(qq);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                if (in[u]) kahan_add(s, c, v[u]);
         }
         __syncthreads();
     }
@@ -467,8 +479,10 @@ __global__ __launch_bounds__(256) void sumsq_kernel(const float *__restrict__ C,
 // With part given, one block more, the first: f from the forward's partial sums.
 // One kernel for both orders, so that the gradient is formed by the same
 // instructions and an order-1 call returns the bits of an order-2 one.
-template <int D, int MODE>
-__global__ __launch_bounds__(64) void finish_kernel(gt_atoms A, gt_geom G, const PairRec *__restrict__ recs,
+// W waves per atom: with more than 64 angles a lane of one wave would contract
+// several pairs one after the other.
+template <int D, int MODE, int W>
+__global__ __launch_bounds__(64 * W) void finish_kernel(gt_atoms A, gt_geom G, const PairRec *__restrict__ recs,
                                                     const float *__restrict__ mom, const double *__restrict__ sumC2,
                                                     int want_hess, double *__restrict__ fo, double *__restrict__ go,
                                                     double *__restrict__ Ho, const double *__restrict__ part,
@@ -479,11 +493,11 @@ __global__ __launch_bounds__(64) void finish_kernel(gt_atoms A, gt_geom G, const
     // row of lane l: [F, grad (P), upper Hessian by rows (NH)]; the lane
     // accumulates its pairs' Hessian entries there directly (a P x P array
     // per lane in registers would spill)
-    __shared__ double red[64][NV + 1];
+    __shared__ double red[64 * W][NV + 1];
     const int j = (int)blockIdx.x - (part ? 1 : 0), lane = threadIdx.x;
     const int N = A.n;
     if (j < 0) {
-        half_sum<64>(part, (nparts + PART_CHUNK - 1) / PART_CHUNK, PART_CHUNK, ftotal, &red[0][0]);
+        half_sum<64 * W>(part, (nparts + PART_CHUNK - 1) / PART_CHUNK, PART_CHUNK, ftotal, &red[0][0]);
         return;
     }
     double grad[P], F = 0.0;
@@ -492,7 +506,7 @@ __global__ __launch_bounds__(64) void finish_kernel(gt_atoms A, gt_geom G, const
     for (int k = 0; k < NV; k++) row[k] = 0.0;
     PairGeom<D> g;
     load_atom<D>(A, j, g);
-    for (int a = lane; a < G.nA; a += 64) {
+    for (int a = lane; a < G.nA; a += 64 * W) {
         const size_t pi = (size_t)a * N + j;
         const PairRec rec = recs[pi];
         const float *m = mom + pi * MOM_STRIDE;
@@ -518,12 +532,21 @@ __global__ __launch_bounds__(64) void finish_kernel(gt_atoms A, gt_geom G, const
     row[0] = F;
     for (int i = 0; i < P; i++) row[1 + i] = grad[i];
     __syncthreads();
-    for (int col = lane; col < NV; col += 64) {
+    // columns added 64 rows per wave, then over the waves
+    const int row0 = lane & ~63;
+    for (int col = lane & 63; col < NV; col += 64) {
         double s = 0.0;
-        for (int i = 0; i < 64; i++) s += red[i][col];
-        red[0][col] = s;  // rows 1..63 of this column are no longer read
+        for (int i = 0; i < 64; i++) s += red[row0 + i][col];
+        red[row0][col] = s;  // the rows after it, of this column, are no longer read
     }
     __syncthreads();
+    if (W > 1) {
+        if (lane >= 64) return;
+        for (int col = lane; col < NV; col += 64)
+#pragma unroll
+            for (int w = 1; w < W; w++) red[0][col] += red[64 * w][col];
+        wave_sync();
+    }
     const double *v = red[0];
     if (!A.iso) {
         // the lanes write the gradient and the full Hessian, one entry each
@@ -674,8 +697,14 @@ static void launch_deriv_kernels(const gt_atoms *A, const gt_geom *G, const Pair
     launch_timed(GT_K_MOMENTS, moments_kernel<K, MODE, ORDER>, dim3((unsigned)((waves + MOM_WAVES - 1) / MOM_WAVES)),
                  dim3(64 * MOM_WAVES), 0, st, recs,
                  A->n, G->nA, G->n0, G->n1, G->p0, G->p1, C, mom, part, nparts);
-    launch_timed(GT_K_FINISH, finish_kernel<D, MODE>, dim3(A->n + (part ? 1 : 0)), dim3(64), 0, st, *A, *G, recs,
-                 mom, sumC2, ORDER == 2 ? 1 : 0, f, g, H, part, nparts, ftotal);
+    // (1D detectors: 180 angles 11.5 us on one wave, 7.2 on four; a 3D atom's
+    // rows fill the LDS of a workgroup with one wave)
+    if (D == 2 && G->nA > 64)
+        launch_timed(GT_K_FINISH, finish_kernel<D, MODE, D == 2 ? 4 : 1>, dim3(A->n + (part ? 1 : 0)), dim3(D == 2 ? 256 : 64), 0,
+                     st, *A, *G, recs, mom, sumC2, ORDER == 2 ? 1 : 0, f, g, H, part, nparts, ftotal);
+    else
+        launch_timed(GT_K_FINISH, finish_kernel<D, MODE, 1>, dim3(A->n + (part ? 1 : 0)), dim3(64), 0, st, *A, *G, recs,
+                     mom, sumC2, ORDER == 2 ? 1 : 0, f, g, H, part, nparts, ftotal);
 }
 
 // part, ftotal (residual mode): the forward's partial sums and where f goes.

@@ -195,7 +195,7 @@ def forward_derivs(atoms, space, data, order=2, out=None, want_f=True):
     if tuple(out.shape) != tuple(geom.shape) or out.dtype != torch.float32 or not out.is_contiguous():
         raise ValueError(f"out must be a contiguous float32 tensor of shape {geom.shape}")
     P = n_params(a.dim, a.iso)
-    f = torch.zeros((), dtype=torch.float64, device=dev) if want_f else None
+    f = torch.empty((), dtype=torch.float64, device=dev) if want_f else None
     g = torch.empty((a.n, P), dtype=torch.float64, device=dev)
     H = torch.empty((a.n, P, P), dtype=torch.float64, device=dev) if order > 1 else None
     need = lib.gt_derivs_workspace(ctypes.byref(a), ctypes.byref(geom.struct), GT_MODE_RESID)
@@ -244,7 +244,7 @@ def forward_derivs_noalloc(atoms, space, data, order=2, out=None, want_f=True):
     if tuple(out.shape) != tuple(geom.shape) or out.dtype != torch.float32 or not out.is_contiguous():
         raise ValueError(f"out must be a contiguous float32 tensor of shape {geom.shape}")
     P = n_params(a.dim, a.iso)
-    f = torch.zeros((), dtype=torch.float64, device=dev) if want_f else None
+    f = torch.empty((), dtype=torch.float64, device=dev) if want_f else None
     g = torch.empty((a.n, P), dtype=torch.float64, device=dev)
     H = torch.empty((a.n, P, P), dtype=torch.float64, device=dev) if order > 1 else None
     check(lib.gt_forward_derivs_noalloc(ctypes.byref(a), ctypes.byref(geom.struct), _ptr(data), order, _ptr(out),

@@ -70,3 +70,20 @@ def test_orders_and_value(gt, cuda, case):
     assert torch.equal(got[0][2], gt.ops.derivs(atoms, space, got[0][0], "resid", order=1)[1])
     resid, f, g, _ = gt.ops.forward_derivs(atoms, space, data, want_f=False)
     assert f is None and torch.equal(g, got[0][2])
+
+
+@pytest.mark.parametrize("det", [(40,), (33, 9)])
+def test_no_atoms(gt, cuda, det):
+    """Without atoms the residual is -data and f its half square, whatever the
+    memory of f held before."""
+    D = 1 + len(det)
+    rng = np.random.default_rng(len(det))
+    axes = tuple(gt.cell_centres(-1, 1, n) for n in det)
+    space = gt.ProjSpace(angles=np.linspace(0, np.pi, 7, endpoint=False), detector=axes)
+    atoms = gt.AtomElement(gt.AtomSpace(D, isotropic=True), np.zeros((0, D)), np.zeros((0, 1)), np.zeros(0), device=cuda)
+    data = torch.as_tensor(rng.normal(size=(7,) + det), dtype=torch.float32, device=cuda)
+    want = 0.5 * float((data.double() ** 2).sum())
+    for call in (gt.ops.forward_derivs, gt.ops.forward_derivs_noalloc):
+        resid, f, g, H = call(atoms, space, data)
+        assert torch.equal(resid, 0.0 - data) and g.shape[0] == 0 and H.shape[0] == 0
+        assert abs(float(f) - want) <= data.numel() * EPS * want
