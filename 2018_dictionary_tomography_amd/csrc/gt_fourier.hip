@@ -119,20 +119,6 @@ __device__ inline float turns(float xh, float xl, float k, float &err)
 // ---------------------------------------------------------------------------
 constexpr int FZ_MAX_ATOMS = 16384;  // more: ft_patch_kernel, without the tables' memory
 
-// Pairing of the m coordinates of one axis under k -> -k, by one block: 0 if
-// k[m-1-i] = -k[i] for every i, 1 if k[m-i] = -k[i] for every i >= 1 (the order of
-// an even-sized FFT's frequencies, whose first one has no partner), else -1.
-__device__ inline int ft_pairing(const float *k, int m)
-{
-    bool p0 = true, p1 = true;
-    for (int i = threadIdx.x; i < m; i += blockDim.x) {
-        p0 = p0 && k[m - 1 - i] == -k[i];
-        p1 = p1 && (i == 0 || k[m - i] == -k[i]);
-    }
-    const int a = __syncthreads_and(p0), b = __syncthreads_and(p1);
-    return a ? 0 : (b ? 1 : -1);
-}
-
 // State of one evaluation: the axes' pairing, the number of listed patches by
 // class of their cell's record count (most first) and the next one to be taken.
 constexpr int FZ_CLASSES = 8;

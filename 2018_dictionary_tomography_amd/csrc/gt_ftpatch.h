@@ -94,4 +94,18 @@ __host__ __device__ inline void kp_row_range(float q0, float q1, float q2, float
     xlo = fmaf(q1, yl, -sqrtf(fmaxf(dl, 0.0f))) * i2 - tol;
 }
 
+// Pairing of the m coordinates of one axis under k -> -k, by one block: 0 if
+// k[m-1-i] = -k[i] for every i, 1 if k[m-i] = -k[i] for every i >= 1 (the order of
+// an even-sized FFT's frequencies, whose first one has no partner), else -1.
+__device__ inline int ft_pairing(const float *k, int m)
+{
+    bool p0 = true, p1 = true;
+    for (int i = threadIdx.x; i < m; i += blockDim.x) {
+        p0 = p0 && k[m - 1 - i] == -k[i];
+        p1 = p1 && (i == 0 || k[m - i] == -k[i]);
+    }
+    const int a = __syncthreads_and(p0), b = __syncthreads_and(p1);
+    return a ? 0 : (b ? 1 : -1);
+}
+
 }  // namespace gt

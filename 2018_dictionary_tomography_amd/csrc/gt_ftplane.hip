@@ -169,9 +169,22 @@ __device__ inline void kp_pair(int D, int iso, double I, const AR *x, const AR *
     }
 }
 
+// pairing, if given (FP32, two sample axes): of the samples under k -> -k, see
+// kp_rect_kernel; {-1, -1} where it does not pair both axes.
 template <typename R>
-__global__ __launch_bounds__(256) void kp_setup_kernel(gt_atoms_t<R> A, KpDev<R> P, double cut, KpRec<R> *recs)
+__global__ __launch_bounds__(256) void kp_setup_kernel(gt_atoms_t<R> A, KpDev<R> P, double cut, KpRec<R> *recs,
+                                                       int *pairing)
 {
+    if constexpr (sizeof(R) == 4) {
+        if (pairing && blockIdx.x == 0) {
+            const int s0 = ft_pairing(P.k0, P.m0), s1 = ft_pairing(P.k1, P.m1);
+            if (threadIdx.x == 0) {
+                const bool both = s0 >= 0 && s1 >= 0 && P.sorted;
+                pairing[0] = both ? s0 : -1;
+                pairing[1] = both ? s1 : -1;
+            }
+        }
+    }
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= (long)A.n * P.nA) return;
     const int a = (int)(t / A.n), j = (int)(t - (long)a * A.n);
@@ -291,15 +304,18 @@ __global__ __launch_bounds__(256) void kp_eval_kernel(const KpRec<R> *__restrict
 // the sine and cosine of one column or row (handed round through LDS), and a
 // sample costs one complex product instead of two phase reductions, a sine and
 // a cosine.  KE_GROUP records' values are summed in FP32 and added to the FP64
-// total.  Bound by VALU issue: 2000 atoms, 61 x 128^2 samples: 0.97 -> 0.35 ms;
-// without the row pairs 0.38.
+// total.  The planes pass through k = 0 and out(-k) = conj(out(k)): on ascending
+// axes that pair k with -k (0: m-1-i, 1: m-i and none for i = 0, an even FFT's)
+// the rectangles of k0 < 0 whose samples all have a partner are written with it.
+// Bound by VALU issue: 2000 atoms, 61 x 128^2 samples: 0.97 -> 0.35 ms, 0.235 with
+// the partners; without the row pairs 0.38.
 static_assert(sizeof(KpRec<float>) == 48, "KpRec<float>: amp, q[3] | ch[2], cl[2] | lo[2], hi[2]");
 constexpr int KE_WAVES = 8, KE_ROWS = 16, KE_COLS = 32, KE_R = KE_ROWS / 2;
 constexpr int KE_GROUP = 8;
 
-__global__ __launch_bounds__(64 * KE_WAVES) void kp_rect_kernel(const KpRec<float> *__restrict__ recs, int N,
-                                                                KpDev<float> P, float cutlog, float2 *__restrict__ out,
-                                                                int e0, int e1)
+__global__ __launch_bounds__(64 * KE_WAVES) void kp_rect_kernel(const KpRec<float> *__restrict__ recs,
+                                                                const int *__restrict__ pairing, int N, KpDev<float> P,
+                                                                float cutlog, float2 *__restrict__ out, int e0, int e1)
 {
     __shared__ unsigned short wl[1][64 * KE_WAVES];
     __shared__ int cnt[1][KE_WAVES];
@@ -316,12 +332,18 @@ __global__ __launch_bounds__(64 * KE_WAVES) void kp_rect_kernel(const KpRec<floa
     if (t[0] >= tilesR || t[1] >= tilesC) return;  // whole block: no tile of this rank
     const int row0 = centre_out(t[0], tilesR) * KE_ROWS, col0 = centre_out(t[1], tilesC) * KE_COLS;
     const int row1 = min(row0 + KE_ROWS - 1, P.m0 - 1), col1 = min(col0 + KE_COLS - 1, P.m1 - 1);
+    // rectangle (r, c) is written with its partners
+    const int s0 = pairing[0], s1 = pairing[1];
+    const auto mirrored = [&](int r, int c) {
+        return s0 >= 0 && r >= s0 && c >= s1 && P.k0[min(r + KE_ROWS - 1, P.m0 - 1)] < 0.0f;
+    };
+    if (mirrored(row0, col0)) return;  // whole block
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int half = lane >> 5, i1 = col0 + (lane & 31), r0 = row0 + half;
     const float p1 = P.k1[min(i1, P.m1 - 1)], p1sq = p1 * p1;
     // the coordinate whose phase this lane forms, and the axis it belongs to
     // (lanes 32 .. 47: the rows of half 0, then those of half 1)
-    const float pph = half ? P.k0[min(row0 + 2 * (lane & (KE_R - 1)) + ((lane >> 3) & 1), P.m0 - 1)] : p1;
+    const float pph = half ? P.k0[min(row0 + 2 * (lane & (KE_R - 1)) + ((lane / KE_R) & 1), P.m0 - 1)] : p1;
     const float ax0 = half ? 1.0f : 0.0f, ax1 = half ? 0.0f : 1.0f;
     float p0[KE_R];
 #pragma unroll
@@ -452,9 +474,16 @@ __global__ __launch_bounds__(64 * KE_WAVES) void kp_rect_kernel(const KpRec<floa
     }
     if (wave != 0 || i1 >= P.m1) return;
 #pragma unroll
-    for (int r = 0; r < KE_R; r++)
-        if (r0 + 2 * r < P.m0)
-            out[((size_t)a * P.m0 + r0 + 2 * r) * P.m1 + i1] = make_float2((float)sr[r], (float)si[r]);
+    for (int r = 0; r < KE_R; r++) {
+        const int i = r0 + 2 * r;
+        if (i >= P.m0) continue;
+        const float re = (float)sr[r], im = (float)si[r];
+        out[((size_t)a * P.m0 + i) * P.m1 + i1] = make_float2(re, im);
+        if (i < s0 || i1 < s1 || s0 < 0) continue;
+        const int ip = P.m0 - 1 + s0 - i, jp = P.m1 - 1 + s1 - i1;  // the partner
+        if (mirrored(ip / KE_ROWS * KE_ROWS, jp / KE_COLS * KE_COLS))
+            out[((size_t)a * P.m0 + ip) * P.m1 + jp] = make_float2(re, -im);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -828,6 +857,13 @@ template <typename R, typename KP> KpDev<R> kp_dev(const KP *P)
     return d;
 }
 
+// Workspace: the records and, for FP32, the samples' pairing.
+template <typename R, typename KP> size_t kp_bytes(int n, const KP *planes)
+{
+    if (n == 0) return 0;
+    return align_up((size_t)n * planes->nA * sizeof(KpRec<R>)) + (sizeof(R) == 4 ? ALIGN : 0);
+}
+
 template <typename R, typename AT, typename KP>
 int kp_eval(const AT *atoms, const KP *planes, R *out, void *ws, size_t ws_bytes, void *stream, const char *who)
 {
@@ -838,7 +874,7 @@ int kp_eval(const AT *atoms, const KP *planes, R *out, void *ws, size_t ws_bytes
     GT_CHECK_ARG(atoms->n == 0 || (atoms->I && atoms->x && atoms->r), "%s: atom arrays missing", who);
     if ((rc = kp_check<R>(planes, atoms->dim, who))) return rc;
     GT_CHECK_ARG(out != nullptr, "%s: out is NULL", who);
-    const size_t need = align_up((size_t)atoms->n * planes->nA * sizeof(KpRec<R>));
+    const size_t rec_bytes = align_up((size_t)atoms->n * planes->nA * sizeof(KpRec<R>)), need = kp_bytes<R>(atoms->n, planes);
     if (need > ws_bytes || (need > 0 && ws == nullptr)) {
         set_error("%s: workspace of %zu bytes given, %zu needed", who, ws_bytes, need);
         return GT_EWORKSPACE;
@@ -858,7 +894,9 @@ int kp_eval(const AT *atoms, const KP *planes, R *out, void *ws, size_t ws_bytes
     const long npair = (long)atoms->n * planes->nA;
     GT_CHECK_ARG(npair < (1L << 31) * 256L, "%s: too many (atom, angle) pairs", who);
     gt_atoms_t<R> A{atoms->dim, atoms->n, atoms->iso, atoms->I, atoms->x, atoms->r};
-    hipLaunchKernelGGL(kp_setup_kernel<R>, dim3((unsigned)((npair + 255) / 256)), dim3(256), 0, st, A, P, cut, recs);
+    int *pairing = sizeof(R) == 4 && planes->form != GT_KP_2D_LINE ? (int *)((char *)ws + rec_bytes) : nullptr;
+    hipLaunchKernelGGL(kp_setup_kernel<R>, dim3((unsigned)((npair + 255) / 256)), dim3(256), 0, st, A, P, cut, recs,
+                       pairing);
     const long tiles = ((long)planes->m0 * planes->m1 + 255) / 256;
     const long blocks = tiles * planes->nA;
     GT_CHECK_ARG(blocks < (1L << 31), "%s: too many samples", who);
@@ -872,8 +910,9 @@ int kp_eval(const AT *atoms, const KP *planes, R *out, void *ws, size_t ws_bytes
             const int e1 = ceil_log2((planes->m1 + KE_COLS - 1) / KE_COLS);
             const unsigned long long rects = (unsigned long long)planes->nA << (e0 + e1);
             if (rects < (1ull << 31)) {
-                hipLaunchKernelGGL(kp_rect_kernel, dim3((unsigned)rects), dim3(64 * KE_WAVES), 0, st, recs, atoms->n, P,
-                                   (float)(-0.5 * KP_LOG2E * cut), (float2 *)out, e0, e1);
+                hipLaunchKernelGGL(kp_rect_kernel, dim3((unsigned)rects), dim3(64 * KE_WAVES), 0, st, recs, pairing,
+                                   atoms->n, P, (float)(-0.5 * KP_LOG2E * cut),
+                                   (float2 *)out, e0, e1);
                 prof_end(st, GT_K_FT);
                 GT_HIP(hipGetLastError());
                 return 0;
@@ -893,7 +932,7 @@ using namespace gt;
 extern "C" size_t gt_ft_planes_workspace(int n_atoms, const gt_kplanes *planes)
 {
     if (!planes || n_atoms < 0) return 0;
-    return align_up((size_t)n_atoms * planes->nA * sizeof(KpRec<float>));
+    return kp_bytes<float>(n_atoms, planes);
 }
 
 extern "C" int gt_ft_planes_eval(const gt_atoms *atoms, const gt_kplanes *planes, float *out, void *ws, size_t ws_bytes,
@@ -905,7 +944,7 @@ extern "C" int gt_ft_planes_eval(const gt_atoms *atoms, const gt_kplanes *planes
 extern "C" size_t gt_ft_planes_workspace_f64(int n_atoms, const gt_kplanes64 *planes)
 {
     if (!planes || n_atoms < 0) return 0;
-    return align_up((size_t)n_atoms * planes->nA * sizeof(KpRec<double>));
+    return kp_bytes<double>(n_atoms, planes);
 }
 
 extern "C" int gt_ft_planes_eval_f64(const gt_atoms64 *atoms, const gt_kplanes64 *planes, double *out, void *ws,
