@@ -107,8 +107,11 @@ def work_per_update(spec):
 
 
 # Fixed cost of one atom update advanced by a group (setup, contraction,
-# barriers, the solve repeated in every member), pixel units.
-GROUP_UPDATE_OVERHEAD = 4.1e5
+# barriers, the solve repeated in every member), pixel units: 43 us at 162 us
+# per 10^6 pixels and workgroup, least squares over 24 to 120 angles of 48^2 to
+# 256^2 at 4 workgroups to one per angle.  (4.1e5 gave launches of 60% of the
+# time that the quotas are meant for: a burst of short fits took a second one.)
+GROUP_UPDATE_OVERHEAD = 2.65e5
 
 
 def update_cost(spec, group):
