@@ -129,8 +129,9 @@ def steady_leg(torch, args, dev, launches=4, budget=100):
     `budget` updates per fit after one warm-up launch of 10.  Reports atom
     updates/s and, for the first fit of each (detector side, more than 75
     angles) class, the fit kernel's wall-clock ticks (100 MHz) per phase and
-    update: setup, moments + per-angle contraction, angle sums, solve,
-    proposal set-up, energy pass, decision, commit."""
+    update: setup (the hand-over of the records: the set-up itself runs
+    beside the commit and counts there), moments + per-angle contraction,
+    angle sums, solve, proposal set-up, energy pass, decision, commit."""
     Sv = importlib.import_module("2018_dictionary_tomography_amd.serving")
     F = importlib.import_module("2018_dictionary_tomography_amd.fit")
     specs = Sv.c5_stream(2000, rate=200.0, seed=2024, n_range=(50, 5000))
