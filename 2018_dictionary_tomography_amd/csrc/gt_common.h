@@ -108,6 +108,17 @@ __device__ inline float buffer_load_f32(__amdgpu_buffer_rsrc_t r, unsigned voff,
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
 }
 
+// A pointer that is the same in every lane, held in scalar registers whatever
+// the compiler knows of where it came from: a buffer resource made from one it
+// holds per lane costs every load a loop over the lanes' distinct bases.
+template <typename T> __device__ inline T *uniform_ptr(T *p)
+{
+    const unsigned long long v = (unsigned long long)(uintptr_t)p;
+    const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)v);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(v >> 32));
+    return (T *)(uintptr_t)(((unsigned long long)hi << 32) | lo);
+}
+
 // Read-only array of an earlier kernel, read at wave-uniform indices through
 // the scalar cache: the values land in scalar registers, which cost no LDS
 // bandwidth and no vector registers (a wave-uniform index is made with

@@ -37,10 +37,11 @@
 // The members meet at two device-wide barriers per atom update (after the
 // per-angle contractions and after the per-angle energy changes); a barrier
 // wait is bounded in time.  An update is one latency chain: 300 atoms, 61 x
-// 96^2, 63 us at G = 4 (14 moments and contraction, 14 meeting and sums over
-// angles, 7 solve, 3 + 14 the proposal's setup and energy, 2 accept, 9 commit
-// beside the next atom's setup); 66 us with that setup after the commit, 69 us
-// with a barrier word that the last arrival resets and
+// 96^2, 61 us at G = 4 (13 moments and contraction, 13 meeting and sums over
+// angles, 7 solve, 3 + 15 the proposal's setup and energy, 2 accept, 9 commit
+// beside the next atom's setup).  What it took on the way there: 63 us with the
+// moments' residual base in vector registers, 66 us with that setup after the
+// commit, 69 us with a barrier word that the last arrival resets and
 // releases, per-angle records read a line per lane, and the atom, its step
 // size and its place in the order read one after the other.  The solve and the accept logic run redundantly in
 // every member; member 0 writes the progress fields back at the end.

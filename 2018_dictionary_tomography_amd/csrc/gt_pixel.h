@@ -512,6 +512,11 @@ __device__ inline void pair_moments_rows(const PairRec &rec, const float *p0, co
 // expressions of row_table).  For a wave that walks many small boxes whose
 // residual rows sit in HBM (the fitter's one atom at a time over every
 // angle), the span set-up costs more than the corners it skips.
+// The base and the row step are the same in every lane but reach the walk
+// through memory, so they are put into scalar registers here: with the base
+// per lane each load was a loop over distinct bases, 343 instructions per 8
+// rows instead of 174 (256 fits of the serving stream on a workgroup each:
+// 195e3 atom updates/s before, 216e3 after).
 template <int MODE, int UNR, int TROWS, int BOXW = 64>
 __device__ inline void pair_moments_box(const PairRec &rec, const float *p0, const float *p1,
                                         const gmem<float> *__restrict__ Ca, int n1, int lane, float *acc,
@@ -520,7 +525,7 @@ __device__ inline void pair_moments_box(const PairRec &rec, const float *p0, con
     const int W = rec.hi[1] - rec.lo[1] + 1;
     const int Hbox = rec.hi[0] - rec.lo[0] + 1;
     if (W <= 0 || Hbox <= 0) return;
-    const __amdgpu_buffer_rsrc_t crs = buffer_rsrc((const float *)Ca);
+    const __amdgpu_buffer_rsrc_t crs = buffer_rsrc(uniform_ptr((const float *)Ca));
     const unsigned rowb = 4u * (unsigned)n1;
     for (int w0 = 0; w0 < Hbox; w0 += TROWS) {
         const int H = min(TROWS, Hbox - w0);
@@ -541,12 +546,12 @@ __device__ inline void pair_moments_box(const PairRec &rec, const float *p0, con
             const float rowlin = fmaf(rec.q[1], dp1, rec.q[3]);
             const float colt = fmaf(fmaf(rec.q[2], dp1, rec.q[4]), dp1, rec.q[5]);
             float A[5] = {0, 0, 0, 0, 0}, B[5] = {0, 0, 0, 0, 0};
-            const int r0 = cc.ro;
+            const int r0 = cc.ro, step = __builtin_amdgcn_readfirstlane(cc.R);
             const unsigned off = 4u * ((unsigned)(row0 + r0) * (unsigned)n1 + (unsigned)i1);
-            if (cc.R == 2)
+            if (step == 2)
                 moment_rows<MODE, UNR, 2, 4>(rec, crs, off, rowb, tab + r0, 2, r0, H - 1, rowlin, colt, A, B, acc);
             else
-                moment_rows<MODE, UNR, 0, 4>(rec, crs, off, rowb, tab + r0, cc.R, r0, H - 1, rowlin, colt, A, B, acc);
+                moment_rows<MODE, UNR, 0, 4>(rec, crs, off, rowb, tab + r0, step, r0, H - 1, rowlin, colt, A, B, acc);
             const float y2 = dp1 * dp1;
             const float yp[5] = {1.0f, dp1, y2, y2 * dp1, y2 * y2};
 #pragma unroll
