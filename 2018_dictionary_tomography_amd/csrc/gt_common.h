@@ -108,6 +108,11 @@ __device__ inline float buffer_load_f32(__amdgpu_buffer_rsrc_t r, unsigned voff,
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
 }
 
+__device__ inline void buffer_store_f32(__amdgpu_buffer_rsrc_t r, float v, unsigned voff, unsigned soff)
+{
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, voff, soff, 0);
+}
+
 // A pointer that is the same in every lane, held in scalar registers whatever
 // the compiler knows of where it came from: a buffer resource made from one it
 // holds per lane costs every load a loop over the lanes' distinct bases.

@@ -37,10 +37,11 @@
 // The members meet at two device-wide barriers per atom update (after the
 // per-angle contractions and after the per-angle energy changes); a barrier
 // wait is bounded in time.  An update is one latency chain: 300 atoms, 61 x
-// 96^2, 61 us at G = 4 (13 moments and contraction, 13 meeting and sums over
-// angles, 7 solve, 3 + 15 the proposal's setup and energy, 2 accept, 9 commit
-// beside the next atom's setup).  What it took on the way there: 63 us with the
-// moments' residual base in vector registers, 66 us with that setup after the
+// 96^2, 58 us at G = 4 (13 moments and contraction, 12 meeting and sums over
+// angles, 7 solve, 3 + 12 the proposal's setup and energy, 2 accept, 8 commit
+// beside the next atom's setup).  What it took on the way there: 61 us with an
+// address per pixel in the energy and commit walks, 63 us with the moments'
+// residual base in vector registers, 66 us with that setup after the
 // commit, 69 us with a barrier word that the last arrival resets and
 // releases, per-angle records read a line per lane, and the atom, its step
 // size and its place in the order read one after the other.  The solve and the accept logic run redundantly in
@@ -220,6 +221,61 @@ __device__ inline float pair_value(const PairRec &rec, float p0v, float p1v)
     return (q >= (float)KAPPA) ? rec.alpha * __builtin_amdgcn_exp2f(q) : 0.0f;
 }
 
+// What the pixels of one lane's column share: the row coefficients and heights
+// of the old and the new Gaussian and their terms of the column (a copy, so
+// that no store is followed by another read of the records).
+struct DeltaCol {
+    float qo, qn, ao, an, lo, ln, co, cn;
+};
+
+// FIT_UNR rows of a lane's column in pair_delta4, rows at uniform distances
+// (rstep bytes, step table entries).  Whole groups address their loads and
+// stores by the scalar offsets of the rows; in the last group of a column (FULL
+// false) the places past the window, left rows from the group's first one,
+// read that first row again and change nothing.  Bound by VALU issue: 31
+// instructions a pixel, 7 of them FP64 sums or exponentials; 39 with an
+// address and a bound for each pixel (300 atoms, 61 x 96^2 on one workgroup:
+// energy 43 -> 35 us, commit 23 -> 20 us of an update; 256 fits of the serving
+// stream at once: 216e3 -> 238e3 updates/s).
+template <int mode, bool FULL>
+__device__ inline double delta_group(const DeltaCol c, __amdgpu_buffer_rsrc_t rr, __amdgpu_buffer_rsrc_t sr,
+                                     unsigned off, unsigned rstep, const float2 *drow, int step, int left, double acc)
+{
+    const float kap = (float)KAPPA;
+    float old[FIT_UNR];
+    float2 d0[FIT_UNR];
+#pragma unroll
+    for (int u = 0; u < FIT_UNR; u++) {
+        if (FULL) {
+            old[u] = buffer_load_f32(rr, off, (unsigned)u * rstep);
+            d0[u] = drow[u * step];
+        } else {
+            const bool ok = u * step < left;
+            old[u] = buffer_load_f32(rr, off + (ok ? (unsigned)u * rstep : 0u), 0u);
+            d0[u] = drow[ok ? u * step : 0];
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < FIT_UNR; u++) {
+        const bool ok = FULL || u * step < left;
+        const float qo = fmaf(fmaf(c.qo, d0[u].x, c.lo), d0[u].x, c.co);
+        const float qn = fmaf(fmaf(c.qn, d0[u].y, c.ln), d0[u].y, c.cn);
+        const float vo = (qo >= kap) ? c.ao * __builtin_amdgcn_exp2f(qo) : 0.0f;
+        const float vn = (qn >= kap) ? c.an * __builtin_amdgcn_exp2f(qn) : 0.0f;
+        float dR = ok ? vn - vo : 0.0f;
+        // both needed here in any case: the load stays with the others, and is
+        // waited for when its pixel's turn comes
+        asm volatile("" : "+v"(old[u]), "+v"(dR));
+        const bool chg = dR != 0.0f;
+        if (mode == 2 && ok) buffer_store_f32(sr, old[u], off, (unsigned)u * rstep);
+        // an unchanged pixel adds exactly 0, whatever its residual holds
+        const float od = chg ? old[u] : 0.0f, nw = od + dR;
+        if (mode != 0 && chg) buffer_store_f32(rr, nw, off, (unsigned)u * rstep);
+        if (mode != 1) acc += ((double)nw - (double)od) * ((double)nw + (double)od);
+    }
+    return acc;
+}
+
 // Replacing rec_old by rec_new over the union box, both values evaluated per
 // pixel with the same FP32 expressions in every mode; returns the lane's FP64
 // energy-change partial (modes 0 and 2): the sum of (new - old)(new + old),
@@ -248,8 +304,10 @@ __device__ inline double pair_delta4(const PairRec &ro, const PairRec &rn, const
     if (total == 0) return acc;
     if (K == 2) {
         // column-owning walk (ColChunk): per-column terms of both Gaussians once
-        // per lane; 32-bit element offsets within the angle's slab
-        const float kap = (float)KAPPA;
+        // per lane; 32-bit byte offsets within the angle's slab
+        const __amdgpu_buffer_rsrc_t rr = buffer_rsrc(uniform_ptr((const float *)Ra));
+        const __amdgpu_buffer_rsrc_t sr = buffer_rsrc(uniform_ptr((const float *)Sa));
+        const unsigned rowb = 4u * (unsigned)n1;
         for (int w0 = 0; w0 < H; w0 += FIT_TROWS) {
             const int Hw = min(FIT_TROWS, H - w0);
             if (w0 > 0) wave_sync();  // the previous window's table is no longer read
@@ -268,37 +326,18 @@ __device__ inline double pair_delta4(const PairRec &ro, const PairRec &rn, const
                 const float rlo = fmaf(ro.q[1], d1o, ro.q[3]), rln = fmaf(rn.q[1], d1n, rn.q[3]);
                 const float clo = fmaf(fmaf(ro.q[2], d1o, ro.q[4]), d1o, ro.q[5]);
                 const float cln = fmaf(fmaf(rn.q[2], d1n, rn.q[4]), d1n, rn.q[5]);
-                const unsigned off0 = (unsigned)(lo[0] + w0) * (unsigned)n1 + (unsigned)i1;
-                for (int r0 = cc.ro; r0 < Hw; r0 += FIT_UNR * cc.R) {
-                    float old[FIT_UNR];
-                    float2 d0[FIT_UNR];
-                    bool ok[FIT_UNR];
-                    unsigned off[FIT_UNR];
-#pragma unroll
-                    for (int u = 0; u < FIT_UNR; u++) {
-                        const int r = r0 + u * cc.R;
-                        ok[u] = r < Hw;
-                        const unsigned rr = ok[u] ? (unsigned)r : 0u;
-                        off[u] = off0 + rr * (unsigned)n1;
-                        old[u] = Ra[off[u]];
-                        d0[u] = dt[rr];
-                    }
-#pragma unroll
-                    for (int u = 0; u < FIT_UNR; u++) {
-                        const float d0o = d0[u].x, d0n = d0[u].y;
-                        const float qo = fmaf(fmaf(ro.q[0], d0o, rlo), d0o, clo);
-                        const float qn = fmaf(fmaf(rn.q[0], d0n, rln), d0n, cln);
-                        const float vo = (qo >= kap) ? ro.alpha * __builtin_amdgcn_exp2f(qo) : 0.0f;
-                        const float vn = (qn >= kap) ? rn.alpha * __builtin_amdgcn_exp2f(qn) : 0.0f;
-                        const float dR = vn - vo;
-                        if (mode == 2 && ok[u]) Sa[off[u]] = old[u];
-                        if (ok[u] && dR != 0.0f) {
-                            const float nw = old[u] + dR;
-                            if (mode != 0) Ra[off[u]] = nw;
-                            if (mode != 1) acc += ((double)nw - (double)old[u]) * ((double)nw + (double)old[u]);
-                        }
-                    }
+                const DeltaCol c = {ro.q[0], rn.q[0], ro.alpha, rn.alpha, rlo, rln, clo, cln};
+                const int step = __builtin_amdgcn_readfirstlane(cc.R);
+                unsigned off = 4u * ((unsigned)(lo[0] + w0 + cc.ro) * (unsigned)n1 + (unsigned)i1);
+                const float2 *drow = dt + cc.ro;
+                int left = Hw - cc.ro;  // rows from this lane's next one to the window's end
+                for (; left > (FIT_UNR - 1) * step; left -= FIT_UNR * step) {
+                    acc = delta_group<mode, true>(c, rr, sr, off, rowb * (unsigned)step, drow, step, left, acc);
+                    off += FIT_UNR * rowb * (unsigned)step;
+                    drow += FIT_UNR * step;
                 }
+                if (left > 0)
+                    acc = delta_group<mode, false>(c, rr, sr, off, rowb * (unsigned)step, drow, step, left, acc);
             }
         }
         wave_sync();  // the table is rewritten for the wave's next pair
