@@ -107,10 +107,12 @@ def work_per_update(spec):
 
 
 # Fixed cost of one atom update advanced by a group (setup, contraction,
-# barriers, the solve repeated in every member), pixel units: 43 us at 162 us
-# per 10^6 pixels and workgroup, least squares over 24 to 120 angles of 48^2 to
-# 256^2 at 4 workgroups to one per angle.  (4.1e5 gave launches of 60% of the
-# time that the quotas are meant for: a burst of short fits took a second one.)
+# barriers, the solve repeated in every member), pixel units: 41 us, counted at
+# 155 us per 10^6 pixels and workgroup, the rate that the launch quotas are set
+# for.  Least squares over 24 to 120 angles of 48^2 to 256^2 at 4 workgroups to
+# one per angle; the pixels themselves now take 122 us per 10^6.  (4.1e5 gave
+# launches of 60% of the time that the quotas are meant for: a burst of short
+# fits took a second one.)
 GROUP_UPDATE_OVERHEAD = 2.65e5
 
 
