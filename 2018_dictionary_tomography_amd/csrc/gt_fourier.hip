@@ -391,9 +391,11 @@ __global__ __launch_bounds__(FZ_THREADS) void ft_grid_kernel(const FtRec *__rest
                 for (int z = 0; z < FZ_K0; z++) {
                     const float w0 = f.u[0] * k0[z], w1 = fmaf(f.u[3], k0[z], v1), w2 = fmaf(f.u[5], k0[z], v2);
                     const float nq = fmaf(w0, w0, fmaf(w1, w1, w2 * w2));
-                    const float E = nq < cut ? __builtin_amdgcn_exp2f(-nq) : 0.0f;
-                    gr[z] = fmaf(E, fmaf(f.a[z].x, pr, -f.a[z].y * pi), gr[z]);
-                    gi[z] = fmaf(E, fmaf(f.a[z].x, pi, f.a[z].y * pr), gi[z]);
+                    const float E = __builtin_amdgcn_exp2f(-nq);
+                    // the terms are chosen, not E: 0 times an infinite amplitude is no 0
+                    const float re = E * fmaf(f.a[z].x, pr, -f.a[z].y * pi), im = E * fmaf(f.a[z].x, pi, f.a[z].y * pr);
+                    gr[z] += nq < cut ? re : 0.0f;
+                    gi[z] += nq < cut ? im : 0.0f;
                 }
                 if ((++n & 3) == 0)
 #pragma unroll

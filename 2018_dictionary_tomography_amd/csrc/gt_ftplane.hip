@@ -433,9 +433,11 @@ __global__ __launch_bounds__(64 * KE_WAVES) void kp_rect_kernel(const KpRec<floa
                 if ((m >> r) & 1u) {
                     const float rc = (r & 1) ? v[r / 2].z : v[r / 2].x, rs = (r & 1) ? v[r / 2].w : v[r / 2].y;
                     const float ex = fmaf(fmaf(q0, p0[r], b), p0[r], c);
-                    const float E = ex > cutlog ? __builtin_amdgcn_exp2f(ex) : 0.0f;
-                    gr[r] = fmaf(E, fmaf(rc, cc, -rs * cn), gr[r]);
-                    gi[r] = fmaf(-E, fmaf(rc, cn, rs * cc), gi[r]);
+                    const float E = __builtin_amdgcn_exp2f(ex);
+                    // the terms are chosen, not E: 0 times an infinite amplitude is no 0
+                    const float re = E * fmaf(rc, cc, -rs * cn), im = E * fmaf(rc, cn, rs * cc);
+                    gr[r] += ex > cutlog ? re : 0.0f;
+                    gi[r] -= ex > cutlog ? im : 0.0f;
                 }
             if ((n & (KE_GROUP - 1)) == KE_GROUP - 1) {
 #pragma unroll

@@ -307,6 +307,12 @@ __device__ inline void psf_node_record(const PsfRec &R, PsfNode2 &T)
     case 6: psf_node_table<6>(R.r, R.s, T); break;
     default: break;
     }
+    // an amplitude that is not finite (or whose weights are not) stays within
+    // its support's box: psf_pixel
+    float t = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 18; k++) t = fmaf(0.0f, T.w[k], t);
+    if (!(t == 0.0f)) T.np = 0;
 }
 
 // half width of the cells of an ascending coordinate vector, from its first
@@ -902,12 +908,18 @@ __global__ __launch_bounds__(PF_WAVES * 64) __attribute__((amdgpu_waves_per_eu(5
                 if ((k >> 2) % PF_GROUPS != grp) continue;  // (the wave's own fours)
                 const int jj = base + __builtin_amdgcn_readfirstlane((int)wl[rect][k]);
                 if (regular && scalar_ptr(na + jj)->np != 0) continue;
-                const float alpha = scalar_ptr(ra + jj)->r.alpha;
+                smem<PairRec> *r = &scalar_ptr(ra + jj)->r;
+                if (i1 < r->lo[1] || i1 > r->hi[1]) continue;
+                const float alpha = r->alpha;
                 float m[1];
-                psf_pixel<2, 1>(ra[jj], prA, pc, m);
-                sA += (double)(alpha * m[0]);
-                psf_pixel<2, 1>(ra[jj], prB, pc, m);
-                sB += (double)(alpha * m[0]);
+                if (rA >= r->lo[0] && rA <= r->hi[0]) {
+                    psf_pixel<2, 1>(ra[jj], prA, pc, m);
+                    sA += (double)(alpha * m[0]);
+                }
+                if (rB >= r->lo[0] && rB <= r->hi[0]) {
+                    psf_pixel<2, 1>(ra[jj], prB, pc, m);
+                    sB += (double)(alpha * m[0]);
+                }
             }
         __syncthreads();
     }
@@ -1439,12 +1451,13 @@ struct alignas(16) PsfNode3 {
 static_assert(sizeof(PsfNode3) == 448, "PsfNode3 must stay 448 bytes");
 
 // Entry idx (m0, m1, m2) of the table: the weights of the node and of its
-// reflections in the second, third and first axis, combined.
+// reflections in the second, third and first axis, combined.  False if it is
+// not finite.
 template <int NP>
-__device__ inline void psf_node_entry(const PsfVolRec &R, const float *hv, int idx, float *w)
+__device__ inline bool psf_node_entry(const PsfVolRec &R, const float *hv, int idx, float *w)
 {
     constexpr int M = PsfNodes<NP>::M;
-    if (idx >= M * M * M) return;
+    if (idx >= M * M * M) return true;
     const int mi[3] = {idx / (M * M), (idx / M) % M, idx % M};
     double d[3], f = (double)R.amp;
 #pragma unroll
@@ -1467,10 +1480,11 @@ __device__ inline void psf_node_entry(const PsfVolRec &R, const float *hv, int i
         const double a0 = R.u[0] * d0 + R.u[3] * d1 + R.u[5] * d2, a1 = R.u[1] * d1 + R.u[4] * d2, a2 = R.u[2] * d2;
         W[k] = 0.25 * f * exp2(-(a0 * a0 + a1 * a1 + a2 * a2));
     }
-    w[idx * 4 + 0] = (float)(W[0] + W[1] + W[2] + W[3]);
-    w[idx * 4 + 1] = (float)(W[0] - W[1] - W[2] + W[3]);
-    w[idx * 4 + 2] = (float)(W[0] - W[1] + W[2] - W[3]);
-    w[idx * 4 + 3] = (float)(W[0] + W[1] - W[2] - W[3]);
+    const float v[4] = {(float)(W[0] + W[1] + W[2] + W[3]), (float)(W[0] - W[1] - W[2] + W[3]),
+                        (float)(W[0] - W[1] + W[2] - W[3]), (float)(W[0] + W[1] - W[2] - W[3])};
+#pragma unroll
+    for (int k = 0; k < 4; k++) w[idx * 4 + k] = v[k];
+    return isfinite(v[0]) && isfinite(v[1]) && isfinite(v[2]) && isfinite(v[3]);
 }
 
 // |column c of U'|^2: the curvature of the exponent along axis c
@@ -1501,14 +1515,18 @@ __global__ __launch_bounds__(64) void psf_voxel_setup_kernel(gt_atoms A, gt_vol 
     }
     const int np = psf_whole_rule(3, hv, sig, cs);
     PsfNode3 &T = nodes[j];
-    if (lane == 0) T.np = np;
+    bool finite = true;
     switch (np) {
-    case 3: psf_node_entry<3>(R, hv, lane, T.w); break;
-    case 4: psf_node_entry<4>(R, hv, lane, T.w); break;
-    case 5: psf_node_entry<5>(R, hv, lane, T.w); break;
-    case 6: psf_node_entry<6>(R, hv, lane, T.w); break;
+    case 3: finite = psf_node_entry<3>(R, hv, lane, T.w); break;
+    case 4: finite = psf_node_entry<4>(R, hv, lane, T.w); break;
+    case 5: finite = psf_node_entry<5>(R, hv, lane, T.w); break;
+    case 6: finite = psf_node_entry<6>(R, hv, lane, T.w); break;
     default: break;
     }
+    // an amplitude that is not finite (or whose weights are not) stays within
+    // its support's box: psf_voxel
+    finite = __all(finite);
+    if (lane == 0) T.np = finite ? np : 0;
 }
 
 template <int NP> __device__ inline float psf_voxel_nodes(smem<float> *w, float t0, float t1, float t2)

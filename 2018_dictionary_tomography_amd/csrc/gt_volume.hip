@@ -222,8 +222,9 @@ __global__ __launch_bounds__(V3_THREADS) void volume3_kernel(const VolRec *__res
             for (int k = 0; k < 4; k++) {
                 const float v0 = fmaf(u0, (y0[k] - xh) - xl, a0);
                 const float ex = fmaf(-v0, v0, c);
-                const float E = ex >= kap ? __builtin_amdgcn_exp2f(ex) : 0.0f;
-                part[k] = fmaf(amp, E, part[k]);
+                // the term is chosen, not its profile: 0 times an infinite amplitude is no 0
+                const float v = amp * __builtin_amdgcn_exp2f(ex);
+                part[k] += ex >= kap ? v : 0.0f;
             }
             if ((++n & 3) == 0) {
 #pragma unroll
