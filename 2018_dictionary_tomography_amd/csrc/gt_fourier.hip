@@ -279,8 +279,7 @@ struct alignas(16) FzTerm {
 // record of the patch's records (a thread per record: index box, then
 // ft_box_meets), their FP64 sums added in wave order.  A sample's phase is the
 // product of three table entries: per record one complex product for the lane's
-// (k1, k2) and one per k0.  Four records' values are summed in FP32 and added to
-// the FP64 total.
+// (k1, k2) and one per k0; the values are added in FP64.
 // Bound by VALU issue on the central patches and by the latency of a patch's
 // staging elsewhere: large blocks keep the first short, the cells' lists and a
 // patch counter the second.  2000 atoms on 128^3: 0.227 ms (patches of 64
@@ -373,10 +372,6 @@ __global__ __launch_bounds__(FZ_THREADS) void ft_grid_kernel(const FtRec *__rest
                 ids[pos] = (unsigned short)j;
             }
             __syncthreads();
-            float gr[FZ_K0], gi[FZ_K0];
-#pragma unroll
-            for (int z = 0; z < FZ_K0; z++) gr[z] = gi[z] = 0.0f;
-            int n = 0;
             // the lane's table entries of the next record are loaded while one is summed
             auto entries = [&](int q, float2 &b, float2 &c) {
                 const size_t o = (size_t)__builtin_amdgcn_readfirstlane((int)ids[min(q, len - 1)]) * m;
@@ -391,19 +386,11 @@ __global__ __launch_bounds__(FZ_THREADS) void ft_grid_kernel(const FtRec *__rest
                 for (int z = 0; z < FZ_K0; z++) {
                     const float w0 = f.u[0] * k0[z], w1 = fmaf(f.u[3], k0[z], v1), w2 = fmaf(f.u[5], k0[z], v2);
                     const float nq = fmaf(w0, w0, fmaf(w1, w1, w2 * w2));
+                    if (!(nq < cut)) continue;  // (0 times an infinite amplitude is no 0)
                     const float E = __builtin_amdgcn_exp2f(-nq);
-                    // the terms are chosen, not E: 0 times an infinite amplitude is no 0
-                    const float re = E * fmaf(f.a[z].x, pr, -f.a[z].y * pi), im = E * fmaf(f.a[z].x, pi, f.a[z].y * pr);
-                    gr[z] += nq < cut ? re : 0.0f;
-                    gi[z] += nq < cut ? im : 0.0f;
+                    sr[z] += (double)(E * fmaf(f.a[z].x, pr, -f.a[z].y * pi));
+                    si[z] += (double)(E * fmaf(f.a[z].x, pi, f.a[z].y * pr));
                 }
-                if ((++n & 3) == 0)
-#pragma unroll
-                    for (int z = 0; z < FZ_K0; z++) {
-                        sr[z] += (double)gr[z];
-                        si[z] += (double)gi[z];
-                        gr[z] = gi[z] = 0.0f;
-                    }
             };
             if (wave < len) {
                 float2 b, c, bn, cn;
@@ -416,11 +403,6 @@ __global__ __launch_bounds__(FZ_THREADS) void ft_grid_kernel(const FtRec *__rest
                     sum(q, bn, cn);
                     if ((q += FZ_WAVES) >= len) break;
                 }
-            }
-#pragma unroll
-            for (int z = 0; z < FZ_K0; z++) {
-                sr[z] += (double)gr[z];
-                si[z] += (double)gi[z];
             }
             __syncthreads();
         }

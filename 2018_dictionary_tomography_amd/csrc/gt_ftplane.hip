@@ -303,15 +303,13 @@ __global__ __launch_bounds__(256) void kp_eval_kernel(const KpRec<R> *__restrict
 // The phase is a row part plus a column part: per record each lane evaluates
 // the sine and cosine of one column or row (handed round through LDS), and a
 // sample costs one complex product instead of two phase reductions, a sine and
-// a cosine.  KE_GROUP records' values are summed in FP32 and added to the FP64
-// total.  The planes pass through k = 0 and out(-k) = conj(out(k)): on ascending
+// a cosine.  A sample's values are added in FP64.  The planes pass through k = 0 and out(-k) = conj(out(k)): on ascending
 // axes that pair k with -k (0: m-1-i, 1: m-i and none for i = 0, an even FFT's)
 // the rectangles of k0 < 0 whose samples all have a partner are written with it.
 // Bound by VALU issue: 2000 atoms, 61 x 128^2 samples: 0.97 -> 0.35 ms, 0.235 with
 // the partners; without the row pairs 0.38.
 static_assert(sizeof(KpRec<float>) == 48, "KpRec<float>: amp, q[3] | ch[2], cl[2] | lo[2], hi[2]");
 constexpr int KE_WAVES = 8, KE_ROWS = 16, KE_COLS = 32, KE_R = KE_ROWS / 2;
-constexpr int KE_GROUP = 8;
 
 __global__ __launch_bounds__(64 * KE_WAVES) void kp_rect_kernel(const KpRec<float> *__restrict__ recs,
                                                                 const int *__restrict__ pairing, int N, KpDev<float> P,
@@ -380,9 +378,6 @@ __global__ __launch_bounds__(64 * KE_WAVES) void kp_rect_kernel(const KpRec<floa
         }
         wave_lists<KE_WAVES, 1>(hit, wl, cnt, wlen);
         const int len = __builtin_amdgcn_readfirstlane(wlen[0]);
-        float gr[KE_R], gi[KE_R];
-#pragma unroll
-        for (int r = 0; r < KE_R; r++) gr[r] = gi[r] = 0.0f;
         // software pipeline: while record k is summed, record k + KE_WAVES is on
         // its way to scalar registers; its phases follow, into the other half
         // of the wave's phase buffer
@@ -433,28 +428,14 @@ __global__ __launch_bounds__(64 * KE_WAVES) void kp_rect_kernel(const KpRec<floa
                 if ((m >> r) & 1u) {
                     const float rc = (r & 1) ? v[r / 2].z : v[r / 2].x, rs = (r & 1) ? v[r / 2].w : v[r / 2].y;
                     const float ex = fmaf(fmaf(q0, p0[r], b), p0[r], c);
+                    if (!(ex > cutlog)) continue;  // (0 times an infinite amplitude is no 0)
                     const float E = __builtin_amdgcn_exp2f(ex);
-                    // the terms are chosen, not E: 0 times an infinite amplitude is no 0
-                    const float re = E * fmaf(rc, cc, -rs * cn), im = E * fmaf(rc, cn, rs * cc);
-                    gr[r] += ex > cutlog ? re : 0.0f;
-                    gi[r] -= ex > cutlog ? im : 0.0f;
+                    sr[r] += (double)(E * fmaf(rc, cc, -rs * cn));
+                    si[r] -= (double)(E * fmaf(rc, cn, rs * cc));
                 }
-            if ((n & (KE_GROUP - 1)) == KE_GROUP - 1) {
-#pragma unroll
-                for (int r = 0; r < KE_R; r++) {
-                    sr[r] += (double)gr[r];
-                    si[r] += (double)gi[r];
-                    gr[r] = gi[r] = 0.0f;
-                }
-            }
             phases(&nr, rph[wave][(n + 1) & 1]);
             m = mn;
             wave_sync();
-        }
-#pragma unroll
-        for (int r = 0; r < KE_R; r++) {
-            sr[r] += (double)gr[r];
-            si[r] += (double)gi[r];
         }
         __syncthreads();
     }

@@ -691,8 +691,8 @@ __device__ inline int psf_stage(const PsfRec *__restrict__ ra, int base, int N, 
 // Vector issue and the evenness of the blocks bound it.  Every exponential of a
 // cell is a factor of its column times a factor of its row (PfTab): a wave forms
 // those of four records at once, 1.5 exponentials per record, lane and node pair
-// instead of 8 (two pixels, two axes, two signs) and a product per pixel.  Four
-// records' values are summed in FP32 and added to an FP64 total.  1000 atoms, 61
+// instead of 8 (two pixels, two axes, two signs) and a product per pixel.  A
+// pixel's values are added in FP64.  1000 atoms, 61
 // x 128^2: 1.59 ms with a form per node, 0.45 with the node weights tabulated
 // (8 x 64 pixels per block), 0.39 with the factors tabulated, 0.35 with 8 x 32
 // pixels, 0.34 with two waves per rectangle (four: 0.40).
@@ -881,7 +881,6 @@ __global__ __launch_bounds__(PF_WAVES * 64) __attribute__((amdgpu_waves_per_eu(5
                 }
                 wave_sync();
                 wd = word(e + 4 * PF_GROUPS);
-                float gA = 0.0f, gB = 0.0f;
 #pragma unroll 1
                 for (int u = 0; u < 4 && e + u < len; u++) {
                     const int jj = base + (u < 2 ? (u == 0 ? jjs[0] : jjs[1]) : (u == 2 ? jjs[2] : jjs[3]));
@@ -896,11 +895,9 @@ __global__ __launch_bounds__(PF_WAVES * 64) __attribute__((amdgpu_waves_per_eu(5
                     case 6: psf_two_pixels<6>(T, u, q0u, w, lane, vA, vB); break;
                     default: pieces = true;
                     }
-                    gA += vA;
-                    gB += vB;
+                    sA += (double)vA;
+                    sB += (double)vB;
                 }
-                sA += (double)gA;
-                sB += (double)gB;
             }
         }
         if (pieces)
@@ -1584,8 +1581,8 @@ template <int NP> __device__ inline float psf_voxel_nodes(smem<float> *w, float 
 // the plane through the cube's centre across the exponent's gradient g there
 // (the support reaches |v| rho along it, v = U'(yc - x), rho^2 = -kappa; the
 // cube comes as near as |v|^2 - sum |g_c| extent_c).  Records and node tables are
-// read into scalar registers; four records' values are summed in FP32 and
-// added to an FP64 total, the groups' totals in group order.  Bound by VALU
+// read into scalar registers; a voxel's values are added in FP64, the groups'
+// totals in group order.  Bound by VALU
 // issue: a voxel costs 7 to 19 exponentials instead of 27 to 216, and the cube
 // test drops what the boxes of slanted ellipsoids keep; 1000 atoms on 64^3:
 // 1.75 -> 0.165 ms with bricks of 4 x 8 x 8 and 16 waves, 0.146 with 8 waves,
@@ -1662,8 +1659,6 @@ __global__ __launch_bounds__(PX_THREADS) __attribute__((amdgpu_waves_per_eu(5)))
         }
         wave_lists<PX_WAVES, PX_CUBES>(mask, wl, cnt, wlen);
         const int len = __builtin_amdgcn_readfirstlane(wlen[cube]);
-        float part = 0.0f;
-        int n4 = 0;
         bool pieces = false;  // records that no rule covers whole
         for (int k = grp; k < len; k += PX_GROUPS) {
             const int jj = base + __builtin_amdgcn_readfirstlane((int)wl[cube][k]);
@@ -1684,13 +1679,8 @@ __global__ __launch_bounds__(PX_THREADS) __attribute__((amdgpu_waves_per_eu(5)))
             case 6: v = psf_cell_value<6>(w, g, hv, ex); break;
             default: v = 0.0f, pieces = true;
             }
-            part += v;
-            if ((++n4 & 3) == 0) {
-                s += (double)part;
-                part = 0.0f;
-            }
+            s += (double)v;
         }
-        s += (double)part;
         if (pieces)
             for (int k = grp; k < len; k += PX_GROUPS) {
                 const int jj = base + __builtin_amdgcn_readfirstlane((int)wl[cube][k]);

@@ -130,8 +130,8 @@ constexpr int VCHUNK = 128;
 // coordinates) the plane through the part's centre across the exponent's
 // gradient g there: the support reaches |v| rho along g (v = U'(yc - x), rho^2 =
 // -kappa), the voxels come as near as |v|^2 - sum |g_c| extent_c.  Records are read
-// into scalar registers; four records' values are summed in FP32 and added to
-// the voxel's FP64 total, the groups' totals in group order.
+// into scalar registers; a voxel's values are added in FP64, the groups' totals
+// in group order.
 // Bound by VALU issue and by the central bricks, which meet the most atoms: the
 // parts' lists are split so that no wave is much longer than the rest.  1000
 // atoms on 128^3: 0.22 ms with 4 x 4 x 64 bricks culled by index box, 0.086 now;
@@ -209,8 +209,6 @@ __global__ __launch_bounds__(V3_THREADS) void volume3_kernel(const VolRec *__res
         }
         wave_lists<V3_WAVES, V3_PARTS>(mask, wl, cnt, wlen);
         const int len = __builtin_amdgcn_readfirstlane(wlen[sub]);
-        float part[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        int n = 0;
         for (int q = grp; q < len; q += V3_GROUPS) {
             smem<VolRec> *r = scalar_ptr(recs) + (base + __builtin_amdgcn_readfirstlane((int)wl[sub][q]));
             const float d1 = (y1 - r->xh[1]) - r->xl[1], d2 = (y2 - r->xh[2]) - r->xl[2];
@@ -224,18 +222,9 @@ __global__ __launch_bounds__(V3_THREADS) void volume3_kernel(const VolRec *__res
                 const float ex = fmaf(-v0, v0, c);
                 // the term is chosen, not its profile: 0 times an infinite amplitude is no 0
                 const float v = amp * __builtin_amdgcn_exp2f(ex);
-                part[k] += ex >= kap ? v : 0.0f;
-            }
-            if ((++n & 3) == 0) {
-#pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    s[k] += (double)part[k];
-                    part[k] = 0.0f;
-                }
+                s[k] += (double)(ex >= kap ? v : 0.0f);
             }
         }
-#pragma unroll
-        for (int k = 0; k < 4; k++) s[k] += (double)part[k];
         __syncthreads();
     }
     // the groups' totals, in group order

@@ -1,0 +1,60 @@
+"""The sums over atoms are carried in FP64: 96 copies of one atom, their
+amplitudes 2^20, 1 and -2^20 times one value in any order, give 32 times the
+output of the one atom, bit for bit.  (A factor of a power of two scales every
+term exactly, and the FP64 sum of terms of 24 bits, at most 26 binary places
+apart, is exact in any order; a sum in 24 bits is off by a sixteenth of a term at
+each step.)
+"""
+import importlib
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _copies(rng, I, x, r):
+    f = np.tile([2.0 ** 20, 1.0, -(2.0 ** 20)], 32)
+    rng.shuffle(f)
+    return I * f, np.tile(x, (96, 1)), np.tile(r, (96, 1))
+
+
+def _same(many, one):
+    assert torch.isfinite(one).all() and one.abs().max() > 0
+    assert torch.equal(many, 32 * one)
+
+
+# (widths from a few cells to less than one: every rule of the point-spread cells)
+@pytest.mark.parametrize("width", [0.3, 0.08, 0.03])
+@pytest.mark.parametrize("op,call", [("GaussTomo", "volume"), ("SingleParticleGaussTomo", "volume"),
+                                     ("SingleParticleGaussTomo", "projection")])
+def test_renders_and_point_spread_projection(gt, cuda, width, op, call):
+    rng = np.random.default_rng(3)
+    I, x = np.array([0.75]), rng.uniform(-0.2, 0.2, (1, 3))
+    r = np.concatenate((1.0 / (width * rng.uniform(0.8, 1.2, (1, 3))), rng.normal(0, 0.5 / width, (1, 3)) / 3), 1)
+    r = r / np.sqrt(60.0) * 2
+    space = gt.AtomSpace(3, isotropic=False)
+    T, ortho = gt.spaces.axis_tilt_geometry(np.linspace(-1, 1, 3), [0, 1, 0], ref=np.array([1.0, 0, 0]))
+    P = gt.ProjSpace(orientations=T, ortho=ortho, detector=[gt.cell_centres(-1, 1, m) for m in (40, 37)])
+    A = getattr(gt, op)(space, gt.VolSpace([gt.cell_centres(-1, 1, m) for m in (28, 25, 30)]), P)
+    run = A.discretise if call == "volume" else A
+    one = run(gt.AtomElement(space, x, r, I, device=cuda)).data
+    In, xn, rn = _copies(rng, I, x, r)
+    _same(run(gt.AtomElement(space, xn, rn, In, device=cuda)).data, one)
+
+
+@pytest.mark.parametrize("planes", [False, True])
+def test_fourier(gt, cuda, planes):
+    fo = importlib.import_module("2018_dictionary_tomography_amd.fourier")
+    rng = np.random.default_rng(3)
+    I, x = np.array([0.75]), rng.uniform(-0.2, 0.2, (1, 3))
+    r = np.concatenate((rng.uniform(0.3, 0.9, (1, 3)), rng.normal(0, 0.1, (1, 3))), 1)
+    k = [np.arange(m, dtype=np.float32) - m // 2 for m in (24, 27, 30)]
+    S = k
+    if planes:
+        T, ortho = gt.spaces.axis_tilt_geometry(np.linspace(-1, 1, 3), [0, 1, 0], ref=np.array([1.0, 0, 0]))
+        S = (k[1], k[2], *ortho)
+    one = fo.evaluate(fo.FTAtoms(I, x, r, device=cuda), S)
+    In, xn, rn = _copies(rng, I, x, r)
+    _same(torch.view_as_real(fo.evaluate(fo.FTAtoms(In, xn, rn, device=cuda), S)), torch.view_as_real(one))
