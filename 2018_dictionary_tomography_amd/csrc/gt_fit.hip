@@ -1053,33 +1053,37 @@ __global__ __launch_bounds__(FIT_THREADS) void fit_kernel(gt_fit_slot *__restric
         __syncthreads();
         GT_FIT_TICK(3);
         if (L.stop) break;
-        if (L.skip) {  // block variant: nothing to try for this block
-            __syncthreads();  // (the flag is cleared with the next choice)
-            if (tid == 0) fit_advance(L.c, S, true);
-            continue;
+        if (!L.skip) {
+            // ---- phase E: detector Gaussians of the proposal -------------------
+            for (int k = tid; k < nOwn; k += FIT_THREADS) {
+                PairGeom<D> g;
+                atom_from_theta<D>(L.th_new, iso, g);
+                angle_from_stash<D>(L.geo[k], Gm.lenT, g);
+                pair_setup<D>(g, det, nd, S.sorted, L.rec_new[k]);
+            }
+            __syncthreads();
+            GT_FIT_TICK(4);
+            // ---- phase F: per-angle FP64 energy changes -----------------------
+            for (int k = next_angle(&L.next[1], lane); k < nOwn; k = next_angle(&L.next[1], lane)) {
+                const int a = member + G * k;
+                gmem<float> *Ra = resid + (size_t)a * slab;
+                float2 *dt = reinterpret_cast<float2 *>(L.tab[wave]);
+                double acc = stage ? pair_delta4<K, 2>(L.rec_old[k], L.rec_new[k], L.p0, L.p1, Ra,
+                                                       stage + (size_t)a * slab, n1, lane, dt)
+                                   : pair_delta4<K, 0>(L.rec_old[k], L.rec_new[k], L.p0, L.p1, Ra, nullptr, n1, lane, dt);
+                acc = wave_sum_f64(acc);
+                if (lane == 0) xput(dEa + a, acc);
+            }
         }
-        // ---- phase E: detector Gaussians of the proposal -------------------
-        for (int k = tid; k < nOwn; k += FIT_THREADS) {
-            PairGeom<D> g;
-            atom_from_theta<D>(L.th_new, iso, g);
-            angle_from_stash<D>(L.geo[k], Gm.lenT, g);
-            pair_setup<D>(g, det, nd, S.sorted, L.rec_new[k]);
-        }
-        __syncthreads();
-        GT_FIT_TICK(4);
-        // ---- phase F: per-angle FP64 energy changes -----------------------
-        for (int k = next_angle(&L.next[1], lane); k < nOwn; k = next_angle(&L.next[1], lane)) {
-            const int a = member + G * k;
-            gmem<float> *Ra = resid + (size_t)a * slab;
-            float2 *dt = reinterpret_cast<float2 *>(L.tab[wave]);
-            double acc = stage ? pair_delta4<K, 2>(L.rec_old[k], L.rec_new[k], L.p0, L.p1, Ra,
-                                                   stage + (size_t)a * slab, n1, lane, dt)
-                               : pair_delta4<K, 0>(L.rec_old[k], L.rec_new[k], L.p0, L.p1, Ra, nullptr, n1, lane, dt);
-            acc = wave_sum_f64(acc);
-            if (lane == 0) xput(dEa + a, acc);
-        }
+        // (a block with nothing to try meets here as well: no member writes its
+        // next entries while another still adds the last ones up)
         GT_FIT_MEET();
         GT_FIT_TICK(5);
+        if (L.skip) {
+            if (tid == 0) fit_advance(L.c, S, true);
+            __syncthreads();  // all of wave 0 reads the new place at the top
+            continue;
+        }
         // ---- phase G: accept / reject, step size, flags -------------------
         if (wave == 0) {
             double dE = 0.0;
