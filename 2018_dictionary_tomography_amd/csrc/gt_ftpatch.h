@@ -69,19 +69,32 @@ __host__ __device__ inline bool ft_box_meets(const FtL &r, float m0, float m1, f
     return !(n2 * (1.0f - 1e-4f) - reach > rho * (1.0f + 1e-3f) * sqrtf(n2));
 }
 
+// A form that the two tests below may not cull by: not strictly concave, or so
+// long and slanted an ellipse that its FP32 coefficients do not place it.
+// det = 4 q0 q2 - q1^2 is off by at most 8 u q0 q2 = 4.8e-7 q0 q2, so the half-width
+// and the extreme point of kp_row_range by det's relative error / 2 (2.4e-4 at
+// the limit) and a root whose discriminant cancels by 5.5e-4 of the half-width:
+// less than its widening of 1e-3 down to det = 1e-3 q0 q2 (axis ratio 126 at 45
+// degrees).  With a limit of 1e-6 rows with samples up to 1e-3 of the peak went
+// missing at ratios from 700 on.
+__host__ __device__ inline bool kp_thin(float q0, float q1, float q2)
+{
+    return !(q0 < 0.0f) || !(q2 < 0.0f) || !(4.0f * q0 * q2 - q1 * q1 > 1e-3f * q0 * q2);
+}
+
 // The rows [xlo, xhi] that the ellipse {q0 x^2 + q1 x y + q2 y^2 >= cut} (cut <
 // 0) has in the band ya <= y <= yb: its convex part in the band spans from the
 // least to the largest x, each at the ellipse's own extreme point when that
 // lies in the band, else on the nearer band edge.  Widened by a relative 1e-3;
-// everything for a form that is not strictly concave; empty (xlo > xhi) when
-// the band misses the ellipse.
+// everything for a thin form; empty (xlo > xhi) when the band misses the
+// ellipse.
 __host__ __device__ inline void kp_row_range(float q0, float q1, float q2, float cut, float ya, float yb, float &xlo,
                                              float &xhi)
 {
     xlo = -3.0e38f;
     xhi = 3.0e38f;
+    if (kp_thin(q0, q1, q2)) return;
     const float det = 4.0f * q0 * q2 - q1 * q1;
-    if (!(q0 < 0.0f) || !(q2 < 0.0f) || !(det > 1e-6f * q0 * q2)) return;
     const float hw = sqrtf(4.0f * cut * q2 / det);  // half-width in x
     const float ys = -0.5f * q1 / q2 * hw;          // y of the point x = hw (x = -hw: -ys)
     const float yr = fminf(fmaxf(ys, ya), yb), yl = fminf(fmaxf(-ys, ya), yb);

@@ -360,7 +360,8 @@ __global__ __launch_bounds__(64 * KE_WAVES) void kp_rect_kernel(const KpRec<floa
             const float4 f0 = reinterpret_cast<const float4 *>(ra + j)[0];  // amp, q
             const int4 bx = reinterpret_cast<const int4 *>(ra + j)[2];      // lo, hi
             if ((int)(bx.x <= row1) & (int)(bx.z >= row0) & (int)(bx.y <= col1) & (int)(bx.w >= col0))
-                hit = !P.sorted || support_meets_rect(make_float4(0.0f, f0.y, f0.z, f0.w),
+                hit = !P.sorted || kp_thin(f0.y, f0.z, f0.w) ||
+                      support_meets_rect(make_float4(0.0f, f0.y, f0.z, f0.w),
                                                       make_float4(0.0f, 0.0f, 0.0f, 0.0f), xa, xb, ya, yb, cutlog);
             if (hit) {
                 unsigned m = (1u << KE_R) - 1u;
