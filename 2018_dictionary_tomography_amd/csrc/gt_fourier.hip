@@ -111,13 +111,14 @@ __device__ inline float turns(float xh, float xl, float k, float &err)
 // ---------------------------------------------------------------------------
 // Every atom's support {|U^T k|^2 < 30} is an ellipsoid about k = 0 (about 1%
 // of a 128^3 grid), so the samples near the origin see nearly every atom and
-// most patches of samples see few or none.  At most FZ_MAX_ATOMS atoms are
+// most patches of samples see few or none.  With tables (ft_tabulated) atoms are
 // evaluated in three kernels: the atoms' records and phase tables
 // (ft_atoms_kernel); per cell of many patches the list of the records that reach
 // it, and the list of the patches of the cells with any (ft_bin_kernel, which
 // also clears the output); those patches (ft_grid_kernel).
 // ---------------------------------------------------------------------------
 constexpr int FZ_MAX_ATOMS = 16384;  // more: ft_patch_kernel, without the tables' memory
+constexpr size_t FZ_MAX_BYTES = (size_t)256 << 20;  // as above; more only up to the output's size
 
 // State of one evaluation: the axes' pairing, the number of listed patches by
 // class of their cell's record count (most first) and the next one to be taken.
@@ -437,8 +438,31 @@ __global__ __launch_bounds__(FZ_THREADS) void ft_grid_kernel(const FtRec *__rest
     }
 }
 
-// More atoms than FZ_MAX_ATOMS: one block of 4 waves per 8 x 8 (k1, k2) patch at one k0;
-// lane l holds the sample at offset (l / 8, l % 8).  Staging (a thread per
+// One wave per atom j: its rank = the atoms of larger radius, or of equal
+// radius and smaller index; the record is copied to that position.
+__global__ __launch_bounds__(256) void ft_rank_kernel(const FtRec *__restrict__ recs, int N, FtRec *__restrict__ sorted)
+{
+    const int lane = threadIdx.x & 63;
+    const int j = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (j >= N) return;
+    const float rj = recs[j].pad0[0];
+    int rank = 0;
+    for (int i = lane; i < N; i += 64) {
+        const float ri = recs[i].pad0[0];
+        rank += (ri > rj || (ri == rj && i < j)) ? 1 : 0;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) rank += __shfl_xor(rank, o);
+    // eight lanes copy the 128-byte record, 16 bytes each
+    if (lane < 8)
+        reinterpret_cast<int4 *>(sorted + rank)[lane] = reinterpret_cast<const int4 *>(recs + j)[lane];
+}
+
+// Without tables (ft_tabulated, or no room for them): the records of at most
+// FZ_MAX_ATOMS atoms are put in order of decreasing radius of a ball about k = 0
+// holding the support, so that a patch at distance d from the origin only looks at
+// the leading records of radius >= d; more are taken in atom order.  One block of 4
+// waves per 8 x 8 (k1, k2) patch at one k0; lane l holds the sample at offset (l / 8, l % 8).  Staging (a thread per
 // record, records of radius >= the patch's distance from the origin only):
 // the record's index box against the patch and, for an ascending grid, the
 // least |U^T k|^2 over the patch against the cutoff (ft_patch_min, with a
@@ -450,7 +474,8 @@ __global__ __launch_bounds__(FZ_THREADS) void ft_grid_kernel(const FtRec *__rest
 constexpr int FP_THREADS = 256, FP_WAVES = 4, FP_CHUNK = 256, FP_PATCH = 8;
 
 __global__ __launch_bounds__(FP_THREADS) void ft_patch_kernel(const FtRec *__restrict__ recs, int N, gt_kgrid Kg,
-                                                              float2 *__restrict__ out, int e0, int e1, int e2)
+                                                              float2 *__restrict__ out, int e0, int e1, int e2,
+                                                              int by_radius)
 {
     __shared__ FtL list[FP_CHUNK];  // also the reduction buffer at the end
     __shared__ int wcnt[FP_WAVES];
@@ -476,6 +501,8 @@ __global__ __launch_bounds__(FP_THREADS) void ft_patch_kernel(const FtRec *__res
     const float cut_keep = cut * (1.0f + 1e-4f);
     double sr = 0.0, si = 0.0;
     for (int base = 0; base < N; base += FP_CHUNK) {
+        // records in radius order: this and every later one fall short of the patch
+        if (by_radius && recs[base].pad0[0] < dmin) break;
         const int j = base + (int)threadIdx.x;
         bool hit = false;
         if (j < N) {
@@ -541,8 +568,8 @@ __global__ void cfill_kernel(float2 *p, size_t n)
 
 using namespace gt;
 
-// Workspace: the records; for at most FZ_MAX_ATOMS atoms also the state, the
-// cells' record lists, the patch list and the phase tables.
+// Workspace: the records; with tables also the state, the cells' record lists,
+// the patch lists and the phase tables.
 static FzCells ft_cells(const gt_kgrid *g)
 {
     FzCells F;
@@ -574,11 +601,29 @@ static FtLayout ft_layout(const gt_atoms *a, const gt_kgrid *g, const FzCells &F
     return l;
 }
 
+// Without tables: the records and, where they are ranked, their copy in radius order.
+static size_t ft_least(const gt_atoms *a)
+{
+    const size_t one = align_up((size_t)a->n * sizeof(FtRec));
+    return a->n <= FZ_MAX_ATOMS ? 2 * one : one;
+}
+
+// Are the atoms evaluated with tables?  These grow with atoms x (m0 + m1 + m2)
+// and with the number of patches, so a long thin grid of many atoms would take
+// hundreds of times its output (16384 atoms on 2^20 x 1 x 1 samples: 137 GB of
+// tables for 8 MB).
+static bool ft_tabulated(const gt_atoms *a, const gt_kgrid *g)
+{
+    if (a->n > FZ_MAX_ATOMS) return false;
+    const size_t out = (size_t)g->m0 * g->m1 * g->m2 * sizeof(float2);
+    return ft_layout(a, g, ft_cells(g)).total <= std::max(FZ_MAX_BYTES, out);
+}
+
 extern "C" size_t gt_ft_workspace(const gt_atoms *atoms, const gt_kgrid *grid)
 {
     if (!atoms || atoms->n <= 0) return 0;
     const bool ok = grid && grid->m0 >= 1 && grid->m1 >= 1 && grid->m2 >= 1;
-    if (atoms->n > FZ_MAX_ATOMS || !ok) return align_up((size_t)atoms->n * sizeof(FtRec));
+    if (!ok || !ft_tabulated(atoms, grid)) return ft_least(atoms);
     return ft_layout(atoms, grid, ft_cells(grid)).total;
 }
 
@@ -593,7 +638,10 @@ extern "C" int gt_ft_eval(const gt_atoms *atoms, const gt_kgrid *grid, float *ou
     GT_CHECK_ARG(grid->m0 < (1 << 24) && grid->m1 < (1 << 24) && grid->m2 < (1 << 24), "gt_ft_eval: grid too large");
     GT_CHECK_ARG(grid->k0 && grid->k1 && grid->k2, "gt_ft_eval: grid vectors must be non-NULL");
     GT_CHECK_ARG(out != nullptr, "gt_ft_eval: out is NULL");
-    const size_t need = gt_ft_workspace(atoms, grid);
+    // (a workspace that holds no tables is enough for the kernel without them)
+    const size_t tables = atoms->n > 0 && ft_tabulated(atoms, grid) ? gt_ft_workspace(atoms, grid) : 0;
+    const bool tabulated = tables > 0 && tables <= ws_bytes;
+    const size_t need = atoms->n <= 0 ? 0 : (tables > 0 ? std::min(tables, ft_least(atoms)) : ft_least(atoms));
     if (need > ws_bytes || (need > 0 && ws == nullptr)) {
         set_error("gt_ft_eval: workspace of %zu bytes given, %zu needed", ws_bytes, need);
         return GT_EWORKSPACE;
@@ -613,7 +661,7 @@ extern "C" int gt_ft_eval(const gt_atoms *atoms, const gt_kgrid *grid, float *ou
     const int e[3] = {ceil_log2(grid->m0), ceil_log2((grid->m1 + FP_PATCH - 1) / FP_PATCH),
                       ceil_log2((grid->m2 + FP_PATCH - 1) / FP_PATCH)};
     GT_CHECK_ARG(e[0] + e[1] + e[2] <= 30, "gt_ft_eval: grid too large");
-    if (atoms->n <= FZ_MAX_ATOMS) {
+    if (tabulated) {
         const FzCells F = ft_cells(grid);
         const FtLayout l = ft_layout(atoms, grid, F);
         char *w = (char *)ws;
@@ -635,10 +683,17 @@ extern "C" int gt_ft_eval(const gt_atoms *atoms, const gt_kgrid *grid, float *ou
         return 0;
     }
     hipLaunchKernelGGL(ft_setup_kernel, dim3(sb), dim3(256), 0, st, *atoms, *grid, recs);
+    const FtRec *order = recs;
+    if (atoms->n <= FZ_MAX_ATOMS) {
+        FtRec *sorted = (FtRec *)((char *)ws + align_up((size_t)atoms->n * sizeof(FtRec)));
+        hipLaunchKernelGGL(ft_rank_kernel, dim3((unsigned)((atoms->n + 3) / 4)), dim3(256), 0, st, recs, atoms->n,
+                           sorted);
+        order = sorted;
+    }
     const unsigned blocks = 1u << (e[0] + e[1] + e[2]);
     prof_begin(st, GT_K_FT);
-    hipLaunchKernelGGL(ft_patch_kernel, dim3(blocks), dim3(FP_THREADS), 0, st, recs, atoms->n, *grid, (float2 *)out,
-                       e[0], e[1], e[2]);
+    hipLaunchKernelGGL(ft_patch_kernel, dim3(blocks), dim3(FP_THREADS), 0, st, order, atoms->n, *grid, (float2 *)out,
+                       e[0], e[1], e[2], order != recs ? 1 : 0);
     prof_end(st, GT_K_FT);
     GT_HIP(hipGetLastError());
     return 0;

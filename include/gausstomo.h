@@ -162,7 +162,9 @@ int gt_volume(const gt_atoms *atoms, const gt_vol *vol, float *u, void *ws, size
 /* Fourier evaluation on a separable 3D grid (FTGaussian3D.__grid_eval_*,
  * GaussDictCode/bin/FTGaussian3D.py:95-110,151-164).  atoms hold FT-space
  * parameters (Fourier_Transform.py:293-333).  out: [m0][m1][m2] complex64
- * as interleaved (re, im) floats. */
+ * as interleaved (re, im) floats.  The workspace holds phase tables where they pay
+ * and stay below 256 MiB or the size of out; gt_ft_workspace(atoms, NULL) bytes
+ * (256 per atom, 128 above 16384 atoms) are enough for any grid, evaluated without them. */
 size_t gt_ft_workspace(const gt_atoms *atoms, const gt_kgrid *grid);
 int gt_ft_eval(const gt_atoms *atoms, const gt_kgrid *grid, float *out, void *ws, size_t ws_bytes,
                void *stream);
