@@ -188,23 +188,28 @@ __device__ inline void ft_sincos_turns(float t, float &sn, float &cs)
     cs = __builtin_amdgcn_cosf(t);
 }
 
-// The same by polynomials: t is reduced to the nearest quarter turn (exactly)
-// and sin(2 pi r) / r, cos(2 pi r) are interpolated in r^2 at the Chebyshev
-// points of |r| <= 1/8 (4 and 5 terms); maximum absolute error 8.2e-8 and
-// 5.8e-8, rms 2e-8.  About 24 operations, for phases that many samples share.
-__device__ inline void ft_sincos_shared(float t, float &sn, float &cs)
+// The same by polynomials, t = q / 4 + r with |r| <= 1/8: sin(2 pi r) / r and
+// cos(2 pi r) are interpolated in r^2 at the Chebyshev points (4 and 5 terms);
+// maximum absolute error 8.2e-8 and 5.8e-8, rms 2e-8.
+__device__ inline void ft_sincos_quarter(int q, float r, float &sn, float &cs)
 {
-    const float n = rintf(4.0f * t);
-    const float r = fmaf(-0.25f, n, t), z = r * r;
+    const float z = r * r;
     const float s = r * fmaf(fmaf(fmaf(-75.39643085838416f, z, 81.59244143217468f), z, -41.341662093897966f), z,
                              6.2831852875017855f);
     const float c = fmaf(fmaf(fmaf(fmaf(59.21609823587779f, z, -85.44273312246247f), z, 64.9393151998861f), z,
                               -19.739208647687875f), z, 1.0f);
-    const int q = (int)n;
     const bool odd = (q & 1) != 0;
     const unsigned ss = ((unsigned)q & 2u) << 30, sc = ((unsigned)(q + 1) & 2u) << 30;
     sn = __uint_as_float(__float_as_uint(odd ? c : s) ^ ss);
     cs = __uint_as_float(__float_as_uint(odd ? s : c) ^ sc);
+}
+
+// A phase in FP32, reduced to the nearest quarter turn exactly: about 24
+// operations in all, for phases that many samples share.
+__device__ inline void ft_sincos_shared(float t, float &sn, float &cs)
+{
+    const float n = rintf(4.0f * t);
+    ft_sincos_quarter((int)n, fmaf(-0.25f, n, t), sn, cs);
 }
 
 int check_atoms(const gt_atoms *a);

@@ -128,11 +128,12 @@ struct FzState {
     unsigned next, count[FZ_CLASSES];
 };
 
-// Phase tables and records.  Blocks below `tabs`: one wave per atom, its phase
-// table exp(-i x_c k) over the m0 + m1 + m2 grid coordinates, from FP64, the first
-// axis' entries times the amplitude (block 0 also finds the axes' pairing).
+// Phase tables and records.  Blocks below `tabs`: one wave per FZ_TAB entries of an
+// atom's phase table exp(-i x_c k) over the m0 + m1 + m2 grid coordinates, from FP64,
+// the first axis' entries times the amplitude (block 0 also finds the axes' pairing).
 // Later blocks: one thread per atom, its record (an isotropic atom's form |k|^2 /
 // r^2 as the diagonal U = Id / r).
+constexpr int FZ_TAB = 512;
 __global__ __launch_bounds__(256) void ft_atoms_kernel(gt_atoms A, gt_kgrid Kg, unsigned tabs, FtRec *recs,
                                                        FzState *state, float2 *__restrict__ tab)
 {
@@ -158,18 +159,19 @@ __global__ __launch_bounds__(256) void ft_atoms_kernel(gt_atoms A, gt_kgrid Kg, 
         }
     }
     const int lane = threadIdx.x & 63;
-    const int j = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int m = Kg.m0 + Kg.m1 + Kg.m2, parts = (m + FZ_TAB - 1) / FZ_TAB;
+    const unsigned w = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int j = (int)(w / (unsigned)parts), first = (int)(w % (unsigned)parts) * FZ_TAB;
     if (j >= A.n) return;
-    const int m = Kg.m0 + Kg.m1 + Kg.m2;
     const double x0 = A.x[(size_t)j * 3], x1 = A.x[(size_t)j * 3 + 1], x2 = A.x[(size_t)j * 3 + 2], amp = A.I[j];
     float2 *tj = tab + (size_t)j * m;
-    for (int i = lane; i < m; i += 64) {
+    for (int i = first + lane; i < min(first + FZ_TAB, m); i += 64) {
         const bool f0 = i < Kg.m0, f1 = i < Kg.m0 + Kg.m1;
         const float k = f0 ? Kg.k0[i] : (f1 ? Kg.k1[i - Kg.m0] : Kg.k2[i - Kg.m0 - Kg.m1]);
-        const double t = (f0 ? x0 : (f1 ? x1 : x2)) * (double)k / TWO_PI, w = f0 ? amp : 1.0;
+        const double t = (f0 ? x0 : (f1 ? x1 : x2)) * (double)k / TWO_PI, am = f0 ? amp : 1.0;
         double sn, cs;
         sincospi(2.0 * (t - rint(t)), &sn, &cs);
-        tj[i] = make_float2((float)(w * cs), (float)(-w * sn));
+        tj[i] = make_float2((float)(am * cs), (float)(-am * sn));
     }
 }
 
@@ -473,6 +475,10 @@ __global__ __launch_bounds__(256) void ft_rank_kernel(const FtRec *__restrict__ 
 // wave order: every sample's sum has an order fixed by the record order.
 constexpr int FP_THREADS = 256, FP_WAVES = 4, FP_CHUNK = 256, FP_PATCH = 8;
 
+// FINE: the phase in FP64 (of ranked, so at most FZ_MAX_ATOMS records), as
+// accurate as the tables; the others' is a sum of FP32 pairs through the hardware
+// sine and cosine.
+template <bool FINE>
 __global__ __launch_bounds__(FP_THREADS) void ft_patch_kernel(const FtRec *__restrict__ recs, int N, gt_kgrid Kg,
                                                               float2 *__restrict__ out, int e0, int e1, int e2,
                                                               int by_radius)
@@ -533,11 +539,19 @@ __global__ __launch_bounds__(FP_THREADS) void ft_patch_kernel(const FtRec *__res
                 const float v2 = fmaf(r.u[4], k1, fmaf(r.u[5], k0, r.u[2] * k2));
                 nq = fmaf(v0, v0, fmaf(v1, v1, v2 * v2));
             }
-            float err = 0.0f;
-            const float t01 = turns(r.xh[0], r.xl[0], k0, err) + turns(r.xh[1], r.xl[1], k1, err);
-            const float tt = (t01 + turns(r.xh[2], r.xl[2], k2, err)) + err;
             float sn, cs;
-            ft_sincos_turns(tt, sn, cs);
+            if (FINE) {
+                const double t = fma((double)r.xh[0] + (double)r.xl[0], (double)k0,
+                                     fma((double)r.xh[1] + (double)r.xl[1], (double)k1,
+                                         ((double)r.xh[2] + (double)r.xl[2]) * (double)k2));
+                const double q = rint(4.0 * t);
+                ft_sincos_quarter((int)(q - 4.0 * rint(0.25 * q)), (float)fma(-0.25, q, t), sn, cs);
+            } else {
+                float err = 0.0f;
+                const float t01 = turns(r.xh[0], r.xl[0], k0, err) + turns(r.xh[1], r.xl[1], k1, err);
+                const float tt = (t01 + turns(r.xh[2], r.xl[2], k2, err)) + err;
+                ft_sincos_turns(tt, sn, cs);
+            }
             const float a = nq < cut ? r.amp * __builtin_amdgcn_exp2f(-nq) : 0.0f;
             sr += (double)(a * cs);
             si += (double)(-a * sn);
@@ -611,10 +625,27 @@ static size_t ft_least(const gt_atoms *a)
 // Are the atoms evaluated with tables?  These grow with atoms x (m0 + m1 + m2)
 // and with the number of patches, so a long thin grid of many atoms would take
 // hundreds of times its output (16384 atoms on 2^20 x 1 x 1 samples: 137 GB of
-// tables for 8 MB).
+// tables for 8 MB).  And few atoms on a small grid are evaluated sooner without: the
+// patch kernel costs 2.1 ns per block of 1 x 8 x 8 samples and hardly anything per
+// atom until some 128 fill a chunk of records, the tables' kernels 10 us for their
+// cells and patches.  Call times with and without tables, us: 64^3 samples, 16 atoms
+// 28 and 20, 64 33 and 23, 256 44 and 45; 48^3, 64 atoms 31 and 20, 256 36 and 44;
+// 16^3, 128 atoms 18 and 20; 8 x 8 x 4096 (long tables), 64 atoms 27 and 20, 256 34
+// and 30, 512 42 and 51; beyond 4096 blocks: 80^3, 16 atoms 30 and 67, 256 x 256 x
+// 4, 16 atoms 24 and 30.
+static int ft_bits(const gt_kgrid *g, int *e)
+{
+    e[0] = ceil_log2(g->m0);
+    e[1] = ceil_log2((g->m1 + FP_PATCH - 1) / FP_PATCH);
+    e[2] = ceil_log2((g->m2 + FP_PATCH - 1) / FP_PATCH);
+    return e[0] + e[1] + e[2];
+}
 static bool ft_tabulated(const gt_atoms *a, const gt_kgrid *g)
 {
     if (a->n > FZ_MAX_ATOMS) return false;
+    int e[3];
+    const int bits = ft_bits(g, e);
+    if (bits <= 12 && a->n <= 128 + (1 << bits) / 64 + (g->m0 + g->m1 + g->m2) / 32) return false;
     const size_t out = (size_t)g->m0 * g->m1 * g->m2 * sizeof(float2);
     return ft_layout(a, g, ft_cells(g)).total <= std::max(FZ_MAX_BYTES, out);
 }
@@ -658,9 +689,8 @@ extern "C" int gt_ft_eval(const gt_atoms *atoms, const gt_kgrid *grid, float *ou
     FtRec *recs = (FtRec *)ws;
     const unsigned sb = (unsigned)((atoms->n + 255) / 256);
     // patches of 1 x 8 x 8 samples, numbered by Morton index over 2^e0 x 2^e1 x 2^e2 centre-out ranks
-    const int e[3] = {ceil_log2(grid->m0), ceil_log2((grid->m1 + FP_PATCH - 1) / FP_PATCH),
-                      ceil_log2((grid->m2 + FP_PATCH - 1) / FP_PATCH)};
-    GT_CHECK_ARG(e[0] + e[1] + e[2] <= 30, "gt_ft_eval: grid too large");
+    int e[3];
+    GT_CHECK_ARG(ft_bits(grid, e) <= 30, "gt_ft_eval: grid too large");
     if (tabulated) {
         const FzCells F = ft_cells(grid);
         const FtLayout l = ft_layout(atoms, grid, F);
@@ -671,7 +701,8 @@ extern "C" int gt_ft_eval(const gt_atoms *atoms, const gt_kgrid *grid, float *ou
         int4 *list = (int4 *)(w + l.list);
         float2 *tab = (float2 *)(w + l.tab);
         const size_t patches = (size_t)F.nb[0] * F.nb[1] * F.nb[2];
-        const unsigned tabs = (unsigned)((atoms->n + 3) / 4);
+        const size_t axes = (size_t)grid->m0 + grid->m1 + grid->m2;
+        const unsigned tabs = (unsigned)((atoms->n * ((axes + FZ_TAB - 1) / FZ_TAB) + 3) / 4);
         hipLaunchKernelGGL(ft_atoms_kernel, dim3(tabs + sb), dim3(256), 0, st, *atoms, *grid, tabs, recs, state, tab);
         prof_begin(st, GT_K_FT);
         hipLaunchKernelGGL(ft_bin_kernel, dim3(std::max(F.cells, 1024u)), dim3(FB_THREADS), 0, st, recs, atoms->n, *grid, F,
@@ -692,8 +723,12 @@ extern "C" int gt_ft_eval(const gt_atoms *atoms, const gt_kgrid *grid, float *ou
     }
     const unsigned blocks = 1u << (e[0] + e[1] + e[2]);
     prof_begin(st, GT_K_FT);
-    hipLaunchKernelGGL(ft_patch_kernel, dim3(blocks), dim3(FP_THREADS), 0, st, order, atoms->n, *grid, (float2 *)out,
-                       e[0], e[1], e[2], order != recs ? 1 : 0);
+    if (order != recs)
+        hipLaunchKernelGGL(ft_patch_kernel<true>, dim3(blocks), dim3(FP_THREADS), 0, st, order, atoms->n, *grid,
+                           (float2 *)out, e[0], e[1], e[2], 1);
+    else
+        hipLaunchKernelGGL(ft_patch_kernel<false>, dim3(blocks), dim3(FP_THREADS), 0, st, order, atoms->n, *grid,
+                           (float2 *)out, e[0], e[1], e[2], 0);
     prof_end(st, GT_K_FT);
     GT_HIP(hipGetLastError());
     return 0;

@@ -96,11 +96,12 @@ def test_point_spread_projection(gt, cuda, bad, n0):
 
 
 @pytest.mark.parametrize("bad", BAD)
-@pytest.mark.parametrize("planes", [False, True])
-def test_fourier(gt, cuda, bad, planes):
+@pytest.mark.parametrize("planes,m", [(False, (40, 48, 44)), (False, (70, 66, 40)), (True, (40, 48, 44))])
+def test_fourier(gt, cuda, bad, planes, m):
+    """Planes; a grid for so few atoms without and one with phase tables."""
     fo = importlib.import_module("2018_dictionary_tomography_amd.fourier")
     rng = np.random.default_rng(6)
-    n, at, m = 20, 7, (40, 48, 44)
+    n, at = 20, 7
     I, x = rng.uniform(0.5, 1.5, n), rng.uniform(-0.1, 0.1, (n, 3))
     r = np.concatenate((rng.uniform(0.3, 0.9, (n, 3)), rng.normal(0, 0.1, (n, 3))), 1)
     I[at] = bad

@@ -44,13 +44,14 @@ def test_renders_and_point_spread_projection(gt, cuda, width, op, call):
     _same(run(gt.AtomElement(space, xn, rn, In, device=cuda)).data, one)
 
 
-@pytest.mark.parametrize("planes", [False, True])
-def test_fourier(gt, cuda, planes):
+@pytest.mark.parametrize("planes,m", [(False, (24, 27, 30)), (False, (70, 66, 40)), (True, (24, 27, 30))])
+def test_fourier(gt, cuda, planes, m):
+    """Planes; a grid for so few atoms without and one with phase tables."""
     fo = importlib.import_module("2018_dictionary_tomography_amd.fourier")
     rng = np.random.default_rng(3)
     I, x = np.array([0.75]), rng.uniform(-0.2, 0.2, (1, 3))
     r = np.concatenate((rng.uniform(0.3, 0.9, (1, 3)), rng.normal(0, 0.1, (1, 3))), 1)
-    k = [np.arange(m, dtype=np.float32) - m // 2 for m in (24, 27, 30)]
+    k = [np.arange(c, dtype=np.float32) - c // 2 for c in m]
     S = k
     if planes:
         T, ortho = gt.spaces.axis_tilt_geometry(np.linspace(-1, 1, 3), [0, 1, 0], ref=np.array([1.0, 0, 0]))
