@@ -324,9 +324,8 @@ __global__ __launch_bounds__(64 * KE_WAVES) void kp_rect_kernel(const KpRec<floa
     __shared__ double2 red[KE_WAVES / 2][KE_R][64];
     const int tilesR = (P.m0 + KE_ROWS - 1) / KE_ROWS, tilesC = (P.m1 + KE_COLS - 1) / KE_COLS;
     const int a = (int)(blockIdx.x % (unsigned)P.nA);
-    const int e[3] = {e0, e1, 0};
-    int t[3];
-    morton_ranks(blockIdx.x / (unsigned)P.nA, e, t);
+    int t[2];
+    morton_ranks2(blockIdx.x / (unsigned)P.nA, e0, e1, t);
     if (t[0] >= tilesR || t[1] >= tilesC) return;  // whole block: no tile of this rank
     const int row0 = centre_out(t[0], tilesR) * KE_ROWS, col0 = centre_out(t[1], tilesC) * KE_COLS;
     const int row1 = min(row0 + KE_ROWS - 1, P.m0 - 1), col1 = min(col0 + KE_COLS - 1, P.m1 - 1);

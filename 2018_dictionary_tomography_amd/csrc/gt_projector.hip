@@ -188,9 +188,8 @@ __global__ __launch_bounds__(F3_WAVES * 64) __attribute__((amdgpu_waves_per_eu(8
     __shared__ F3Tab tab[F3_WAVES];
     const int tilesR = (n0 + TILE_ROWS - 1) / TILE_ROWS, tilesC = (n1 + TILE_COLS - 1) / TILE_COLS;
     const int a = (int)(blockIdx.x % (unsigned)nA);
-    const int e[3] = {e0, e1, 0};
-    int t[3];
-    morton_ranks(blockIdx.x / (unsigned)nA, e, t);
+    int t[2];
+    morton_ranks2(blockIdx.x / (unsigned)nA, e0, e1, t);
     if (t[0] >= tilesR || t[1] >= tilesC) return;  // whole block: no tile of this rank
     const int row0 = centre_out(t[0], tilesR) * TILE_ROWS, col0 = centre_out(t[1], tilesC) * TILE_COLS;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);

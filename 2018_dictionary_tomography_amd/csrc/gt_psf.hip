@@ -776,9 +776,8 @@ __global__ __launch_bounds__(PF_WAVES * 64) __attribute__((amdgpu_waves_per_eu(5
     __shared__ double part[PF_WAVES - PF_RECTS][2][64];
     const int tilesR = (n0 + PF_ROWS - 1) / PF_ROWS, tilesC = (n1 + PF_COLS - 1) / PF_COLS;
     const int a = (int)(blockIdx.x % (unsigned)nA);
-    const int e[3] = {e0, e1, 0};
-    int t[3];
-    morton_ranks(blockIdx.x / (unsigned)nA, e, t);
+    int t[2];
+    morton_ranks2(blockIdx.x / (unsigned)nA, e0, e1, t);
     if (t[0] >= tilesR || t[1] >= tilesC) return;  // whole block: no tile of this rank
     const int row0 = centre_out(t[0], tilesR) * PF_ROWS, col0 = centre_out(t[1], tilesC) * PF_COLS;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -955,9 +954,8 @@ __global__ __launch_bounds__(256) void psf_forward_kernel(const PsfRec *__restri
     if (K == 2) {
         const int ntr = (n0 + 15) / 16, ntc = (n1 + 15) / 16;
         a = (int)(blockIdx.x % (unsigned)nA);
-        const int e[3] = {e0, e1, 0};
-        int t[3];
-        morton_ranks(blockIdx.x / (unsigned)nA, e, t);
+        int t[2];
+        morton_ranks2(blockIdx.x / (unsigned)nA, e0, e1, t);
         if (t[0] >= ntr || t[1] >= ntc) return;  // whole block: no tile of this rank
         const int tr = centre_out(t[0], ntr), tcc = centre_out(t[1], ntc);
         i0 = tr * 16 + (int)(threadIdx.x >> 4);
