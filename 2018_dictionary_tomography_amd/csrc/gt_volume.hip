@@ -11,6 +11,8 @@
 // atoms whose support meets them; the 2D render gives each block a tile,
 // stages the atoms whose box meets it in LDS (in atom order), and accumulates
 // 4 voxels per lane with Kahan sums.
+#include <algorithm>
+
 #include "gt_common.h"
 
 namespace gt {
@@ -139,7 +141,10 @@ constexpr int VCHUNK = 128;
 constexpr int V3_PARTS = 2, V3_GROUPS = 2, V3_WAVES = V3_PARTS * V3_GROUPS, V3_THREADS = 64 * V3_WAVES;
 constexpr int V3_N1 = V3_PARTS == 4 ? 2 : 1, V3_N2 = V3_PARTS / V3_N1;  // parts per axis
 constexpr int V3_B1 = 8 * V3_N1, V3_B2 = 8 * V3_N2;
+constexpr unsigned V3_BLOCKS = 16384;
 
+// SPARSE: a block walks the ranks, its own and every gridDim.x-th after it.
+template <bool SPARSE>
 __global__ __launch_bounds__(V3_THREADS) void volume3_kernel(const VolRec *__restrict__ recs, int N, gt_vol V,
                                                              float *__restrict__ u, int e0, int e1, int e2)
 {
@@ -151,95 +156,149 @@ __global__ __launch_bounds__(V3_THREADS) void volume3_kernel(const VolRec *__res
     const int sub = wave % V3_PARTS, grp = wave / V3_PARTS;
     const int nb0 = (V.m0 + 3) / 4, nb1 = (V.m1 + V3_B1 - 1) / V3_B1, nb2 = (V.m2 + V3_B2 - 1) / V3_B2;
     const int e[3] = {e0, e1, e2};
-    int t[3];
-    morton_ranks(blockIdx.x, e, t);
-    if (t[0] >= nb0 || t[1] >= nb1 || t[2] >= nb2) return;  // whole block: no brick of this rank
-    const int b0 = centre_out(t[0], nb0) * 4, b1 = centre_out(t[1], nb1) * V3_B1, b2 = centre_out(t[2], nb2) * V3_B2;
-    const int j1 = b1 + 8 * (sub / V3_N2) + (lane >> 3), j2 = b2 + 8 * (sub % V3_N2) + (lane & 7);
-    const float y1 = V.y1[min(j1, V.m1 - 1)], y2 = V.y2[min(j2, V.m2 - 1)];
-    float y0[4];
+    unsigned rank = blockIdx.x;
+    do {
+        int t[3];
+        morton_ranks(rank, e, t);
+        if (t[0] >= nb0 || t[1] >= nb1 || t[2] >= nb2) continue;  // whole block: no brick of this rank
+        const int b0 = centre_out(t[0], nb0) * 4, b1 = centre_out(t[1], nb1) * V3_B1, b2 = centre_out(t[2], nb2) * V3_B2;
+        const int j1 = b1 + 8 * (sub / V3_N2) + (lane >> 3), j2 = b2 + 8 * (sub % V3_N2) + (lane & 7);
+        const float y1 = V.y1[min(j1, V.m1 - 1)], y2 = V.y2[min(j2, V.m2 - 1)];
+        float y0[4];
 #pragma unroll
-    for (int k = 0; k < 4; k++) y0[k] = V.y0[min(b0 + k, V.m0 - 1)];
-    // centre and half extent of the waves' voxels per axis
-    float c0, h0, c1[2], h1[2], c2[2], h2[2];
-    {
-        const float za = V.y0[b0], zb = V.y0[min(b0 + 3, V.m0 - 1)];
-        c0 = 0.5f * (za + zb);
-        h0 = 0.5f * (zb - za);
+        for (int k = 0; k < 4; k++) y0[k] = V.y0[min(b0 + k, V.m0 - 1)];
+        // centre and half extent of the waves' voxels per axis
+        float c0, h0, c1[2], h1[2], c2[2], h2[2];
+        {
+            const float za = V.y0[b0], zb = V.y0[min(b0 + 3, V.m0 - 1)];
+            c0 = 0.5f * (za + zb);
+            h0 = 0.5f * (zb - za);
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const float ya = V.y1[min(b1 + 8 * h, V.m1 - 1)], yb = V.y1[min(b1 + 8 * h + 7, V.m1 - 1)];
-            const float xa = V.y2[min(b2 + 8 * h, V.m2 - 1)], xb = V.y2[min(b2 + 8 * h + 7, V.m2 - 1)];
-            c1[h] = 0.5f * (ya + yb);
-            h1[h] = 0.5f * (yb - ya);
-            c2[h] = 0.5f * (xa + xb);
-            h2[h] = 0.5f * (xb - xa);
-        }
-    }
-    const float kap = (float)KAPPA;
-    double s[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int base = 0; base < N; base += V3_THREADS) {
-        unsigned mask = 0;
-        const int j = base + (int)threadIdx.x;
-        if (j < N) {
-            const float4 *src = reinterpret_cast<const float4 *>(recs + j);
-            // amp, xh[0..2] | xl[0..2], u0 | u1..u4 | u5, pad ; lo[3], hi[3]
-            const float4 f0 = src[0], f1 = src[1], f2 = src[2], f3 = src[3];
-            const int4 bx = reinterpret_cast<const int4 *>(src)[4];
-            const int2 by = reinterpret_cast<const int2 *>(src)[10];
-            if ((int)(bx.x <= b0 + 3) & (int)(bx.w >= b0) & (int)(bx.y <= b1 + V3_B1 - 1) & (int)(by.x >= b1) &
-                (int)(bx.z <= b2 + V3_B2 - 1) & (int)(by.y >= b2)) {
-                const float d0 = (c0 - f0.y) - f1.x;
-#pragma unroll
-                for (int w = 0; w < V3_PARTS; w++) {
-                    const int q1 = w / V3_N2, q2 = w % V3_N2, a1 = b1 + 8 * q1, a2 = b2 + 8 * q2;
-                    const float d1 = (c1[q1] - f0.z) - f1.y, d2 = (c2[q2] - f0.w) - f1.z;
-                    const float v0 = fmaf(f1.w, d0, fmaf(f2.z, d1, f3.x * d2)), v1 = fmaf(f2.x, d1, f2.w * d2);
-                    const float v2 = f2.y * d2;
-                    const float n2 = fmaf(v0, v0, fmaf(v1, v1, v2 * v2));
-                    const float g0 = f1.w * v0, g1 = fmaf(f2.z, v0, f2.x * v1);
-                    const float g2 = fmaf(f3.x, v0, fmaf(f2.w, v1, f2.y * v2));
-                    const float reach = fmaf(fabsf(g0), h0, fmaf(fabsf(g1), h1[q1], fabsf(g2) * h2[q2]));
-                    // NaN keeps the record
-                    const bool apart =
-                        V.sorted && n2 * (1.0f - 1e-4f) - reach > ((float)SQRT_NEG_KAPPA + 1e-2f) * sqrtf(n2);
-                    if (bx.y <= a1 + 7 && by.x >= a1 && bx.z <= a2 + 7 && by.y >= a2 && !apart) mask |= 1u << w;
-                }
+            for (int h = 0; h < 2; h++) {
+                const float ya = V.y1[min(b1 + 8 * h, V.m1 - 1)], yb = V.y1[min(b1 + 8 * h + 7, V.m1 - 1)];
+                const float xa = V.y2[min(b2 + 8 * h, V.m2 - 1)], xb = V.y2[min(b2 + 8 * h + 7, V.m2 - 1)];
+                c1[h] = 0.5f * (ya + yb);
+                h1[h] = 0.5f * (yb - ya);
+                c2[h] = 0.5f * (xa + xb);
+                h2[h] = 0.5f * (xb - xa);
             }
         }
-        wave_lists<V3_WAVES, V3_PARTS>(mask, wl, cnt, wlen);
-        const int len = __builtin_amdgcn_readfirstlane(wlen[sub]);
-        for (int q = grp; q < len; q += V3_GROUPS) {
-            smem<VolRec> *r = scalar_ptr(recs) + (base + __builtin_amdgcn_readfirstlane((int)wl[sub][q]));
-            const float d1 = (y1 - r->xh[1]) - r->xl[1], d2 = (y2 - r->xh[2]) - r->xl[2];
-            const float a0 = fmaf(r->u[3], d1, r->u[5] * d2);
-            const float v1 = fmaf(r->u[1], d1, r->u[4] * d2), v2 = r->u[2] * d2;
-            const float c = -fmaf(v1, v1, v2 * v2);
-            const float amp = r->amp, u0 = r->u[0], xh = r->xh[0], xl = r->xl[0];
+        const float kap = (float)KAPPA;
+        double s[4] = {0.0, 0.0, 0.0, 0.0};
+        for (int base = 0; base < N; base += V3_THREADS) {
+            unsigned mask = 0;
+            const int j = base + (int)threadIdx.x;
+            if (j < N) {
+                const float4 *src = reinterpret_cast<const float4 *>(recs + j);
+                // amp, xh[0..2] | xl[0..2], u0 | u1..u4 | u5, pad ; lo[3], hi[3]
+                const float4 f0 = src[0], f1 = src[1], f2 = src[2], f3 = src[3];
+                const int4 bx = reinterpret_cast<const int4 *>(src)[4];
+                const int2 by = reinterpret_cast<const int2 *>(src)[10];
+                if ((int)(bx.x <= b0 + 3) & (int)(bx.w >= b0) & (int)(bx.y <= b1 + V3_B1 - 1) & (int)(by.x >= b1) &
+                    (int)(bx.z <= b2 + V3_B2 - 1) & (int)(by.y >= b2)) {
+                    const float d0 = (c0 - f0.y) - f1.x;
+#pragma unroll
+                    for (int w = 0; w < V3_PARTS; w++) {
+                        const int q1 = w / V3_N2, q2 = w % V3_N2, a1 = b1 + 8 * q1, a2 = b2 + 8 * q2;
+                        const float d1 = (c1[q1] - f0.z) - f1.y, d2 = (c2[q2] - f0.w) - f1.z;
+                        const float v0 = fmaf(f1.w, d0, fmaf(f2.z, d1, f3.x * d2)), v1 = fmaf(f2.x, d1, f2.w * d2);
+                        const float v2 = f2.y * d2;
+                        const float n2 = fmaf(v0, v0, fmaf(v1, v1, v2 * v2));
+                        const float g0 = f1.w * v0, g1 = fmaf(f2.z, v0, f2.x * v1);
+                        const float g2 = fmaf(f3.x, v0, fmaf(f2.w, v1, f2.y * v2));
+                        const float reach = fmaf(fabsf(g0), h0, fmaf(fabsf(g1), h1[q1], fabsf(g2) * h2[q2]));
+                        // NaN keeps the record
+                        const bool apart =
+                            V.sorted && n2 * (1.0f - 1e-4f) - reach > ((float)SQRT_NEG_KAPPA + 1e-2f) * sqrtf(n2);
+                        if (bx.y <= a1 + 7 && by.x >= a1 && bx.z <= a2 + 7 && by.y >= a2 && !apart) mask |= 1u << w;
+                    }
+                }
+            }
+            wave_lists<V3_WAVES, V3_PARTS>(mask, wl, cnt, wlen);
+            const int len = __builtin_amdgcn_readfirstlane(wlen[sub]);
+            for (int q = grp; q < len; q += V3_GROUPS) {
+                smem<VolRec> *r = scalar_ptr(recs) + (base + __builtin_amdgcn_readfirstlane((int)wl[sub][q]));
+                const float d1 = (y1 - r->xh[1]) - r->xl[1], d2 = (y2 - r->xh[2]) - r->xl[2];
+                const float a0 = fmaf(r->u[3], d1, r->u[5] * d2);
+                const float v1 = fmaf(r->u[1], d1, r->u[4] * d2), v2 = r->u[2] * d2;
+                const float c = -fmaf(v1, v1, v2 * v2);
+                const float amp = r->amp, u0 = r->u[0], xh = r->xh[0], xl = r->xl[0];
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const float v0 = fmaf(u0, (y0[k] - xh) - xl, a0);
+                    const float ex = fmaf(-v0, v0, c);
+                    // the term is chosen, not its profile: 0 times an infinite amplitude is no 0
+                    const float v = amp * __builtin_amdgcn_exp2f(ex);
+                    s[k] += (double)(ex >= kap ? v : 0.0f);
+                }
+            }
+            __syncthreads();
+        }
+        // the groups' totals, in group order
+        if (grp > 0)
+#pragma unroll
+            for (int k = 0; k < 4; k++) red[grp - 1][sub][k][lane] = s[k];
+        __syncthreads();
+        if (grp > 0) continue;  // (red is written again after the next brick's barriers)
+        for (int g = 0; g < V3_GROUPS - 1; g++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) s[k] += red[g][sub][k][lane];
+        if (j1 < V.m1 && j2 < V.m2)
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                if (b0 + k < V.m0) u[((size_t)(b0 + k) * V.m1 + j1) * V.m2 + j2] = (float)s[k];
+    } while (SPARSE && (rank += gridDim.x) < (1u << (e0 + e1 + e2)));
+}
+
+// 3D, few atoms: block = brick of 4 (j0, one per wave) x 4 (j1, per lane) x 64 (j2, lane).
+__global__ __launch_bounds__(256) void volume3_rows_kernel(const VolRec *__restrict__ recs, int N, gt_vol V,
+                                                           float *__restrict__ u)
+{
+    __shared__ VolRec list[VCHUNK];
+    __shared__ int wcnt[4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int nb2 = (V.m2 + 63) / 64, nb1 = (V.m1 + 3) / 4;
+    int b = blockIdx.x;
+    const int bb2 = b % nb2;
+    b /= nb2;
+    const int bb1 = b % nb1;
+    const int bb0 = b / nb1;
+    const int j0 = bb0 * 4 + wave, j1b = bb1 * 4, j2 = bb2 * 64 + lane;
+    const int blo[3] = {bb0 * 4, j1b, bb2 * 64};
+    const int bhi[3] = {min(bb0 * 4 + 3, V.m0 - 1), min(j1b + 3, V.m1 - 1), min(bb2 * 64 + 63, V.m2 - 1)};
+    const float y0 = V.y0[min(j0, V.m0 - 1)];
+    const float y2 = V.y2[min(j2, V.m2 - 1)];
+    float y1[4];
+    double s[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < 4; k++) y1[k] = V.y1[min(j1b + k, V.m1 - 1)];
+    for (int base = 0; base < N; base += VCHUNK) {
+        // stage with the first VCHUNK threads only
+        const int total = vol_stage(recs, base, min(N, base + VCHUNK), blo, bhi, list, wcnt);
+        for (int e = 0; e < total; e++) {
+            const VolRec &r = list[e];
+            if (r.lo[0] > j0 || r.hi[0] < j0) continue;
+            const float d0 = (y0 - r.xh[0]) - r.xl[0];
+            const float d2 = (y2 - r.xh[2]) - r.xl[2];
+            const float a0 = fmaf(r.u[0], d0, r.u[5] * d2);
+            const float a1 = r.u[4] * d2;
+            const float u2 = r.u[2] * d2;
+            const float c2 = u2 * u2;
 #pragma unroll
             for (int k = 0; k < 4; k++) {
-                const float v0 = fmaf(u0, (y0[k] - xh) - xl, a0);
-                const float ex = fmaf(-v0, v0, c);
-                // the term is chosen, not its profile: 0 times an infinite amplitude is no 0
-                const float v = amp * __builtin_amdgcn_exp2f(ex);
-                s[k] += (double)(ex >= kap ? v : 0.0f);
+                const float d1 = (y1[k] - r.xh[1]) - r.xl[1];
+                const float u0 = fmaf(r.u[3], d1, a0);
+                const float u1 = fmaf(r.u[1], d1, a1);
+                const float q = -fmaf(u0, u0, fmaf(u1, u1, c2));
+                if (q >= (float)KAPPA) s[k] += (double)(r.amp * __builtin_amdgcn_exp2f(q));
             }
         }
         __syncthreads();
     }
-    // the groups' totals, in group order
-    if (grp > 0)
-#pragma unroll
-        for (int k = 0; k < 4; k++) red[grp - 1][sub][k][lane] = s[k];
-    __syncthreads();
-    if (grp > 0) return;
-    for (int g = 0; g < V3_GROUPS - 1; g++)
-#pragma unroll
-        for (int k = 0; k < 4; k++) s[k] += red[g][sub][k][lane];
-    if (j1 < V.m1 && j2 < V.m2)
+    if (j0 < V.m0 && j2 < V.m2)
 #pragma unroll
         for (int k = 0; k < 4; k++)
-            if (b0 + k < V.m0) u[((size_t)(b0 + k) * V.m1 + j1) * V.m2 + j2] = (float)s[k];
+            if (j1b + k < V.m1) u[((size_t)j0 * V.m1 + j1b + k) * V.m2 + j2] = (float)s[k];
 }
 
 // 2D: block tile = 16 rows (j0, 4 per lane, 4 waves) x 64 cols (j1, lane).
@@ -337,8 +396,31 @@ extern "C" int gt_volume(const gt_atoms *atoms, const gt_vol *vol, float *u, voi
                           ceil_log2((V.m2 + V3_B2 - 1) / V3_B2)};
         GT_CHECK_ARG(e[0] + e[1] + e[2] <= 30, "gt_volume: grid too large");
         prof_begin(st, GT_K_VOLUME);
-        hipLaunchKernelGGL(volume3_kernel, dim3(1u << (e[0] + e[1] + e[2])), dim3(V3_THREADS), 0, st, recs, atoms->n,
-                           V, u, e[0], e[1], e[2]);
+        const unsigned ranks = 1u << (e[0] + e[1] + e[2]);
+        const unsigned long long bricks =
+            (unsigned long long)((V.m0 + 3) / 4) * ((V.m1 + V3_B1 - 1) / V3_B1) * ((V.m2 + V3_B2 - 1) / V3_B2);
+        const bool sparse = 2 * bricks < ranks;  // most ranks are no bricks
+        // Few atoms on many bricks: most see none, and rows of 64 voxels are written
+        // faster (where there are such rows).  Call times, us, bricks and rows: 256^3
+        // voxels, 1 atom 53 and 24, 32 68 and 54, 64 73 and 78; 512^3, 32 450 and 303, 64
+        // 482 and 482; sparse ones, with the blocks below, 384^3, 64 219 and 179, 128 309
+        // and 303; 320^3, 128 197 and 188; up to 4096 ranks (128^3, 32 atoms) 19 and 18;
+        // rows of 4 voxels (512 x 512 x 4, 32 atoms) 24 and 57.
+        if (V.m2 >= 64 && ranks > 4096 && atoms->n < (sparse && ranks > 32768 ? 128 : 64)) {
+            const unsigned long long rows = (unsigned long long)((V.m0 + 3) / 4) * ((V.m1 + 3) / 4) * ((V.m2 + 63) / 64);
+            GT_CHECK_ARG(rows < (1ull << 31), "gt_volume: grid too large");
+            hipLaunchKernelGGL(volume3_rows_kernel, dim3((unsigned)rows), dim3(256), 0, st, recs, atoms->n, V, u);
+        } else {
+            // sparse ranks are walked by V3_BLOCKS blocks: starting a block for each
+            // costs 1 ns (384^3, 64 atoms 259 us, now 219); with bricks for most ranks
+            // a block each is 3 to 10% faster, it starts when another ends
+            if (sparse)
+                hipLaunchKernelGGL(volume3_kernel<true>, dim3(std::min(ranks, V3_BLOCKS)), dim3(V3_THREADS), 0, st, recs,
+                                   atoms->n, V, u, e[0], e[1], e[2]);
+            else
+                hipLaunchKernelGGL(volume3_kernel<false>, dim3(ranks), dim3(V3_THREADS), 0, st, recs, atoms->n, V, u, e[0],
+                                   e[1], e[2]);
+        }
         prof_end(st, GT_K_VOLUME);
     } else {
         hipLaunchKernelGGL(vol_setup_kernel<2>, dim3(sb), dim3(256), 0, st, *atoms, V, recs);
