@@ -237,6 +237,13 @@ __device__ inline void ft_sincos_quarter(int q, float r, float &sn, float &cs)
     cs = __uint_as_float(__float_as_uint(odd ? s : c) ^ sc);
 }
 
+// A phase in FP64, of any size.
+__device__ inline void ft_sincos_fine(double t, float &sn, float &cs)
+{
+    const double q = rint(4.0 * t);
+    ft_sincos_quarter((int)(q - 4.0 * rint(0.25 * q)), (float)fma(-0.25, q, t), sn, cs);
+}
+
 // A phase in FP32, reduced to the nearest quarter turn exactly: about 24
 // operations in all, for phases that many samples share.
 __device__ inline void ft_sincos_shared(float t, float &sn, float &cs)

@@ -544,8 +544,7 @@ __global__ __launch_bounds__(FP_THREADS) void ft_patch_kernel(const FtRec *__res
                 const double t = fma((double)r.xh[0] + (double)r.xl[0], (double)k0,
                                      fma((double)r.xh[1] + (double)r.xl[1], (double)k1,
                                          ((double)r.xh[2] + (double)r.xl[2]) * (double)k2));
-                const double q = rint(4.0 * t);
-                ft_sincos_quarter((int)(q - 4.0 * rint(0.25 * q)), (float)fma(-0.25, q, t), sn, cs);
+                ft_sincos_fine(t, sn, cs);
             } else {
                 float err = 0.0f;
                 const float t01 = turns(r.xh[0], r.xl[0], k0, err) + turns(r.xh[1], r.xl[1], k1, err);

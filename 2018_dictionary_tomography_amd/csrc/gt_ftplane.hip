@@ -220,7 +220,8 @@ constexpr int KP_CHUNK = 128;
 // Block b takes angle b % nA and the tile of centre-out rank b / nA: the tiles
 // near k = 0 meet the most atoms and start first, the light outer ones fill
 // the tail.
-template <typename R>
+// FINE (FP32): the phase in FP64, as accurate as kp_rect_kernel's.
+template <typename R, bool FINE>
 __global__ __launch_bounds__(256) void kp_eval_kernel(const KpRec<R> *__restrict__ recs, int N, KpDev<R> P,
                                                       double cut, R *__restrict__ out)
 {
@@ -267,10 +268,16 @@ __global__ __launch_bounds__(256) void kp_eval_kernel(const KpRec<R> *__restrict
             const R ex = p0 * (r.q[0] * p0 + r.q[1] * p1) + r.q[2] * p1 * p1;
             if (!(ex > cutlog)) continue;
             if constexpr (sizeof(R) == 4) {
-                float err = 0.0f;
-                const float t = kp_turns(r.ch[0], r.cl[0], p0, err) + kp_turns(r.ch[1], r.cl[1], p1, err) + err;
                 float sn, cs;
-                ft_sincos_turns(t, sn, cs);
+                if (FINE) {
+                    const double t = fma((double)r.ch[0] + (double)r.cl[0], (double)p0,
+                                         ((double)r.ch[1] + (double)r.cl[1]) * (double)p1);
+                    ft_sincos_fine(t, sn, cs);
+                } else {
+                    float err = 0.0f;
+                    const float t = kp_turns(r.ch[0], r.cl[0], p0, err) + kp_turns(r.ch[1], r.cl[1], p1, err) + err;
+                    ft_sincos_turns(t, sn, cs);
+                }
                 const float am = r.amp * __builtin_amdgcn_exp2f(ex);
                 kp_kahan(sr, cr, am * cs);
                 kp_kahan(si, ci, -am * sn);
@@ -885,14 +892,20 @@ int kp_eval(const AT *atoms, const KP *planes, R *out, void *ws, size_t ws_bytes
     GT_CHECK_ARG(blocks < (1L << 31), "%s: too many samples", who);
     prof_begin(st, GT_K_FT);
     if constexpr (sizeof(R) == 4) {
-        // two sample axes: rectangles, at every size (1000 atoms, 60 angles: 0.09
-        // against 0.36 ms at 8 x 8 and at 128 x 8 samples, 0.17 against 0.47 at
-        // 128 x 128); lines keep the 256-sample tiles
+        // two sample axes: rectangles (1000 atoms, 60 angles: 0.09 against 0.36 ms at 8
+        // x 8 and at 128 x 8 samples, 0.17 against 0.47 at 128 x 128), but for few atoms
+        // on large planes: a rectangle costs a fixed 7 ns, most meet no atom. Calls of
+        // 60 angles, us, rectangles and tiles: 128^2 samples, 32 atoms 69 and 72; 256^2,
+        // 32 atoms 99 and 93, 64 103 and 123; 512^2, 1 atom 209 and 115, 64 216 and 210,
+        // 128 223 and 292; 20 angles of 1024^2, 128 atoms 276 and 208, 256 283 and 304.
+        // Lines keep the 256-sample tiles.
+        const long plane = (long)planes->m0 * planes->m1;
+        const bool few = plane > 16384 && atoms->n <= 32 + plane / 8192;
         if (planes->form != GT_KP_2D_LINE) {
             const int e0 = ceil_log2((planes->m0 + KE_ROWS - 1) / KE_ROWS);
             const int e1 = ceil_log2((planes->m1 + KE_COLS - 1) / KE_COLS);
             const unsigned long long rects = (unsigned long long)planes->nA << (e0 + e1);
-            if (rects < (1ull << 31)) {
+            if (rects < (1ull << 31) && !few) {
                 hipLaunchKernelGGL(kp_rect_kernel, dim3((unsigned)rects), dim3(64 * KE_WAVES), 0, st, recs, pairing,
                                    atoms->n, P, (float)(-0.5 * KP_LOG2E * cut),
                                    (float2 *)out, e0, e1);
@@ -902,7 +915,11 @@ int kp_eval(const AT *atoms, const KP *planes, R *out, void *ws, size_t ws_bytes
             }
         }
     }
-    hipLaunchKernelGGL(kp_eval_kernel<R>, dim3((unsigned)blocks), dim3(256), 0, st, recs, atoms->n, P, cut, out);
+    if (planes->form != GT_KP_2D_LINE)
+        hipLaunchKernelGGL((kp_eval_kernel<R, true>), dim3((unsigned)blocks), dim3(256), 0, st, recs, atoms->n, P, cut, out);
+    else
+        hipLaunchKernelGGL((kp_eval_kernel<R, false>), dim3((unsigned)blocks), dim3(256), 0, st, recs, atoms->n, P, cut,
+                           out);
     prof_end(st, GT_K_FT);
     GT_HIP(hipGetLastError());
     return 0;
