@@ -937,7 +937,7 @@ __global__ __launch_bounds__(PF_WAVES * 64) __attribute__((amdgpu_waves_per_eu(5
     }
 }
 
-// Forward of the sampled rule and of 1D detectors: block = (angle, 16 x 16
+// Forward of few atoms, of the sampled rule and of 1D detectors: block = (angle, 16 x 16
 // pixels) for 2D detectors, numbered centre tiles first (block b: angle b % nA, tile of Morton rank b / nA over the
 // centre-out tile ranks, 2^e0 x 2^e1), or (angle = blockIdx.y, 256 pixels) for
 // 1D ones.
@@ -1830,7 +1830,11 @@ extern "C" int gt_psf_forward_rule(const gt_atoms *atoms, const gt_geom *geom, i
         set_error("gt_psf_forward: atoms or geometry is NULL");
         return GT_EINVAL;
     }
-    const bool whole = atoms->dim == 3 && rule == GT_PSF_EXACT;
+    // Few atoms (the host-driven fitters project one at a time): most tiles meet none,
+    // and psf_project_kernel's cost a fixed time more. 60 angles, us, it and
+    // psf_forward_kernel: 512^2 pixels, 1 atom 119 and 73, 4 147 and 103, 6 170 and 153, 8
+    // 169 and 168, 16 200 and 324; 256^2, 1 38 and 26, 6 53 and 50, 8 53 and 55.
+    const bool whole = atoms->dim == 3 && rule == GT_PSF_EXACT && atoms->n > 6;
     PsfNode2 *nodes = whole ? (PsfNode2 *)((char *)ws + psf_rec_bytes(atoms, geom)) : nullptr;
     if ((rc = psf_prepare(atoms, geom, rule, ws, ws_bytes, gt_psf_forward_workspace(atoms, geom), st,
                           "gt_psf_forward", nodes)))
@@ -1856,8 +1860,12 @@ extern "C" int gt_psf_forward_rule(const gt_atoms *atoms, const gt_geom *geom, i
         const int e0 = ceil_log2((geom->n0 + 15) / 16), e1 = ceil_log2((n1 + 15) / 16);
         GT_CHECK_ARG(((unsigned long long)geom->nA << (e0 + e1)) < (1ull << 31), "gt_psf_forward: too many tiles");
         const dim3 grid((unsigned)((unsigned long long)geom->nA << (e0 + e1)));
-        hipLaunchKernelGGL((psf_forward_kernel<2, GT_PSF_SAMPLED>), grid, dim3(256), 0, st, recs, atoms->n, geom->nA,
-                           geom->n0, n1, geom->p0, geom->p1, R, e0, e1);
+        if (rule == GT_PSF_EXACT)
+            hipLaunchKernelGGL((psf_forward_kernel<2, GT_PSF_EXACT>), grid, dim3(256), 0, st, recs, atoms->n, geom->nA,
+                               geom->n0, n1, geom->p0, geom->p1, R, e0, e1);
+        else
+            hipLaunchKernelGGL((psf_forward_kernel<2, GT_PSF_SAMPLED>), grid, dim3(256), 0, st, recs, atoms->n, geom->nA,
+                               geom->n0, n1, geom->p0, geom->p1, R, e0, e1);
     } else {
         const dim3 grid((unsigned)((geom->n0 + 255) / 256), (unsigned)geom->nA);
         if (rule == GT_PSF_SAMPLED)

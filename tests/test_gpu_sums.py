@@ -1,6 +1,6 @@
 """The sums over atoms are carried in FP64: 96 copies of one atom, their
 amplitudes 2^20, 1 and -2^20 times one value in any order, give 32 times the
-output of the one atom, bit for bit.  (A factor of a power of two scales every
+output of the one atom (among 95 of amplitude 0), bit for bit.  (A factor of a power of two scales every
 term exactly, and the FP64 sum of terms of 24 bits, at most 26 binary places
 apart, is exact in any order; a sum in 24 bits is off by a sixteenth of a term at
 each step.)
@@ -15,9 +15,10 @@ pytestmark = pytest.mark.gpu
 
 
 def _copies(rng, I, x, r):
+    """The 96 copies, and as many of which all but one have amplitude 0."""
     f = np.tile([2.0 ** 20, 1.0, -(2.0 ** 20)], 32)
     rng.shuffle(f)
-    return I * f, np.tile(x, (96, 1)), np.tile(r, (96, 1))
+    return [(I * a, np.tile(x, (96, 1)), np.tile(r, (96, 1))) for a in (f, np.arange(96) == 50)]
 
 
 def _same(many, one):
@@ -39,9 +40,7 @@ def test_renders_and_point_spread_projection(gt, cuda, width, op, call):
     P = gt.ProjSpace(orientations=T, ortho=ortho, detector=[gt.cell_centres(-1, 1, m) for m in (40, 37)])
     A = getattr(gt, op)(space, gt.VolSpace([gt.cell_centres(-1, 1, m) for m in (28, 25, 30)]), P)
     run = A.discretise if call == "volume" else A
-    one = run(gt.AtomElement(space, x, r, I, device=cuda)).data
-    In, xn, rn = _copies(rng, I, x, r)
-    _same(run(gt.AtomElement(space, xn, rn, In, device=cuda)).data, one)
+    _same(*[run(gt.AtomElement(space, xn, rn, In, device=cuda)).data for In, xn, rn in _copies(rng, I, x, r)])
 
 
 @pytest.mark.parametrize("planes,m", [(False, (24, 27, 30)), (False, (70, 66, 40)), (True, (24, 27, 30))])
@@ -56,6 +55,5 @@ def test_fourier(gt, cuda, planes, m):
     if planes:
         T, ortho = gt.spaces.axis_tilt_geometry(np.linspace(-1, 1, 3), [0, 1, 0], ref=np.array([1.0, 0, 0]))
         S = (k[1], k[2], *ortho)
-    one = fo.evaluate(fo.FTAtoms(I, x, r, device=cuda), S)
-    In, xn, rn = _copies(rng, I, x, r)
-    _same(torch.view_as_real(fo.evaluate(fo.FTAtoms(In, xn, rn, device=cuda), S)), torch.view_as_real(one))
+    _same(*[torch.view_as_real(fo.evaluate(fo.FTAtoms(In, xn, rn, device=cuda), S))
+            for In, xn, rn in _copies(rng, I, x, r)])
