@@ -905,17 +905,13 @@ __global__ __launch_bounds__(PF_WAVES * 64) __attribute__((amdgpu_waves_per_eu(5
                 const int jj = base + __builtin_amdgcn_readfirstlane((int)wl[rect][k]);
                 if (regular && scalar_ptr(na + jj)->np != 0) continue;
                 smem<PairRec> *r = &scalar_ptr(ra + jj)->r;
-                if (i1 < r->lo[1] || i1 > r->hi[1]) continue;
-                const float alpha = r->alpha;
+                // (chosen by the record's box: 0 times an infinite amplitude is no 0)
+                const bool in = i1 >= r->lo[1] && i1 <= r->hi[1];
                 float m[1];
-                if (rA >= r->lo[0] && rA <= r->hi[0]) {
-                    psf_pixel<2, 1>(ra[jj], prA, pc, m);
-                    sA += (double)(alpha * m[0]);
-                }
-                if (rB >= r->lo[0] && rB <= r->hi[0]) {
-                    psf_pixel<2, 1>(ra[jj], prB, pc, m);
-                    sB += (double)(alpha * m[0]);
-                }
+                psf_pixel<2, 1>(ra[jj], prA, pc, m);
+                sA += (double)(in && rA >= r->lo[0] && rA <= r->hi[0] ? r->alpha * m[0] : 0.0f);
+                psf_pixel<2, 1>(ra[jj], prB, pc, m);
+                sB += (double)(in && rB >= r->lo[0] && rB <= r->hi[0] ? r->alpha * m[0] : 0.0f);
             }
         __syncthreads();
     }
