@@ -25,7 +25,9 @@ regulariser of the regularisation module, evaluated inside the fit kernel.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
+import threading
 
 import numpy as np
 import torch
@@ -67,6 +69,7 @@ class gt_fit_block(ctypes.Structure):
 
 BLOCK_BYTES = ctypes.sizeof(gt_fit_block)
 ANGLES_PER_MEMBER = 4  # see default_group
+ANGLES_PER_MEMBER_SHARED = 16  # beside other fits: one angle per wave of a workgroup
 
 
 def _declare():
@@ -82,6 +85,41 @@ def default_group(nA):
     workgroup leaves the waves of a SIMD in each other's way, fewer gains 4 to
     10% more for twice the workgroups."""
     return max(1, min(8, -(-int(nA) // ANGLES_PER_MEMBER)))
+
+
+class WorkgroupCount:
+    """Fit workgroups that this process has on each device.  The members of a
+    group wait for each other (up to the kernel's limit of 2 s), so all of them
+    must be resident, and a workgroup fills a compute unit: fits launched from
+    many host threads may not ask for more than the device holds."""
+
+    def __init__(self):
+        self._lock = threading.Lock()
+        self._used = {}
+
+    @contextlib.contextmanager
+    def take(self, device, nA, room, group=None):
+        """The size of a fit's group, counted while the block runs: `group`, or
+        default_group alone and one workgroup per 16 angles beside other fits
+        (64 fits of 61 angles then fit 256 workgroups, 32 of default_group
+        would); in any case no more than are left of `room`, and at least the one
+        that waits for nobody."""
+        with self._lock:
+            used = self._used.get(device, 0)
+            if group is None:
+                group = default_group(nA)
+                if used:
+                    group = min(group, max(1, -(-int(nA) // ANGLES_PER_MEMBER_SHARED)))
+            group = max(1, min(int(group), room - used))
+            self._used[device] = used + group
+        try:
+            yield group
+        finally:
+            with self._lock:
+                self._used[device] -= group
+
+
+workgroups = WorkgroupCount()
 
 
 def max_blocks():
@@ -252,24 +290,23 @@ def newton_fit(atoms, space, data, max_iter, tol=1e-4, min_iter=1, seed=1, budge
     """Run one Newton fit (or, with gd_dims, one block gradient descent) to
     completion on the device; returns (request, final slot).  group:
     workgroups advancing the fit together (None: default_group of the angle
-    count; 1: a single workgroup).  The result does not depend on the group
-    size."""
+    count, fewer beside other fits of this process; 1: a single workgroup).  The
+    result does not depend on the group size."""
     req = FitRequest(atoms, space, data, max_iter, tol, min_iter, seed, record, reg=reg, block=block, perm=perm,
                      h=h, gd_dims=gd_dims)
     dev = req.I.device
     table = torch.as_tensor(np.frombuffer(req.slot_bytes(), dtype=np.uint8).copy(), device=dev)
     budget = budget or max(req.N * req.max_inner * req.nblk, 1)
-    group = default_group(req.geom.nA) if group is None else int(group)
-    group = max(1, min(group, max_blocks()))
-    blocks = torch.as_tensor(block_table([group]), device=dev) if group > 1 else None
-    while True:
-        if blocks is None:
-            run_slots(table, 1, req.dim, budget)
-        else:
-            run_blocks(table, 1, blocks, group, req.dim, budget)
-        s = read_slots(table, 1)[0]
-        if s.done or not s.active:
-            break
+    with workgroups.take(dev, req.geom.nA, max_blocks(), group) as group:
+        blocks = torch.as_tensor(block_table([group]), device=dev) if group > 1 else None
+        while True:
+            if blocks is None:
+                run_slots(table, 1, req.dim, budget)
+            else:
+                run_blocks(table, 1, blocks, group, req.dim, budget)
+            s = read_slots(table, 1)[0]
+            if s.done or not s.active:
+                break
     if s.done == 3:
         raise RuntimeError("the workgroups of the fit failed to meet at a barrier (device oversubscribed?)")
     req.final = s
