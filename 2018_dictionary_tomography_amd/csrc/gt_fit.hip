@@ -1053,7 +1053,8 @@ __global__ __launch_bounds__(FIT_THREADS) void fit_kernel(gt_fit_slot *__restric
         __syncthreads();
         GT_FIT_TICK(3);
         if (L.stop) break;
-        if (!L.skip) {
+        const int skip = __builtin_amdgcn_readfirstlane(L.skip);
+        if (!skip) {
             // ---- phase E: detector Gaussians of the proposal -------------------
             for (int k = tid; k < nOwn; k += FIT_THREADS) {
                 PairGeom<D> g;
@@ -1079,7 +1080,7 @@ __global__ __launch_bounds__(FIT_THREADS) void fit_kernel(gt_fit_slot *__restric
         // next entries while another still adds the last ones up)
         GT_FIT_MEET();
         GT_FIT_TICK(5);
-        if (L.skip) {
+        if (skip) {
             if (tid == 0) fit_advance(L.c, S, true);
             __syncthreads();  // all of wave 0 reads the new place at the top
             continue;
