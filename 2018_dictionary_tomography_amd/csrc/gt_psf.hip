@@ -950,8 +950,12 @@ __global__ __launch_bounds__(256) void psf_forward_kernel(const PsfRec *__restri
     if (K == 2) {
         const int ntr = (n0 + 15) / 16, ntc = (n1 + 15) / 16;
         a = (int)(blockIdx.x % (unsigned)nA);
-        int t[2];
-        morton_ranks2(blockIdx.x / (unsigned)nA, e0, e1, t);
+        const int e[3] = {e0, e1, 0};
+        int t[3];
+        if (RULE == GT_PSF_SAMPLED)
+            morton_ranks_loop(blockIdx.x / (unsigned)nA, e, t);
+        else
+            morton_ranks2(blockIdx.x / (unsigned)nA, e0, e1, t);
         if (t[0] >= ntr || t[1] >= ntc) return;  // whole block: no tile of this rank
         const int tr = centre_out(t[0], ntr), tcc = centre_out(t[1], ntc);
         i0 = tr * 16 + (int)(threadIdx.x >> 4);
@@ -1713,7 +1717,7 @@ __global__ __launch_bounds__(PV_THREADS) void psf_volume_kernel(const PsfVolRec 
     const int nb0 = (V.m0 + B0 - 1) / B0, nb1 = (V.m1 + B1 - 1) / B1, nb2 = (V.m2 + B2 - 1) / B2;
     const int e[3] = {e0, e1, e2};
     int tb[3];
-    morton_ranks(blockIdx.x, e, tb);
+    morton_ranks_loop(blockIdx.x, e, tb);
     if (tb[0] >= nb0 || tb[1] >= nb1 || tb[2] >= nb2) return;  // whole block
     const int bb0 = centre_out(tb[0], nb0), bb1 = centre_out(tb[1], nb1), bb2 = centre_out(tb[2], nb2);
     const int i0 = bb0 * B0 + t / (B1 * B2), i1 = bb1 * B1 + (t / B2) % B1, i2 = bb2 * B2 + t % B2;
