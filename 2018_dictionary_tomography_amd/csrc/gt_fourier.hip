@@ -179,7 +179,7 @@ __global__ __launch_bounds__(256) void ft_atoms_kernel(gt_atoms A, gt_kgrid Kg, 
 // 16 x 8 x 8 of them, numbered by Morton index over 2^e0 x 2^e1 x 2^e2 centre-out
 // ranks: those near k = 0, which meet the most atoms, first.
 constexpr int FZ_WAVES = 16, FZ_THREADS = 64 * FZ_WAVES, FZ_K0 = 2, FZ_PATCH = 8;
-constexpr unsigned FZ_BLOCKS = 512;  // two blocks of ft_grid_kernel per CU
+constexpr unsigned FZ_BLOCKS = 512;  // (one per CU is resident at its 75 registers; 256 blocks: 1% slower)
 constexpr int FB_THREADS = 512;       // ft_bin_kernel
 struct FzCells {
     int nb[3], q[3], nc[3], e[3];  // patches, patches per cell, cells, bits per axis
@@ -286,9 +286,10 @@ struct alignas(16) FzTerm {
 // Bound by VALU issue on the central patches and by the latency of a patch's
 // staging elsewhere: large blocks keep the first short, the cells' lists and a
 // patch counter the second.  2000 atoms on 128^3: 0.227 ms (patches of 64
-// samples, every block scanning the atoms in radius order) -> 0.072; with (waves,
-// k0's) = (8, 2) 0.083, (8, 4) 0.098, (16, 4) 0.086, (16, 1) 0.114; patches in no
-// order 0.105 to 0.13.
+// samples, every block scanning the atoms in radius order) -> 0.072 with four
+// values at a time summed in FP32, 0.076 now; with four, (waves, k0's) = (8, 2)
+// 0.083, (8, 4) 0.098, (16, 4) 0.086, (16, 1) 0.114; patches in no order 0.105 to
+// 0.13.
 __global__ __launch_bounds__(FZ_THREADS) void ft_grid_kernel(const FtRec *__restrict__ recs,
                                                              const float2 *__restrict__ tab, int N, gt_kgrid Kg,
                                                              FzState *__restrict__ state,
@@ -526,7 +527,15 @@ __global__ __launch_bounds__(FP_THREADS) void ft_patch_kernel(const FtRec *__res
             if (w < wave) off += wcnt[w];
             total += wcnt[w];
         }
-        if (hit) list[off + __popcll(m & ((1ull << lane) - 1ull))] = *reinterpret_cast<const FtL *>(recs + j);
+        if (hit) {
+            FtL rec = *reinterpret_cast<const FtL *>(recs + j);
+            if (FINE) {  // the position as doubles, in the place of its float pairs
+                const double x[3] = {(double)rec.xh[0] + (double)rec.xl[0], (double)rec.xh[1] + (double)rec.xl[1],
+                                     (double)rec.xh[2] + (double)rec.xl[2]};
+                __builtin_memcpy(&rec.xh[0], x, sizeof x);
+            }
+            list[off + __popcll(m & ((1ull << lane) - 1ull))] = rec;
+        }
         __syncthreads();
         for (int q = wave; q < total; q += FP_WAVES) {
             const FtL &r = list[q];
@@ -541,9 +550,9 @@ __global__ __launch_bounds__(FP_THREADS) void ft_patch_kernel(const FtRec *__res
             }
             float sn, cs;
             if (FINE) {
-                const double t = fma((double)r.xh[0] + (double)r.xl[0], (double)k0,
-                                     fma((double)r.xh[1] + (double)r.xl[1], (double)k1,
-                                         ((double)r.xh[2] + (double)r.xl[2]) * (double)k2));
+                double x[3];
+                __builtin_memcpy(x, &r.xh[0], sizeof x);
+                const double t = fma(x[0], (double)k0, fma(x[1], (double)k1, x[2] * (double)k2));
                 ft_sincos_fine(t, sn, cs);
             } else {
                 float err = 0.0f;

@@ -306,15 +306,19 @@ __global__ __launch_bounds__(256) void kp_eval_kernel(const KpRec<R> *__restrict
 // every KE_WAVES-th record of its list (records whose box and ellipse meet the
 // rectangle, in atom order), their FP64 sums added in a fixed order; central
 // rectangles start first.  With the list goes, per record, the mask of the row
-// pairs that the ellipse can reach (kp_row_pairs), and the others are skipped.
+// pairs that the ellipse can reach (kp_row_range), and the others are skipped.
 // The phase is a row part plus a column part: per record each lane evaluates
 // the sine and cosine of one column or row (handed round through LDS), and a
 // sample costs one complex product instead of two phase reductions, a sine and
-// a cosine.  A sample's values are added in FP64.  The planes pass through k = 0 and out(-k) = conj(out(k)): on ascending
-// axes that pair k with -k (0: m-1-i, 1: m-i and none for i = 0, an even FFT's)
-// the rectangles of k0 < 0 whose samples all have a partner are written with it.
-// Bound by VALU issue: 2000 atoms, 61 x 128^2 samples: 0.97 -> 0.35 ms, 0.235 with
-// the partners; without the row pairs 0.38.
+// a cosine.  A sample's values are added in FP64.  The planes pass through k = 0
+// and out(-k) = conj(out(k)): on ascending axes that pair k with -k (0: m-1-i, 1:
+// m-i and none for i = 0, an even FFT's) the rectangles of k0 < 0 whose samples
+// all have a partner are written with it.
+// Bound by VALU issue (0.85 instructions per cycle and CU, conversions and FP64
+// additions among them; LDS 17%) and the few central rectangles: 2000 atoms, 61 x
+// 128^2 samples: 0.97 ms in tiles of 256 samples, 0.35 here, 0.235 with the partners
+// (without the row pairs 0.38 before them), 0.26 with every value added in FP64
+// instead of eight at a time in FP32.
 static_assert(sizeof(KpRec<float>) == 48, "KpRec<float>: amp, q[3] | ch[2], cl[2] | lo[2], hi[2]");
 constexpr int KE_WAVES = 8, KE_ROWS = 16, KE_COLS = 32, KE_R = KE_ROWS / 2;
 

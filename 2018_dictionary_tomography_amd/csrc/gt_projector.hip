@@ -309,7 +309,7 @@ __global__ __launch_bounds__(256) void forward2_kernel(const PairRec *__restrict
         const int total = stage_chunk<4>(ra, base, N, row0, thi, 0, 0, list, wcnt);
         // four records at a time: their values first, then the compensated sum
         // takes them in list order (a few waves per CU: one at a time, every
-        // record's LDS reads and exponential were waited for: 51 atoms, 180 angles
+        // record's LDS reads and exponential were waited for: 50 atoms, 180 angles
         // 12.0 us, now 10.4)
         for (int e = 0; e < total; e += 4) {
             float v[4];
@@ -732,7 +732,7 @@ static void launch_deriv_kernels(const gt_atoms *A, const gt_geom *G, const Pair
                  A->n, G->nA, G->n0, G->n1, G->p0, G->p1, C, mom, MODE == MODE_L2 ? sumC2 : part,
                  MODE == MODE_L2 ? nsq : nparts);
     // (1D detectors: 180 angles 11.5 us on one wave, 7.2 on four; a 3D atom's
-    // rows fill the LDS of a workgroup with one wave)
+    // rows take 34 KB per wave, four waves' more than the 64 KB of a static slab)
     if (D == 2 && G->nA > 64)
         launch_timed(GT_K_FINISH, finish_kernel<D, MODE, D == 2 ? 4 : 1>, dim3(A->n + (part ? 1 : 0)), dim3(D == 2 ? 256 : 64), 0,
                      st, *A, *G, recs, mom, sumC2, ORDER == 2 ? 1 : 0, f, g, H, part, nparts, ftotal);

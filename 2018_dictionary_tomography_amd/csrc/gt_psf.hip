@@ -692,10 +692,11 @@ __device__ inline int psf_stage(const PsfRec *__restrict__ ra, int base, int N, 
 // cell is a factor of its column times a factor of its row (PfTab): a wave forms
 // those of four records at once, 1.5 exponentials per record, lane and node pair
 // instead of 8 (two pixels, two axes, two signs) and a product per pixel.  A
-// pixel's values are added in FP64.  1000 atoms, 61
-// x 128^2: 1.59 ms with a form per node, 0.45 with the node weights tabulated
-// (8 x 64 pixels per block), 0.39 with the factors tabulated, 0.35 with 8 x 32
-// pixels, 0.34 with two waves per rectangle (four: 0.40).
+// pixel's values are added in FP64.  1000 atoms, 61 x 128^2: 1.59 ms with a form per
+// node, 0.45 with the node weights tabulated (8 x 64 pixels per block), 0.39 with
+// the factors tabulated, 0.35 with 8 x 32 pixels, 0.32 with two waves per rectangle
+// (four: 0.40); 0.86 vector instructions per cycle and CU, exponentials at half
+// rate among them, and the LDS busy 26% of the cycles.
 constexpr int PF_RECTS = 2, PF_GROUPS = 2, PF_WAVES = PF_RECTS * PF_GROUPS;
 constexpr int PF_CHUNK = PF_WAVES * 64, PF_ROWS = 8, PF_COLS = 16 * PF_RECTS;
 
@@ -1584,7 +1585,7 @@ template <int NP> __device__ inline float psf_voxel_nodes(smem<float> *w, float 
 // issue: a voxel costs 7 to 19 exponentials instead of 27 to 216, and the cube
 // test drops what the boxes of slanted ellipsoids keep; 1000 atoms on 64^3:
 // 1.75 -> 0.165 ms with bricks of 4 x 8 x 8 and 16 waves, 0.146 with 8 waves,
-// 0.135 with bricks of 4 x 4 x 8 and 4 or 2 waves per cube (8 per cube: 0.163):
+// 0.124 with bricks of 4 x 4 x 8 and 4 waves per cube (8 per cube: 0.163):
 // smaller blocks leave less to the last ones.
 constexpr int PX_GROUPS = 4, PX_ROW = 1, PX_CUBES = 2 * PX_ROW, PX_WAVES = PX_GROUPS * PX_CUBES, PX_THREADS = 64 * PX_WAVES;
 

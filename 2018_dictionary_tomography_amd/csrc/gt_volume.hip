@@ -8,9 +8,9 @@
 // float pair, U scaled so that the exponent is exp2(-|U'(y-x)|^2), and the
 // index box of the ellipsoid |U(y-x)| <= 1 on each (ascending) coordinate
 // vector.  The 3D render gives each wave 4 x 8 x 8 voxels and the list of the
-// atoms whose support meets them; the 2D render gives each block a tile,
-// stages the atoms whose box meets it in LDS (in atom order), and accumulates
-// 4 voxels per lane with Kahan sums.
+// atoms whose support meets them; the 2D render, and the 3D one of few atoms on
+// large grids, give each block a tile or rows, stage the atoms whose box meets it
+// in LDS (in atom order), and accumulate 4 voxels per lane (2D with Kahan sums).
 #include <algorithm>
 
 #include "gt_common.h"
@@ -136,8 +136,9 @@ constexpr int VCHUNK = 128;
 // in group order.
 // Bound by VALU issue and by the central bricks, which meet the most atoms: the
 // parts' lists are split so that no wave is much longer than the rest.  1000
-// atoms on 128^3: 0.22 ms with 4 x 4 x 64 bricks culled by index box, 0.086 now;
-// (parts, groups) = (4, 1) 0.116, (4, 2) 0.092, (2, 4) 0.095, (1, 4) 0.089.
+// atoms on 128^3: 0.22 ms with 4 x 4 x 64 bricks culled by index box, 0.083 now;
+// with four values at a time summed in FP32 0.081, then (parts, groups) = (4, 1)
+// 0.116, (4, 2) 0.092, (2, 4) 0.095, (1, 4) 0.089 against 0.086.
 constexpr int V3_PARTS = 2, V3_GROUPS = 2, V3_WAVES = V3_PARTS * V3_GROUPS, V3_THREADS = 64 * V3_WAVES;
 constexpr int V3_N1 = V3_PARTS == 4 ? 2 : 1, V3_N2 = V3_PARTS / V3_N1;  // parts per axis
 constexpr int V3_B1 = 8 * V3_N1, V3_B2 = 8 * V3_N2;
@@ -406,7 +407,7 @@ extern "C" int gt_volume(const gt_atoms *atoms, const gt_vol *vol, float *u, voi
         // 482 and 482; sparse ones, with the blocks below, 384^3, 64 219 and 179, 128 309
         // and 303; 320^3, 128 197 and 188; up to 4096 ranks (128^3, 32 atoms) 19 and 18;
         // rows of 4 voxels (512 x 512 x 4, 32 atoms) 24 and 57.
-        if (V.m2 >= 64 && ranks > 4096 && atoms->n < (sparse && ranks > 32768 ? 128 : 64)) {
+        if (V.m2 >= 64 && ranks > 4096 && atoms->n <= (sparse && ranks > 32768 ? 128 : 64)) {
             const unsigned long long rows = (unsigned long long)((V.m0 + 3) / 4) * ((V.m1 + 3) / 4) * ((V.m2 + 63) / 64);
             GT_CHECK_ARG(rows < (1ull << 31), "gt_volume: grid too large");
             hipLaunchKernelGGL(volume3_rows_kernel, dim3((unsigned)rows), dim3(256), 0, st, recs, atoms->n, V, u);

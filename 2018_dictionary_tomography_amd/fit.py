@@ -79,11 +79,10 @@ def _declare():
 def default_group(nA):
     """Workgroups that advance one fit together: one per 4 angles, at most 8 (a
     group's workgroups wait for each other and must all be on the device, so
-    concurrent fits share its 256).  An update at 16 angles per workgroup and
-    at 4, microseconds: 30 angles x 64^2 49.7 and 42.6, 61 x 96^2 63.0 and
-    56.7, 61 x 160^2 99.0 and 88.5, 2D 60 x 128 29.8 and 27.3; more than 4 per
-    workgroup leaves the waves of a SIMD in each other's way, fewer gains 4 to
-    10% more for twice the workgroups."""
+    concurrent fits share its 256: see WorkgroupCount).  An update of 60 atoms
+    at 16 angles per workgroup and at 4, microseconds: 30 angles x 64^2 46.0
+    and 40.1, 60 x 96^2 54.9 and 49.7, 64 x 128^2 68.1 and 60.0; 16 instead of 8
+    workgroups gain 2 to 13% more (39.2, 46.8, 55.9)."""
     return max(1, min(8, -(-int(nA) // ANGLES_PER_MEMBER)))
 
 

@@ -102,7 +102,10 @@ def prepare_payloads(specs, device):
 def work_per_update(spec):
     """Relative cost of one atom update on one workgroup, in detector-pixel
     units: the pixels touched grow with angles x detector area, plus a fixed
-    part (setup, FP64 contraction and solve) worth about 5.3e5 pixels."""
+    part (setup, FP64 contraction and solve) worth 5.3e5 pixels, fitted to an
+    earlier kernel.  (A fit alone on one workgroup now: 51 us, 3.3e5 pixels at the
+    rate below; with that value the 2000-request stream served 11.1 instead of 12.1
+    fits/s, so this one stays.)"""
     return spec.nA * spec.S * spec.S + 5.3e5
 
 
@@ -380,8 +383,8 @@ class FitServer:
 
 
 def group_candidates(nA, capacity):
-    """Group sizes tried for a plain fit of nA angles: the default (about one
-    angle per wave), 16, 32, 64 and one angle per workgroup."""
+    """Group sizes tried for a plain fit of nA angles: the default (one
+    workgroup per 4 angles, at most 8), 16, 32, 64 and one angle per workgroup."""
     c = {F.default_group(nA), 16, 32, 64, int(nA)}
     return sorted(g for g in c if 1 <= g <= min(int(nA), capacity))
 

@@ -34,11 +34,11 @@ def _dense(I, x, r, y, dev):
     return ref, bound
 
 
-# rows of 64 from 4097 brick numbers on and up to 63 atoms (127 where most of more than
+# rows of 64 from 4097 brick numbers on and up to 64 atoms (128 where most of more than
 # 32768 numbers are empty); bricks otherwise
 @pytest.mark.parametrize("shape", [(1, 600, 1030), (5, 131, 2050), (33, 125, 64), (130, 70, 65), (17, 265, 1041),
                                    (600, 515, 3)])
-@pytest.mark.parametrize("n,order", [(1, 1), (63, 1), (64, 1), (7, -1), (127, 1), (129, 1)])
+@pytest.mark.parametrize("n,order", [(1, 1), (64, 1), (65, 1), (7, -1), (128, 1), (129, 1)])
 def test_few_atoms(gt, cuda, shape, n, order):
     W = importlib.import_module("2018_dictionary_tomography_amd.workloads")
     I, x, r, _ = W.draw_aniso3(n, np.random.default_rng(sum(shape) + n))
